@@ -62,56 +62,59 @@ __global__ void k_fill_u32(uint32_t* __restrict__ p, size_t n, uint32_t v) {
 // the next substep, when nothing else moves particles in between.
 // Particle i at position q (valid lanes only).  Every lane of the wave must
 // call this (lanes 0..26 do the marking).
+//
+// Bound by latency: a returning atomic is about 2 us away, and a wave holds up to
+// eight runs.  So the loop over the runs only ranks and marks (wave masks, no
+// memory to wait for), and the counting atomics of all runs go out together, one
+// lane per run.
 __device__ __forceinline__ void bin_mark(const DParams& P, const DGrid& G, uint32_t i, bool valid, float4 q) {
   bool live = valid && !(q.y < ST_DEADY);
   uint32_t key = P.ntiles;
-  // tiles [cc-2, cc+2] >> 3 relative to the particle's own tile, as bits
-  // (dx+1) + 3 (dy+1) + 9 (dz+1); the span is at most two tiles per axis
-  uint32_t nmask = 0;
-  int32_t ox = 0, oy = 0, oz = 0;
+  // whether the span [cc-2, cc+2] reaches the tile below (above) per axis; it
+  // covers at most two tiles
+  bool xl = false, xh = false, yl = false, yh = false, zl = false, zh = false;
   if (live) {
     int3 cc = d_particleCell(P, make_float3(q.x, q.y, q.z));
     key = d_tileOf(P, cc.x, cc.y, cc.z);
-    ox = cc.x >> 3; oy = cc.y >> 3; oz = cc.z >> 3;
-    // per axis, bits of the offsets -1, 0, +1 that the span covers
-    uint32_t bx = 2u | (cc.x - 2 >= 0 && ((cc.x - 2) >> 3) < ox ? 1u : 0u) |
-                  (cc.x + 2 <= int32_t(P.tx) * 8 - 1 && ((cc.x + 2) >> 3) > ox ? 4u : 0u);
-    uint32_t by = 2u | (cc.y - 2 >= 0 && ((cc.y - 2) >> 3) < oy ? 1u : 0u) |
-                  (cc.y + 2 <= int32_t(P.ty) * 8 - 1 && ((cc.y + 2) >> 3) > oy ? 4u : 0u);
-    uint32_t bz = 2u | (cc.z - 2 >= 0 && ((cc.z - 2) >> 3) < oz ? 1u : 0u) |
-                  (cc.z + 2 <= int32_t(P.tz) * 8 - 1 && ((cc.z + 2) >> 3) > oz ? 4u : 0u);
-    uint32_t xy = ((by & 1u) ? bx : 0u) | ((by & 2u) ? bx << 3 : 0u) | ((by & 4u) ? bx << 6 : 0u);
-    nmask = ((bz & 1u) ? xy : 0u) | ((bz & 2u) ? xy << 9 : 0u) | ((bz & 4u) ? xy << 18 : 0u);
+    // below: cc - 2 in the tile below, which is there unless the tile is the first
+    xl = (cc.x & 7) < 2 && cc.x >= 8;
+    yl = (cc.y & 7) < 2 && cc.y >= 8;
+    zl = (cc.z & 7) < 2 && cc.z >= 8;
+    xh = (cc.x & 7) > 5 && cc.x + 2 <= int32_t(P.tx) * 8 - 1;
+    yh = (cc.y & 7) > 5 && cc.y + 2 <= int32_t(P.ty) * 8 - 1;
+    zh = (cc.z & 7) > 5 && cc.z + 2 <= int32_t(P.tz) * 8 - 1;
   }
-  // runs of equal bins in the wave: one bin count atomic per run (its result is
-  // not waited for); lane l < 27 marks neighbour l of the run's tile if any
-  // particle of the run needs it
+  // lane l < 27 stands for the neighbour tile (l % 3, l / 3 % 3, l / 9) - 1 of a
+  // run's tile: sel holds the lanes whose span reaches that neighbour
   const uint32_t ln = lane_id();
-  const int32_t mdx = int32_t(ln % 3u) - 1, mdy = int32_t((ln / 3u) % 3u) - 1, mdz = int32_t(ln / 9u) - 1;
-  uint32_t rank = 0u;
+  const uint32_t dx = ln % 3u, dy = (ln / 3u) % 3u, dz = ln / 9u;
+  const int32_t off = int32_t(dx) - 1 + int32_t(P.tx) * (int32_t(dy) - 1 + int32_t(P.ty) * (int32_t(dz) - 1));
+  const uint64_t mxl = __ballot(xl), mxh = __ballot(xh), myl = __ballot(yl), myh = __ballot(yh), mzl = __ballot(zl), mzh = __ballot(zh);
+  const uint64_t sel = (dx == 0u ? mxl : dx == 1u ? ~0ull : mxh) & (dy == 0u ? myl : dy == 1u ? ~0ull : myh) &
+                       (dz == 0u ? mzl : dz == 1u ? ~0ull : mzh);
+  uint32_t rank = 0u, count = 0u;
+  int lead = int(ln);
   uint64_t rem = __ballot(valid);
   while (rem) {
-    int leader = __ffsll((unsigned long long)rem) - 1;
-    uint32_t k = (uint32_t)__shfl((int)key, leader);
-    uint64_t m = __ballot(valid && key == k) & rem;
-    bool inrun = (m >> ln) & 1ull;
-    uint32_t um = inrun ? nmask : 0u;
-    for (int off = 32; off > 0; off >>= 1) um |= (uint32_t)__shfl_xor((int)um, off);
-    // the run's places in the bin: one returning atomic, read at the end
-    uint32_t base = 0u;
-    if (int(ln) == leader) base = atomicAdd(&G.binCount[k], (uint32_t)__popcll(m));
-    base = (uint32_t)__shfl((int)base, leader);
-    if (inrun) rank = base + (uint32_t)__popcll(m & lanemask_lt());
-    if (k < P.ntiles) {
-      int32_t tx0 = __shfl(ox, leader), ty0 = __shfl(oy, leader), tz0 = __shfl(oz, leader);
-      if (ln < 27u && ((um >> ln) & 1u))
-        G.need[uint32_t(tx0 + mdx) + P.tx * (uint32_t(ty0 + mdy) + P.ty * uint32_t(tz0 + mdz))] = 1u;
+    const int leader = __ffsll((unsigned long long)rem) - 1;
+    const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)key, leader);
+    const bool mine = valid && key == k;
+    const uint64_t m = __ballot(mine);
+    if (mine) {
+      lead = leader;
+      rank = (uint32_t)__popcll(m & lanemask_lt());
+      count = (uint32_t)__popcll(m);
     }
+    if (ln < 27u && k < P.ntiles && (sel & m) != 0ull) G.need[uint32_t(int32_t(k) + off)] = 1u;
     rem &= ~m;
   }
+  // the runs' places in their bins: one returning atomic per run, all in flight together
+  uint32_t base = 0u;
+  if (valid && lead == int(ln)) base = atomicAdd(&G.binCount[key], count);
+  base = (uint32_t)__shfl((int)base, lead);
   if (valid) {
     G.binKey[i] = key;
-    G.binRank[i] = rank;
+    G.binRank[i] = base + rank;
   }
 }
 
