@@ -162,6 +162,9 @@ struct Sim {
   uint32_t normCap = 0;           // workgroups normPart has room for
   hipStream_t ownStream = nullptr;  // the tank's own stream while it is in a batch
 
+  // tiles the particles would fill at rest density
+  uint32_t fullTiles() const { return uint32_t(double(N) / (512.0 * rest)); }
+
   LaunchCtx ctx() const {
     LaunchCtx L;
     L.P = &cur->P;
@@ -181,6 +184,7 @@ struct Sim {
     L.nbOn = nbOn;
     L.initStep = initStep;
     L.smax = sprayCap;
+    L.fullTiles = fullTiles();
     L.extrap = extrapOnStep;
     L.exMask = exMask;
     return L;
@@ -1751,13 +1755,17 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
   DParams* hP = (DParams*)(h + b->offP);
   DCols* hC = (DCols*)(h + b->offC);
   uint32_t* hTab = (uint32_t*)(h + b->offTab);
+  uint32_t full = 0;
+  for (const Sim* s : b->tanks) full += s->fullTiles();
+  const uint32_t split = g2p_split(full);
   for (uint32_t t = 0; t < nt; t++) {
     Sim* s = b->tanks[t];
     BTankPlan& pl = b->plan[t];
-    pl = BTankPlan{0u, s->ntiles, s->scap, 0u, false, false};
+    pl = BTankPlan{0u, s->ntiles, s->scap, 0u, false, false, split};
     hT[t].P = (const DParams*)(d + b->offP) + t;
     hT[t].C = (const DCols*)(d + b->offC) + t;
     hT[t].G = s->G;
+    hT[t].split = split;
     if (!s->N) continue;  // step() does nothing when N = 0
     if ((rc = prepStep(s, prm + (nprm == 1u ? 0u : t), hP[t], hC[t]))) return rc;
     pl.n = s->N;

@@ -36,6 +36,7 @@ struct LaunchCtx {
   bool nbOn;          // narrow band on this step
   uint32_t initStep;  // narrow-band start: 1 restart, 2 water added, 0 none
   uint32_t smax;      // whitewater slots (host copy of P->smax)
+  uint32_t fullTiles; // tiles the particles would fill (n / particles of a full tile), for launch shapes
   uint32_t extrap;    // opt-in face velocity extrapolation: layers (host copy of P->extrap)
   uint8_t* exMask;    // its face masks, two per pool cell (ping-pong)
 };
@@ -60,6 +61,7 @@ struct BTank {
   const DParams* P;
   const DCols* C;
   DGrid G;
+  uint32_t split;  // g2p workgroups per tile
 };
 #define ST_BATCH_MAX 256
 // per tank, what one batched substep launches for it
@@ -70,6 +72,7 @@ struct BTankPlan {
   uint32_t iters;   // SOR iterations
   bool binned;      // need, binCount and binKey already hold A's marks and bins
   bool solid;       // rebuild the per-cell collider lookup
+  uint32_t split;   // g2p workgroups per tile
 };
 // Block tables of a batched substep: table k holds nt + 1 workgroup starts, one
 // range per tank (empty where the tank has no work in that launch).  Table
@@ -110,6 +113,8 @@ uint32_t sor_coop_grid(uint32_t cus);
 void morton_tiles(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t* out);
 void launch_project(hipStream_t st, const LaunchCtx& L);
 void launch_g2p(hipStream_t st, const LaunchCtx& L);
+// g2p workgroups per tile for particles that would fill this many tiles
+uint32_t g2p_split(uint32_t fullTiles);
 void launch_unsort(hipStream_t st, const float4* src, const uint32_t* pid, float4* out, uint32_t n);
 // the live view: what one packing needs (positions quantised to 16 bits across the box)
 struct ViewParams {

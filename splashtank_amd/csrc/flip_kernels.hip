@@ -537,6 +537,7 @@ __device__ __forceinline__ int32_t wface(const DParams& P, uint32_t axis, int32_
 
 // ---------------------------------------------------------------------------
 // p2g (wgsl-solver.js:16-40), one workgroup per tile in use
+template <uint32_t W>
 __device__ __forceinline__ void p2g_tile_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid) {
   const DParams& P = *PP;
   // per face: weight in the low 32 bits, velocity in the high 32 bits of one
@@ -550,10 +551,10 @@ __device__ __forceinline__ void p2g_tile_body(const DParams* __restrict__ PP, co
     uint32_t s = G.slotList[b], t = G.slotTile[s];
     int3 org;
     load_wslots(P, G, s, t, wslots, org);
-    for (uint32_t q = threadIdx.x; q < WIN3; q += WG) {
+    for (uint32_t q = threadIdx.x; q < WIN3; q += W) {
       sVW[0][q] = 0ull; sVW[1][q] = 0ull; sVW[2][q] = 0ull;
     }
-    for (uint32_t q = threadIdx.x; q < 512u; q += WG) sC[q] = 0;
+    for (uint32_t q = threadIdx.x; q < 512u; q += W) sC[q] = 0;
     __syncthreads();
     uint32_t beg = G.binStart[t], end = G.binStart[t + 1];
     const bool wscaleSmall = P.scale <= 2147483520.0f;
@@ -561,12 +562,11 @@ __device__ __forceinline__ void p2g_tile_body(const DParams* __restrict__ PP, co
     // bit for bit: scaling by 2^k commutes with rounding where w * vc is normal, and
     // where it is subnormal (or zero) both products round to the integer 0.
     const bool scalePow2 = (st_f2u(P.scale) & 0x807fffffu) == 0u && P.scale >= 1.0f && P.scale <= 1048576.0f;
-    // the four waves take every fourth entry of each run of WG bin entries:
+    // the W / 64 waves take every (W / 64)-th entry of each run of W bin entries:
     // neighbouring entries tend to be neighbouring particles (last substep's
     // order), and lanes adding to the same LDS word in one instruction queue
-    static_assert(WG == 256, "four waves of 64 cover a run of WG entries");
-    for (uint32_t k0 = beg; k0 < end; k0 += WG) {
-      const uint32_t k = k0 + (threadIdx.x & 63u) * 4u + (threadIdx.x >> 6);
+    for (uint32_t k0 = beg; k0 < end; k0 += W) {
+      const uint32_t k = k0 + (threadIdx.x & 63u) * (W / 64u) + (threadIdx.x >> 6);
       if (k >= end) continue;
       uint32_t i = G.binIdx[k];
       float4 p4 = G.pos[i];
@@ -623,9 +623,9 @@ __device__ __forceinline__ void p2g_tile_body(const DParams* __restrict__ PP, co
     // boundary cells wait in their halo records, which k_p2g_merge adds in);
     // the halo shell goes to this tile's record, except for cells of tiles
     // without storage (the spare slot), which every tile adds to directly.
-    for (uint32_t q = threadIdx.x; q < 512u; q += WG) G.cnt[s * 512u + q] = sC[q];
+    for (uint32_t q = threadIdx.x; q < 512u; q += W) G.cnt[s * 512u + q] = sC[q];
     int32_t* rec = G.p2gHalo + size_t(s) * P2G_HALO_WORDS;
-    for (uint32_t q = threadIdx.x; q < WIN3; q += WG) {
+    for (uint32_t q = threadIdx.x; q < WIN3; q += W) {
       const uint32_t wx = q % WIN, wy = (q / WIN) % WIN, wz = q / (WIN * WIN);
       const unsigned long long e[3] = {sVW[0][q], sVW[1][q], sVW[2][q]};
       const bool own = wx - 1u < 8u && wy - 1u < 8u && wz - 1u < 8u;
@@ -658,18 +658,19 @@ __device__ __forceinline__ void p2g_tile_body(const DParams* __restrict__ PP, co
   }
   // fastest particle: one partial per workgroup (k_reduce_stats folds them into
   // ctl[6]); same-address atomics from every wave would serialise chip-wide
-  __shared__ uint32_t wmax[WG / 64];
+  __shared__ uint32_t wmax[W / 64];
   vmaxBits = wave_max_u32(vmaxBits);
   if (lane_id() == 0) wmax[threadIdx.x >> 6] = vmaxBits;
   __syncthreads();
   if (threadIdx.x == 0) {
     uint32_t m = 0;
-    for (int q = 0; q < WG / 64; q++) m = max(m, wmax[q]);
+    for (int q = 0; q < int(W / 64); q++) m = max(m, wmax[q]);
     G.part[bid] = m;
   }
 }
-__global__ void __launch_bounds__(WG) k_p2g_tile(const DParams* __restrict__ PP, DGrid G) {
-  p2g_tile_body(PP, G, blockIdx.x, gridDim.x);
+template <uint32_t W>
+__global__ void __launch_bounds__(W) k_p2g_tile(const DParams* __restrict__ PP, DGrid G) {
+  p2g_tile_body<W>(PP, G, blockIdx.x, gridDim.x);
 }
 
 // After p2g: every tile in use adds to the faces of its boundary cells (a local
@@ -1977,9 +1978,11 @@ __device__ __forceinline__ void g2p_particle(const DParams& P, const DCols* __re
   vo4 = make_float4(v.x, v.y, v.z, foam);
 }
 
-// g2p over the bins: one workgroup per tile (bin ntiles holds the dead
-// particles, which are copied).  Reads A through the bin list and writes the new
-// state into B in bin order; the host then swaps A and B.
+// g2p over the bins: `split` workgroups per tile (g2p_split); the dead particles
+// (bin ntiles) are copied, all workgroups sharing them: a narrow band parks a third
+// of its particles there, and one workgroup alone took 290 us over 100,000.
+// Reads A through the bin list and writes the new state into B in bin order; the
+// host then swaps A and B.
 // With `keys` set it also bins the new positions for the next substep
 // (bin_mark); the particle loops then run whole waves, so every lane calls it.
 __device__ __forceinline__ void g2p_emit(const DParams& P, const DGrid& G, uint32_t keys, uint32_t k, uint32_t i, bool valid,
@@ -1993,29 +1996,33 @@ __device__ __forceinline__ void g2p_emit(const DParams& P, const DGrid& G, uint3
 }
 
 __device__ __forceinline__ void g2p_tile_body(const DParams* __restrict__ PP, const DCols* __restrict__ C, const DGrid& G,
-                                              uint32_t keys, uint32_t bid, uint32_t nbid) {
+                                              uint32_t keys, uint32_t split, uint32_t bid, uint32_t nbid) {
   const DParams& P = *PP;
   __shared__ float2 sNO[3][WIN3];
   __shared__ int32_t sC[WIN3];
   __shared__ int32_t sS[DSUM3];
   __shared__ uint32_t wslots[27];
-  for (uint32_t t = bid; t <= P.ntiles; t += nbid) {
-    uint32_t beg = G.binStart[t], end = G.binStart[t + 1];
-    if (beg == end) continue;
-    if (t == P.ntiles) {
-      for (uint32_t k0 = beg; k0 < end; k0 += WG) {
-        uint32_t k = k0 + threadIdx.x;
-        bool valid = k < end;
-        uint32_t i = valid ? G.binIdx[k] : 0u;
-        float4 po = make_float4(0.f, -1.0e6f, 0.f, 0.f), vo = po;
-        if (valid) {
-          po = G.pos[i];
-          vo = G.vel[i];
-        }
-        g2p_emit(P, G, keys, k, i, valid, po, vo);
-      }
-      continue;
+  // the dead particles (bin ntiles), copied by all workgroups
+  for (uint32_t k0 = G.binStart[P.ntiles] + bid * WG, end = G.binStart[P.ntiles + 1]; k0 < end; k0 += nbid * WG) {
+    const uint32_t k = k0 + threadIdx.x;
+    const bool valid = k < end;
+    const uint32_t i = valid ? G.binIdx[k] : 0u;
+    float4 po = make_float4(0.f, -1.0e6f, 0.f, 0.f), vo = po;
+    if (valid) {
+      po = G.pos[i];
+      vo = G.vel[i];
     }
+    g2p_emit(P, G, keys, k, i, valid, po, vo);
+  }
+  for (uint32_t u = bid; u < P.ntiles * split; u += nbid) {
+    const uint32_t t = u / split, part = u - t * split;
+    uint32_t beg = G.binStart[t], end = G.binStart[t + 1];
+    if (split > 1u) {  // this workgroup's part of the bin, whole groups of WG
+      const uint32_t chunk = ((end - beg + split * WG - 1u) / (split * WG)) * WG;
+      beg += part * chunk;
+      end = min(end, beg + chunk);
+    }
+    if (beg >= end) continue;
     bool storage = G.tmap[t] != ST_NONE;
     if (!storage) {  // its block had no room this step: falls freely (wgsl-solver.js:215)
       GlobalGrid gg{P, G};
@@ -2074,8 +2081,8 @@ __device__ __forceinline__ void g2p_tile_body(const DParams* __restrict__ PP, co
   }
 }
 __global__ void __launch_bounds__(WG) k_g2p_tile(const DParams* __restrict__ PP, const DCols* __restrict__ C, DGrid G,
-                                                 uint32_t keys) {
-  g2p_tile_body(PP, C, G, keys, blockIdx.x, gridDim.x);
+                                                 uint32_t keys, uint32_t split) {
+  g2p_tile_body(PP, C, G, keys, split, blockIdx.x, gridDim.x);
 }
 
 // kept grid velocity at a point, all three components (wgsl-core.js:185-197)
@@ -2522,7 +2529,7 @@ __global__ void kb_clear(BATCH_ARGS) { BATCH_TANK; clear_body(T.G, b.blk, b.nblk
 __global__ void __launch_bounds__(WG) kb_p2g_tile(BATCH_ARGS) {
   BATCH_TANK;
   const DGrid G = T.G;  // local: the body's stores cannot touch it
-  p2g_tile_body(TP, G, b.blk, b.nblk);
+  p2g_tile_body<WG>(TP, G, b.blk, b.nblk);
 }
 __global__ void __launch_bounds__(P2G_MERGE_WG) kb_p2g_merge(BATCH_ARGS) {
   BATCH_TANK;
@@ -2668,7 +2675,7 @@ __global__ void __launch_bounds__(WG, 4) kb_g2p_tile(BATCH_ARGS) {
   __shared__ DParams sP;
   batch_stage_params(sP, TP);
   const DGrid G = T.G;  // local: the body's stores cannot touch it
-  g2p_tile_body(&sP, TC, G, 1u, b.blk, b.nblk);
+  g2p_tile_body(&sP, TC, G, 1u, T.split, b.blk, b.nblk);
 }
 
 // ---------------------------------------------------------------------------
@@ -2719,7 +2726,11 @@ void launch_clear(hipStream_t st, const LaunchCtx& L) {
 
 void launch_p2g(hipStream_t st, const LaunchCtx& L) {
   if (!L.n) return;
-  hipLaunchKernelGGL(k_p2g_tile, dim3(L.tileGrid), dim3(WG), 0, st, L.P, L.G);
+  // 512 threads per tile while the tiles leave CUs idle or lightly loaded (stage
+  // 48.6 -> 37.1 us at 123 full tiles, 121 -> 112 at 1050), 256 above, where more
+  // workgroups per CU hide a tile's barriers better (575 against 620 us at 8430)
+  if (L.fullTiles < 2048u) hipLaunchKernelGGL(k_p2g_tile<512>, dim3(L.tileGrid), dim3(512), 0, st, L.P, L.G);
+  else hipLaunchKernelGGL(k_p2g_tile<256>, dim3(L.tileGrid), dim3(256), 0, st, L.P, L.G);
   hipLaunchKernelGGL(k_p2g_merge, dim3(L.tileGrid), dim3(P2G_MERGE_WG), 0, st, L.G);
   hipLaunchKernelGGL(k_reduce_stats, dim3(1), dim3(1024), 0, st, L.G, L.tileGrid, 0u);
 }
@@ -2837,6 +2848,14 @@ void launch_project(hipStream_t st, const LaunchCtx& L) {
   if (L.nbOn) hipLaunchKernelGGL(k_save_vel, dim3(L.cellGrid), dim3(WG), 0, st, L.G);
 }
 
+// Workgroups that share one tile's particles in g2p.  A full tile is 16 rounds of
+// 256 particles, one after another in one workgroup; with few tiles that chain is
+// the kernel's time, so they are split, each part staging the tile's window again.
+// Measured (g2p stage, us at 1 / 2 / 4 / 8 parts): 15 full tiles 55 / 38 / 30 / 24,
+// 123: 80 / 54 / 48 / 47, 415: 101 / 76 / 78 / 98, 1050: 188 / 171 / 212 / 242,
+// 8430: 1056 / 1061; a narrow band of 84: 37 / 29 / 32 / 40.
+uint32_t g2p_split(uint32_t fullTiles) { return fullTiles < 48u ? 8u : fullTiles < 256u ? 4u : fullTiles < 2048u ? 2u : 1u; }
+
 void launch_g2p(hipStream_t st, const LaunchCtx& L) {
   if (!L.n) return;
   if (L.binNext) {  // the next substep's tile marks and bin counts start here
@@ -2844,8 +2863,9 @@ void launch_g2p(hipStream_t st, const LaunchCtx& L) {
     launch_fill_u32(st, L.G.binCount, size_t(L.ntiles) + 1, 0u);
   }
   hipLaunchKernelGGL(k_foam_table, dim3(FOAM_TAB / WG), dim3(WG), 0, st, L.P, L.G);
-  uint32_t g = std::min<uint32_t>(L.ntiles + 1, 8192u);
-  hipLaunchKernelGGL(k_g2p_tile, dim3(g), dim3(WG), 0, st, L.P, L.C, L.G, L.binNext ? 1u : 0u);
+  const uint32_t split = g2p_split(L.fullTiles);
+  uint32_t g = std::min<uint32_t>(L.ntiles * split, 8192u);
+  hipLaunchKernelGGL(k_g2p_tile, dim3(g), dim3(WG), 0, st, L.P, L.C, L.G, L.binNext ? 1u : 0u, split);
 }
 
 void launch_unsort(hipStream_t st, const float4* src, const uint32_t* pid, float4* out, uint32_t n) {
@@ -2902,7 +2922,7 @@ void batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t itersMax, uint32_
           case BT_SOLID: c = p.solid ? cell : 0u; break;
           case BT_COPY: c = (p.iters & 1u) ? cell : 0u; break;
           case BT_FOAM: c = FOAM_TAB / WG; break;
-          case BT_G2P: c = batch_share(BATCH_TILE_WG, p.ntiles + 1u, binTot, std::min<uint32_t>(p.ntiles + 1u, 8192u)); break;
+          case BT_G2P: c = batch_share(BATCH_TILE_WG, p.ntiles + 1u, binTot, std::min<uint32_t>((p.ntiles + 1u) * p.split, 8192u)); break;
           case BT_FILL_NEXT: c = bins; break;
           default: {
             // SOR: the tank's share of the resident workgroups by pool size,
