@@ -62,7 +62,7 @@ template <class T> void dfree(T*& p) {
 // them are the same again.
 struct StepGraph {
   DGrid G;
-  bool binned, solid;
+  bool binned, marksClean, solid;
   int iters;
   uint32_t N, scap, pipe;
   // which whitewater kernels the spray stage launches, and over how many
@@ -132,6 +132,8 @@ struct Sim {
   // need, binCount and binKey already hold the marks and bins of A's positions
   // (the last g2p made them and nothing has moved a particle since)
   bool binned = false;
+  bool marksClean = false;  // need and binCount are zero (the blocks stage leaves them so, until positions are marked)
+  bool barClean = false;    // so are the streaming SOR's barrier words (until a solve)
   NbScratch nb{};
   void* batch = nullptr;          // the batch the tank belongs to (its stream is the batch's)
   // whitewater (setSprayCap, airAlloc; sim.js:333-351)
@@ -179,6 +181,9 @@ struct Sim {
     L.coopGrid = sorMode == 1u ? 0u : coopGrid;
     L.sorStream = sorMode == 2u;
     L.sorSeq = sorSeq;
+    L.full = !onlyTiles;
+    L.marksClean = marksClean;
+    L.barClean = barClean;
     L.binned = binned;
     L.binNext = !nbOn;  // the narrow band's reseed moves particles after g2p
     L.nbOn = nbOn;
@@ -267,9 +272,9 @@ void destroySim(Sim* s) {
   if (s->st) (void)hipStreamSynchronize(s->st);
   freeNb(s->nb);
   dfree(s->G.pos); dfree(s->G.vel); dfree(s->G.pid); dfree(s->G.posB); dfree(s->G.velB); dfree(s->G.pidB); dfree(s->G.binIdx);
-  dfree(s->G.binKey); dfree(s->G.binRank); dfree(s->G.binCount); dfree(s->G.binStart); dfree(s->G.scanTmp);
+  dfree(s->G.binKey); dfree(s->G.binRank); dfree(s->G.binCount); dfree(s->G.binStart); dfree(s->G.scanW);
   dfree(s->G.tmap); dfree(s->G.need); dfree(s->G.newList); dfree(s->G.wg); dfree(s->G.ctl); dfree(s->G.part); dfree(s->G.foamTab);
-  dfree(s->G.mortonTiles); dfree(s->G.coopFlags); dfree(s->G.coopOffs); dfree(s->G.sorBar);
+  dfree(s->G.mortonTiles); dfree(s->G.sorBar);
   dfree(s->G.scratch4);
   dfree(s->normPart);
   dfree(s->G.sPos); dfree(s->G.sVel); dfree(s->G.sAux); dfree(s->G.sctl); dfree(s->G.sprCnt); dfree(s->G.sprOff); dfree(s->G.sprSums);
@@ -554,20 +559,25 @@ int beginStep(Sim* s, const st_params* o) {
   return ST_OK;
 }
 
-int runStage(Sim* s, int stage) {
+// `alone`: the caller may look at the state after this stage (st_stage)
+int runStage(Sim* s, int stage, bool alone = false) {
   if (!s->begun) return fail(ST_ERR_STATE, "st_stage: no step begun");
   LaunchCtx L = s->ctx();
   hipStream_t st = s->st;
   bool full = !s->onlyTiles;
   switch (stage) {
     case ST_STAGE_SORT: break;
-    case ST_STAGE_BLOCKS: launch_blocks(st, L); s->binned = false; break;
-    case ST_STAGE_CLEAR: if (full) launch_clear(st, L); break;
+    case ST_STAGE_BLOCKS:
+      launch_blocks(st, L);
+      s->binned = false;
+      s->marksClean = s->barClean = true;
+      break;
+    case ST_STAGE_CLEAR: break;  // part of the blocks stage's last launch
     case ST_STAGE_P2G: if (full) launch_p2g(st, L); break;
     case ST_STAGE_NARROWBAND: if (full && s->nbOn) launch_narrowband(st, L); break;
     case ST_STAGE_CLASSIFY:
       if (full) {
-        launch_classify(st, L, s->solidDirty);
+        launch_classify(st, L, s->solidDirty, alone);
         s->solidDirty = false;
       }
       break;
@@ -577,6 +587,7 @@ int runStage(Sim* s, int stage) {
       if (full) {
         L.sorSeq = ++s->sorSeq;
         if (launch_pressure(st, L, s->iters) != hipSuccess) s->coopGrid = 0;  // per-iteration launches from now on
+        s->barClean = false;
       }
       break;
     case ST_STAGE_PROJECT: if (full) launch_project(st, L); break;
@@ -584,6 +595,7 @@ int runStage(Sim* s, int stage) {
       if (full) {
         launch_g2p(st, L);
         s->binned = L.binNext && L.n != 0;
+        if (s->binned) s->marksClean = false;
         if (L.n) {  // g2p wrote the new state into the other buffer
           std::swap(s->G.pos, s->G.posB);
           std::swap(s->G.vel, s->G.velB);
@@ -654,7 +666,7 @@ int graphStep(Sim* s, const st_params* o) {
   s->begun = true;
   const uint32_t pipe = s->ctx().pipeGrid;
   for (StepGraph& g : s->graphs) {
-    if (std::memcmp(&g.G, &s->G, sizeof(DGrid)) != 0 || g.binned != s->binned || g.solid != s->solidDirty ||
+    if (std::memcmp(&g.G, &s->G, sizeof(DGrid)) != 0 || g.binned != s->binned || g.marksClean != s->marksClean || g.solid != s->solidDirty ||
         g.iters != s->iters || g.N != s->N || g.scap != s->scap || g.pipe != pipe || g.airOn != s->airOnStep ||
         g.sprOn != s->sprOnStep || g.dripOn != s->dripOnStep || g.ndrip != s->ndrip || g.airN != s->airN ||
         g.sprayCap != s->sprayCap || g.extrap != s->extrapOnStep)
@@ -664,6 +676,7 @@ int graphStep(Sim* s, const st_params* o) {
     s->solidDirty = false;
     s->sorSeq++;
     s->binned = true;
+    s->marksClean = s->barClean = false;
     std::swap(s->G.pos, s->G.posB);
     std::swap(s->G.vel, s->G.velB);
     std::swap(s->G.pid, s->G.pidB);
@@ -672,6 +685,7 @@ int graphStep(Sim* s, const st_params* o) {
   StepGraph e;
   e.G = s->G;
   e.binned = s->binned;
+  e.marksClean = s->marksClean;
   e.solid = s->solidDirty;
   e.iters = s->iters;
   e.N = s->N;
@@ -912,12 +926,11 @@ int st_create(const st_opts* o, void** out) {
   if ((rc = dalloc(&s->G.pos, M)) || (rc = dalloc(&s->G.vel, M)) || (rc = dalloc(&s->G.pid, M)) || (rc = dalloc(&s->G.scratch4, M)) ||
       (rc = dalloc(&s->G.posB, M)) || (rc = dalloc(&s->G.velB, M)) || (rc = dalloc(&s->G.pidB, M)) || (rc = dalloc(&s->G.binKey, M)) || (rc = dalloc(&s->G.binIdx, M)) ||
       (rc = dalloc(&s->G.binCount, nbin)) || (rc = dalloc(&s->G.binStart, size_t(nbin) + 1)) || (rc = dalloc(&s->G.binRank, M)) ||
-      (rc = dalloc(&s->G.scanTmp, size_t(nbin + 1023) / 1024 + 1)) ||
+      (rc = dalloc(&s->G.scanW, scan_word_count(s->ntiles))) ||
       (rc = dalloc(&s->G.tmap, s->ntiles)) || (rc = dalloc(&s->G.need, s->ntiles)) || (rc = dalloc(&s->G.newList, size_t(s->ntiles) * 2)) ||
-      (rc = dalloc(&s->G.wg, size_t((s->ntiles + 255) / 256) * 3 + 3)) || (rc = dalloc(&s->G.ctl, 16)) || (rc = allocSlots(s, s->scap)) ||
+      (rc = dalloc(&s->G.wg, scan_word_count(s->ntiles))) || (rc = dalloc(&s->G.ctl, 16)) || (rc = allocSlots(s, s->scap)) ||
       (rc = dalloc(&s->G.part, 2 * 8192 + 64)) || (rc = dalloc(&s->G.foamTab, FOAM_TAB)) ||
-      (rc = dalloc(&s->G.mortonTiles, s->ntiles)) || (rc = dalloc(&s->G.coopFlags, s->ntiles)) ||
-      (rc = dalloc(&s->G.coopOffs, size_t(s->ntiles) + 1)) || (rc = dalloc(&s->G.sorBar, COOP_MAX_WG + 4)) ||
+      (rc = dalloc(&s->G.mortonTiles, s->ntiles)) || (rc = dalloc(&s->G.sorBar, COOP_MAX_WG + 4)) ||
       (rc = dalloc(&s->dSlots, RING))) {
     destroySim(s);
     return rc;
@@ -945,6 +958,7 @@ int st_create(const st_opts* o, void** out) {
       hipMemcpy(s->G.tmap, tm.data(), size_t(s->ntiles) * 4, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(s->G.mortonTiles, mort.data(), size_t(s->ntiles) * 4, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(s->G.sorBar, 0, (COOP_MAX_WG + 4) * 4) != hipSuccess ||
+      hipMemset(s->G.scanW, 0, scan_word_count(s->ntiles) * 8) != hipSuccess ||
       hipMemcpy(s->G.ctl, ctl, 64, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(s->G.pos, 0, M * 16) != hipSuccess || hipMemset(s->G.vel, 0, M * 16) != hipSuccess ||
       hipMemset(s->G.need, 0, size_t(s->ntiles) * 4) != hipSuccess) {
@@ -1075,7 +1089,7 @@ int st_begin_step(void* p, const st_params* prm) {
 int st_stage(void* p, int32_t stage) {
   Sim* s = getSim(p);
   if (!s) return fail(ST_ERR_ARG, "st_stage: null sim");
-  return runStage(s, stage);
+  return runStage(s, stage, true);
 }
 
 int st_step(void* p, const st_params* prm) {
@@ -1173,6 +1187,7 @@ int st_grow(void* p, uint32_t n) {
   HIPCHK(hipMemcpy(s->G.slotTile, keep.slotTile, size_t(old) * 4, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.fstack, keep.fstack, size_t(old) * 4, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.slotList, keep.slotList, size_t(old) * 4, hipMemcpyDeviceToDevice));
+  HIPCHK(hipMemcpy(s->G.coopList, keep.coopList, size_t(old) * 4, hipMemcpyDeviceToDevice));
   rc = zeroSlots(s, old, n);
   if (rc) return rc;
   // growFree (wgsl-blocks.js:57-60): the new slots go on the free stack
@@ -1761,7 +1776,7 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
   for (uint32_t t = 0; t < nt; t++) {
     Sim* s = b->tanks[t];
     BTankPlan& pl = b->plan[t];
-    pl = BTankPlan{0u, s->ntiles, s->scap, 0u, false, false, split};
+    pl = BTankPlan{0u, s->ntiles, s->scap, 0u, false, false, false, split};
     hT[t].P = (const DParams*)(d + b->offP) + t;
     hT[t].C = (const DCols*)(d + b->offC) + t;
     hT[t].G = s->G;
@@ -1771,6 +1786,7 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
     pl.n = s->N;
     pl.iters = uint32_t(s->iters);
     pl.binned = s->binned;
+    pl.marksClean = s->marksClean;
     pl.solid = s->solidDirty;
   }
   batch_tables(b->plan.data(), nt, itersMax, b->sorResident, hTab);
@@ -1830,6 +1846,7 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
     s->solidDirty = false;
     s->sorSeq++;
     s->binned = true;
+    s->marksClean = s->barClean = false;
     s->cur = nullptr;
     s->begun = false;
     std::swap(s->G.pos, s->G.posB);

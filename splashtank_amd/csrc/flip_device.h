@@ -90,7 +90,7 @@ struct DGrid {
   uint32_t* binRank;   // per particle (A order): its place within its bin
   uint32_t* binCount;  // per tile (+1 dead bin): particles whose cell is in the tile
   uint32_t* binStart;  // exclusive prefix of binCount (ntiles + 2 entries, last = N)
-  uint32_t* scanTmp;   // per-1024-block sums of the bin scan
+  uint64_t* scanW;     // the tile scans' two tickets, then their blocks' published totals
   uint32_t* tmap;
   uint32_t* need;
   uint32_t* newList;   // pairs: tile, slot (or NONE)
@@ -99,7 +99,7 @@ struct DGrid {
   uint32_t* slotList;
   uint32_t* nbr;       // per slot: slots of the 27 tiles around it (0 none, WSLOT_OUT outside)
   uint32_t* nbrL;      // the same rows in slotList order (row b for slotList[b])
-  uint32_t* wg;        // per-workgroup scan scratch
+  uint32_t* wg;        // per scan block: new and kept tiles before it
   uint32_t* part;      // per-workgroup statistics partials (vmax; fluid cells per colour)
   uint32_t* ctl;       // control words, as in the reference's ctl
   int32_t* cnt;
@@ -119,8 +119,6 @@ struct DGrid {
   float4* foamTab;     // per step, for a density sum c < FOAM_TAB: the g2p factors of c (d_foamRow)
   // resident SOR
   uint32_t* mortonTiles; // tile indices in Morton (z-order) order of their tile coordinates
-  uint32_t* coopFlags;   // per Morton position: 1 when the tile is in use
-  uint32_t* coopOffs;    // exclusive prefix of coopFlags
   uint32_t* coopList;    // slots in use, in Morton order (per slot)
   uint64_t* sorHalo;     // per colour, slot and face: the 32 face cells of that colour, each with the tag of
                          // the half-sweep that wrote it (2 x slots x 6 x 32 pairs: value bits low, tag high)

@@ -31,6 +31,9 @@ struct LaunchCtx {
   uint32_t coopGrid;  // resident-SOR workgroups (one per CU), 0 when cooperative launches are unavailable
   uint32_t sorSeq;    // sequence number of this pressure solve
   bool sorStream;     // the cooperative solve streams tile windows even when the tiles fit in LDS
+  bool full;          // the whole substep follows the blocks stage (not a tile-only step)
+  bool marksClean;    // need and binCount are zero
+  bool barClean;      // the streaming SOR's barrier words are zero
   bool binned;        // blocks: need, binCount and binKey already hold A's marks and bins
   bool binNext;       // g2p: mark and bin the positions it writes, for the next substep
   bool nbOn;          // narrow band on this step
@@ -71,6 +74,7 @@ struct BTankPlan {
   uint32_t scap;
   uint32_t iters;   // SOR iterations
   bool binned;      // need, binCount and binKey already hold A's marks and bins
+  bool marksClean;  // need and binCount are zero
   bool solid;       // rebuild the per-cell collider lookup
   uint32_t split;   // g2p workgroups per tile
 };
@@ -78,8 +82,8 @@ struct BTankPlan {
 // range per tank (empty where the tank has no work in that launch).  Table
 // BT_PIPE0 + it belongs to SOR iteration it.
 enum BatchTable {
-  BT_FILL_MARK, BT_MARK, BT_NWG, BT_ONE, BT_ALLOC, BT_CELL, BT_NBR, BT_SCAN, BT_PART,
-  BT_TILE, BT_ONE_N, BT_SOLID, BT_COPY, BT_FOAM, BT_G2P, BT_FILL_NEXT, BT_PIPE0
+  BT_FILL_MARK, BT_MARK, BT_SCAN, BT_PLACE, BT_FINISH, BT_ONE, BT_CELL,
+  BT_TILE, BT_SOLID, BT_COPY, BT_G2P, BT_PIPE0
 };
 size_t batch_table_words(uint32_t nt, uint32_t itersMax);
 // fills the tables (host copy); sorResident = SOR workgroups resident at once
@@ -94,9 +98,11 @@ bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, co
 
 void launch_fill_u32(hipStream_t st, uint32_t* p, size_t n, uint32_t v);
 void launch_blocks(hipStream_t st, const LaunchCtx& L);
-void launch_clear(hipStream_t st, const LaunchCtx& L);
 void launch_p2g(hipStream_t st, const LaunchCtx& L);
-void launch_classify(hipStream_t st, const LaunchCtx& L, bool solid);
+// counts: the fluid counts into ctl[0], ctl[1] now (normFaces does it too)
+void launch_classify(hipStream_t st, const LaunchCtx& L, bool solid, bool counts);
+// 64-bit words of DGrid.scanW
+size_t scan_word_count(uint32_t ntiles);
 void launch_narrowband(hipStream_t st, const LaunchCtx& L);
 void launch_reseed(hipStream_t st, const LaunchCtx& L, const NbScratch& S);
 void launch_norm_faces(hipStream_t st, const LaunchCtx& L);

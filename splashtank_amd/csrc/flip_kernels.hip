@@ -211,169 +211,198 @@ __global__ void __launch_bounds__(WG) k_scan_add(uint32_t* __restrict__ out, uin
   scan_add_body(out, n, sums, copy, blockIdx.x, gridDim.x);
 }
 
-// bin order as an index list: binIdx[binStart[bin] + rank] = i.  The particles
-// themselves stay where they are; p2g and g2p read them through the list (runs
-// of a bin are mostly contiguous in A, which is in last step's bin order).
-__device__ __forceinline__ void bin_scatter_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid) {
-  uint32_t i = bid * blockDim.x + threadIdx.x;
-  if (i >= PP->n) return;
-  G.binIdx[G.binStart[G.binKey[i]] + G.binRank[i]] = i;
-}
-__global__ void __launch_bounds__(WG) k_bin_scatter(const DParams* __restrict__ PP, DGrid G) {
-  bin_scatter_body(PP, G, blockIdx.x, gridDim.x);
-}
+// ---------------------------------------------------------------------------
+// Tile bookkeeping in three launches.  It is bound by launches and by latency
+// (a few words per tile), so each launch does everything whose inputs the one
+// before has made: tiles_scan (flags and bin counts scanned, freed tiles pushed),
+// tiles_place (new and kept tiles take their slots; the bin list), tiles_finish
+// (neighbour rows, new cells, the Morton list of the pressure solve, and what the
+// rest of the substep needs cleared or tabulated).  Nineteen launches before, of
+// which each held the GPU for about 4.5 us; 64^3 substep 468 -> 411 us.
+//
+// A scan over the tiles in one launch: workgroups take blocks of TB tiles by
+// ticket, publish their block's totals and add up the totals of the blocks before
+// theirs.  A block's predecessors have been taken by workgroups that already run
+// and publish before they wait, so every wait ends (and is bounded all the same: a
+// time-out is counted where st_sync reports it).  A published word carries its own
+// valid bit, so no fence is needed; the launch after clears words and ticket.
+#define TB 1024u
+#define SCAN_VALID (1ull << 63)
+__device__ __forceinline__ uint64_t* scan_words(const DGrid& G, uint32_t nb, bool list) { return G.scanW + 2u + (list ? 4u * nb : 0u); }
+__host__ __device__ __forceinline__ uint32_t scan_blocks_of(uint32_t ntiles) { return (ntiles + 1u + TB - 1u) / TB; }
 
-// Flags of one tile: freed (no longer needed, had a slot), new (needed, had
-// none), kept (needed, had one).  tileFree in wgsl-blocks.js:16-21.
-struct TileFlags {
-  bool fr, nw, kp;
-};
-__device__ __forceinline__ TileFlags tile_flags(const DGrid& G, uint32_t t, uint32_t ntiles) {
-  TileFlags f{false, false, false};
-  if (t < ntiles) {
-    uint32_t nd = G.need[t], s = G.tmap[t];
-    f.fr = nd == 0u && s != ST_NONE;
-    f.nw = nd != 0u && s == ST_NONE;
-    f.kp = nd != 0u && s != ST_NONE;
-  }
-  return f;
-}
-
-// workgroup-wide exclusive ranks of three flags (256 threads = 4 waves)
-struct Ranks3 {
-  uint32_t r[3];
-  uint32_t tot[3];
-};
-__device__ __forceinline__ Ranks3 wg_ranks3(bool a, bool b, bool c) {
-  __shared__ uint32_t wsum[3][WG / 64];
-  uint64_t m[3] = {__ballot(a), __ballot(b), __ballot(c)};
-  uint32_t w = threadIdx.x >> 6;
-  if (lane_id() == 0)
-    for (int q = 0; q < 3; q++) wsum[q][w] = uint32_t(__popcll(m[q]));
+__device__ __forceinline__ uint32_t scan_ticket(uint64_t* ticket) {
+  __shared__ uint32_t sB;
+  if (threadIdx.x == 0) sB = uint32_t(atomicAdd((unsigned long long*)ticket, 1ull));
   __syncthreads();
-  Ranks3 R;
-  for (int q = 0; q < 3; q++) {
-    uint32_t before = 0, tot = 0;
-    for (uint32_t v = 0; v < WG / 64; v++) {
-      if (v < w) before += wsum[q][v];
-      tot += wsum[q][v];
+  return sB;
+}
+__device__ __forceinline__ uint64_t shfl_up_u64(uint64_t v, int off) {
+  const uint32_t lo = (uint32_t)__shfl_up((int)uint32_t(v), off), hi = (uint32_t)__shfl_up((int)uint32_t(v >> 32), off);
+  return (uint64_t(hi) << 32) | lo;
+}
+// exclusive scan over the workgroup (WG threads), *tot its total
+__device__ __forceinline__ uint64_t wg_scan_u64(uint64_t v, uint64_t* tot) {
+  __shared__ uint64_t sW[WG / 64];
+  uint64_t inc = v;
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint64_t o = shfl_up_u64(inc, off);
+    if (int(lane_id()) >= off) inc += o;
+  }
+  const uint32_t w = threadIdx.x >> 6;
+  if (lane_id() == 63u) sW[w] = inc;
+  __syncthreads();
+  uint64_t before = 0, all = 0;
+  for (uint32_t u = 0; u < WG / 64; u++) {
+    if (u < w) before += sW[u];
+    all += sW[u];
+  }
+  __syncthreads();
+  *tot = all;
+  return before + inc - v;
+}
+// publishes block b's K totals and returns in pre[K] (shared) those of the blocks before it
+template <uint32_t K>
+__device__ __forceinline__ void scan_chain(uint64_t* W, uint32_t b, const uint64_t (&agg)[K], unsigned long long* pre, uint32_t* timeouts) {
+  if (threadIdx.x < K) pre[threadIdx.x] = 0ull;
+  if (threadIdx.x == 0)
+    for (uint32_t j = 0; j < K; j++) __hip_atomic_store(&W[b * K + j], SCAN_VALID | agg[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  for (uint32_t q = threadIdx.x; q < b * K; q += WG) {
+    uint64_t w = __hip_atomic_load(&W[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (uint32_t spins = 0; !(w & SCAN_VALID); spins++) {
+      if (spins >= GB_SPIN_LIMIT) {
+        atomicAdd(timeouts, 1u);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+      w = __hip_atomic_load(&W[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    R.r[q] = before + uint32_t(__popcll(m[q] & lanemask_lt()));
-    R.tot[q] = tot;
+    atomicAdd(&pre[q % K], (unsigned long long)(w & ~SCAN_VALID));
   }
   __syncthreads();
-  return R;
 }
 
-__device__ __forceinline__ void tile_count_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid) {
-  uint32_t t = bid * WG + threadIdx.x;
-  TileFlags f = tile_flags(G, t, PP->ntiles);
-  Ranks3 R = wg_ranks3(f.fr, f.nw, f.kp);
-  if (threadIdx.x == 0) {
-    G.wg[bid * 3 + 0] = R.tot[0];
-    G.wg[bid * 3 + 1] = R.tot[1];
-    G.wg[bid * 3 + 2] = R.tot[2];
+// tileFree and tileAlloc's counting (wgsl-blocks.js:16-35) in closed form: the
+// k-th new tile (tile order) pops stack entry top1 - 1 - k, so the first
+// min(new, top1) new tiles get slots and the rest count as no room.  Freed tiles
+// push their slot in tile order.  Also the exclusive scan of the bin counts.
+__device__ __forceinline__ void tiles_scan_body(const DParams* __restrict__ PP, const DGrid& G) {
+  const uint32_t ntiles = PP->ntiles, nb = scan_blocks_of(ntiles);
+  __shared__ unsigned long long pre[4];
+  const uint32_t b = scan_ticket(G.scanW);
+  if (b >= nb) return;
+  if (threadIdx.x == 0) {  // the list scan's words, for tiles_finish
+    scan_words(G, nb, true)[b] = 0ull;
+    if (b == 0u) G.scanW[1] = 0ull;
   }
-}
-__global__ void __launch_bounds__(WG) k_tile_count(const DParams* __restrict__ PP, DGrid G) {
-  tile_count_body(PP, G, blockIdx.x, gridDim.x);
-}
-
-// One workgroup: exclusive scan of the per-workgroup counts, then the stack
-// arithmetic of tileFree/tileAlloc/tileFix (wgsl-blocks.js:16-35) in closed form:
-// the k-th new tile (tile order) pops stack entry top1-1-k, so the first
-// min(new, top1) new tiles get slots and the rest count as no room.
-__device__ __forceinline__ void tile_scan_body(const DGrid& G, uint32_t nwg, uint32_t bid, uint32_t nbid) {
-  __shared__ uint32_t part[3][1024 / 64];
-  __shared__ uint32_t carry[3];
-  if (threadIdx.x < 3) carry[threadIdx.x] = 0;
-  __syncthreads();
-  for (uint32_t base = 0; base < nwg; base += 1024) {
-    uint32_t i = base + threadIdx.x;
-    uint32_t v[3];
-    for (int q = 0; q < 3; q++) v[q] = i < nwg ? G.wg[i * 3 + q] : 0u;
-    uint32_t s[3] = {v[0], v[1], v[2]};
-    for (int off = 1; off < 64; off <<= 1)
-      for (int q = 0; q < 3; q++) {
-        uint32_t o = (uint32_t)__shfl_up((int)s[q], off);
-        if (int(lane_id()) >= off) s[q] += o;
-      }
-    uint32_t w = threadIdx.x >> 6;
-    if (lane_id() == 63)
-      for (int q = 0; q < 3; q++) part[q][w] = s[q];
-    __syncthreads();
-    uint32_t before[3] = {0, 0, 0}, tot[3] = {0, 0, 0};
-    for (uint32_t u = 0; u < 1024 / 64; u++)
-      for (int q = 0; q < 3; q++) {
-        if (u < w) before[q] += part[q][u];
-        tot[q] += part[q][u];
-      }
-    if (i < nwg)
-      for (int q = 0; q < 3; q++) G.wg[i * 3 + q] = carry[q] + before[q] + s[q] - v[q];
-    __syncthreads();
-    if (threadIdx.x < 3) carry[threadIdx.x] += tot[threadIdx.x];
-    __syncthreads();
+  const uint32_t t0 = b * TB + threadIdx.x * 4u, top0 = G.ctl[2];
+  uint32_t slot[4], cnt[4];
+  bool fr[4];
+  uint64_t flags = 0, bins = 0;  // freed | new << 16 | kept << 32
+  for (uint32_t q = 0; q < 4u; q++) {
+    const uint32_t t = t0 + q;
+    const bool in = t < ntiles;
+    const bool nd = in && G.need[t] != 0u;
+    slot[q] = in ? G.tmap[t] : ST_NONE;
+    cnt[q] = t <= ntiles ? G.binCount[t] : 0u;
+    fr[q] = !nd && slot[q] != ST_NONE;
+    flags += fr[q] ? 1ull : nd && slot[q] == ST_NONE ? 1ull << 16 : nd ? 1ull << 32 : 0ull;
+    bins += cnt[q];
+  }
+  uint64_t tf, tb;
+  const uint64_t xf = wg_scan_u64(flags, &tf), xb = wg_scan_u64(bins, &tb);
+  const uint64_t agg[4] = {tf & 0xffffu, (tf >> 16) & 0xffffu, tf >> 32, tb};
+  scan_chain<4>(scan_words(G, nb, false), b, agg, pre, G.sorBar + COOP_MAX_WG + 1);
+  uint32_t run = uint32_t(pre[3]) + uint32_t(xb), rank = uint32_t(pre[0]) + uint32_t(xf & 0xffffu);
+  for (uint32_t q = 0; q < 4u; q++) {
+    const uint32_t t = t0 + q;
+    if (t <= ntiles) G.binStart[t] = run;
+    run += cnt[q];
+    if (fr[q]) {
+      G.fstack[top0 + rank++] = slot[q];
+      G.tmap[t] = ST_NONE;
+    }
   }
   if (threadIdx.x == 0) {
-    uint32_t F = carry[0], Nn = carry[1], K = carry[2];
-    uint32_t top0 = G.ctl[2];
-    uint32_t top1 = top0 + F;
-    uint32_t nalloc = min(Nn, top1);
-    G.ctl[2] = top1 - nalloc;
-    G.ctl[3] = Nn;
-    G.ctl[4] = K + nalloc;
-    G.ctl[5] = Nn - nalloc;
-    G.ctl[6] = 0u;
-    G.ctl[12] = top0;
-    G.ctl[13] = top1;
-    G.ctl[14] = nalloc;
+    G.wg[b * 2u] = uint32_t(pre[1]);
+    G.wg[b * 2u + 1u] = uint32_t(pre[2]);
+    if (b == nb - 1u) {
+      const uint32_t top1 = top0 + uint32_t(pre[0] + agg[0]), nn = uint32_t(pre[1] + agg[1]), nalloc = min(nn, top1);
+      G.binStart[ntiles + 1u] = uint32_t(pre[3] + agg[3]);
+      G.ctl[3] = nn;
+      G.ctl[4] = uint32_t(pre[2] + agg[2]) + nalloc;
+      G.ctl[5] = nn - nalloc;
+      G.ctl[6] = 0u;
+      G.ctl[12] = top0;
+      G.ctl[13] = top1;
+      G.ctl[14] = nalloc;  // ctl[2], which every block reads as top0, follows in tiles_place
+    }
   }
 }
-__global__ void __launch_bounds__(1024) k_tile_scan(DGrid G, uint32_t nwg) {
-  tile_scan_body(G, nwg, blockIdx.x, gridDim.x);
-}
+__global__ void __launch_bounds__(WG) k_tiles_scan(const DParams* __restrict__ PP, DGrid G) { tiles_scan_body(PP, G); }
 
-// Freed tiles push their slot (tile order), new tiles are listed (tile order),
-// kept tiles take their place in slotList (tile order).
-__device__ __forceinline__ void tile_scatter_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid) {
-  uint32_t t = bid * WG + threadIdx.x;
-  TileFlags f = tile_flags(G, t, PP->ntiles);
-  Ranks3 R = wg_ranks3(f.fr, f.nw, f.kp);
-  uint32_t baseF = G.wg[bid * 3 + 0], baseN = G.wg[bid * 3 + 1], baseK = G.wg[bid * 3 + 2];
-  uint32_t top0 = G.ctl[12], nalloc = G.ctl[14];
-  if (f.fr) {
-    G.fstack[top0 + baseF + R.r[0]] = G.tmap[t];
-    G.tmap[t] = ST_NONE;
-  } else if (f.nw) {
-    uint32_t k = baseN + R.r[1];
-    G.newList[k * 2] = t;
-    G.newList[k * 2 + 1] = baseK + R.r[2] + k;  // slotList index if it gets a slot
-  } else if (f.kp) {
-    uint32_t nb = baseN + R.r[1];
-    G.slotList[baseK + R.r[2] + min(nb, nalloc)] = G.tmap[t];
+// New tiles take their slots (tileAlloc, wgsl-blocks.js:26-33, in the deterministic
+// pop order) and are listed, new and kept tiles take their place in slotList, all
+// in tile order.  The workgroups after the tile blocks make the bin order as an
+// index list, binIdx[binStart[bin] + rank] = i: the particles themselves stay where
+// they are; p2g and g2p read them through the list (runs of a bin are mostly
+// contiguous in A, which is in last step's bin order).
+__device__ __forceinline__ void tiles_place_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid) {
+  const uint32_t ntiles = PP->ntiles, nb = scan_blocks_of(ntiles);
+  if (bid >= nb) {
+    const uint32_t n = PP->n;
+    for (uint32_t i0 = ((bid - nb) * WG + threadIdx.x) * 4u; i0 < n; i0 += (nbid - nb) * WG * 4u) {
+      if (i0 + 4u <= n) {
+        const uint4 k = *(const uint4*)(G.binKey + i0), r = *(const uint4*)(G.binRank + i0);
+        G.binIdx[G.binStart[k.x] + r.x] = i0;
+        G.binIdx[G.binStart[k.y] + r.y] = i0 + 1u;
+        G.binIdx[G.binStart[k.z] + r.z] = i0 + 2u;
+        G.binIdx[G.binStart[k.w] + r.w] = i0 + 3u;
+      } else {
+        for (uint32_t i = i0; i < n; i++) G.binIdx[G.binStart[G.binKey[i]] + G.binRank[i]] = i;
+      }
+    }
+    return;
   }
-}
-__global__ void __launch_bounds__(WG) k_tile_scatter(const DParams* __restrict__ PP, DGrid G) {
-  tile_scatter_body(PP, G, blockIdx.x, gridDim.x);
-}
-
-// tileAlloc (wgsl-blocks.js:26-33), deterministic pop order
-__device__ __forceinline__ void tile_alloc_body(const DGrid& G, uint32_t bid, uint32_t nbid) {
-  uint32_t nn = G.ctl[3], top1 = G.ctl[13], nalloc = G.ctl[14];
-  for (uint32_t k = bid * blockDim.x + threadIdx.x; k < nn; k += nbid * blockDim.x) {
-    if (k < nalloc) {
-      uint32_t s = G.fstack[top1 - 1u - k], t = G.newList[k * 2], idx = G.newList[k * 2 + 1];
+  const uint32_t top1 = G.ctl[13], nalloc = G.ctl[14], t0 = bid * TB + threadIdx.x * 4u;
+  uint32_t slot[4];
+  bool nd[4];
+  uint64_t flags = 0;  // new | kept << 32 (freed tiles are unmapped and not needed)
+  for (uint32_t q = 0; q < 4u; q++) {
+    const uint32_t t = t0 + q;
+    nd[q] = t < ntiles && G.need[t] != 0u;
+    slot[q] = t < ntiles ? G.tmap[t] : ST_NONE;
+    if (nd[q]) flags += slot[q] == ST_NONE ? 1ull : 1ull << 32;
+  }
+  uint64_t tot;
+  const uint64_t x = wg_scan_u64(flags, &tot);
+  uint32_t k = G.wg[bid * 2u] + uint32_t(x), kept = G.wg[bid * 2u + 1u] + uint32_t(x >> 32);
+  for (uint32_t q = 0; q < 4u; q++) {
+    if (!nd[q]) continue;
+    if (slot[q] != ST_NONE) {
+      G.slotList[kept + min(k, nalloc)] = slot[q];
+      kept++;
+      continue;
+    }
+    const uint32_t t = t0 + q, s = k < nalloc ? G.fstack[top1 - 1u - k] : ST_NONE;
+    G.newList[k * 2u] = t;
+    G.newList[k * 2u + 1u] = s;
+    if (s != ST_NONE) {
       G.tmap[t] = s;
       G.slotTile[s] = t;
-      G.slotList[idx] = s;
-      G.newList[k * 2 + 1] = s;
-    } else {
-      G.newList[k * 2 + 1] = ST_NONE;
+      G.slotList[kept + k] = s;
     }
+    k++;
+  }
+  if (threadIdx.x < 4u) scan_words(G, nb, false)[bid * 4u + threadIdx.x] = 0ull;
+  if (bid == 0u && threadIdx.x == 0u) {
+    G.scanW[0] = 0ull;
+    G.ctl[2] = top1 - nalloc;
   }
 }
-__global__ void k_tile_alloc(DGrid G) {
-  tile_alloc_body(G, blockIdx.x, gridDim.x);
+__global__ void __launch_bounds__(WG) k_tiles_place(const DParams* __restrict__ PP, DGrid G) {
+  tiles_place_body(PP, G, blockIdx.x, gridDim.x);
 }
 
 // Slots of the 27 tiles around every tile in use (itself included), index
@@ -398,9 +427,6 @@ __device__ __forceinline__ void nbr_body(const DParams* __restrict__ PP, const D
     G.nbrL[e] = v;
   }
 }
-__global__ void k_nbr(const DParams* __restrict__ PP, DGrid G) {
-  nbr_body(PP, G, blockIdx.x, gridDim.x);
-}
 
 // initNew (wgsl-blocks.js:38-47): no pressure, collider lookup of each cell
 __device__ __forceinline__ void init_new_body(const DParams* __restrict__ PP, const DCols* __restrict__ C, const DGrid& G,
@@ -422,9 +448,6 @@ __device__ __forceinline__ void init_new_body(const DParams* __restrict__ PP, co
     }
   }
 }
-__global__ void k_init_new(const DParams* __restrict__ PP, const DCols* __restrict__ C, DGrid G) {
-  init_new_body(PP, C, G, blockIdx.x, gridDim.x);
-}
 
 // ---------------------------------------------------------------------------
 // clearSlots (wgsl-solver.js:5-15): the counts and face sums of the slots in use
@@ -444,8 +467,53 @@ __device__ __forceinline__ void clear_body(const DGrid& G, uint32_t bid, uint32_
     G.rhs[c] = 8.0f;
   }
 }
-__global__ void k_clear(DGrid G) {
-  clear_body(G, blockIdx.x, gridDim.x);
+
+__device__ __forceinline__ void foam_table_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid);
+
+// The rest of the tile bookkeeping (after tiles_place): the first workgroups list
+// the slots in use in Morton order (coopList, for the resident SOR); the others
+// make the neighbour rows and the cells of new tiles, clear the marks and bin
+// counts for the next positions (g2p's, or the mark pass's) and the streaming
+// SOR's barrier words, and, when a whole substep follows (`full`), clear the spare
+// slot and tabulate g2p's density factors.
+__device__ __forceinline__ void tiles_finish_body(const DParams* __restrict__ PP, const DCols* __restrict__ C, const DGrid& G, uint32_t full,
+                                                  uint32_t bid, uint32_t nbid) {
+  const uint32_t ntiles = PP->ntiles, nb = scan_blocks_of(ntiles);
+  if (bid < nb) {
+    __shared__ unsigned long long pre[1];
+    const uint32_t b = scan_ticket(G.scanW + 1);
+    if (b >= nb) return;
+    uint32_t slot[4];
+    uint64_t used = 0, tot;
+    for (uint32_t q = 0; q < 4u; q++) {
+      const uint32_t m = b * TB + threadIdx.x * 4u + q;
+      slot[q] = m < ntiles ? G.tmap[G.mortonTiles[m]] : ST_NONE;
+      used += slot[q] != ST_NONE ? 1u : 0u;
+    }
+    uint64_t at = wg_scan_u64(used, &tot);
+    const uint64_t agg[1] = {tot};
+    scan_chain<1>(scan_words(G, nb, true), b, agg, pre, G.sorBar + COOP_MAX_WG + 1);
+    at += pre[0];
+    for (uint32_t q = 0; q < 4u; q++)
+      if (slot[q] != ST_NONE) G.coopList[at++] = slot[q];
+    return;
+  }
+  bid -= nb;
+  nbid -= nb;
+  nbr_body(PP, G, bid, nbid);
+  init_new_body(PP, C, G, bid, nbid);
+  for (uint32_t t = bid * WG + threadIdx.x; t <= ntiles; t += nbid * WG) {
+    if (t < ntiles) G.need[t] = 0u;
+    G.binCount[t] = 0u;
+  }
+  for (uint32_t q = bid * WG + threadIdx.x; q < COOP_MAX_WG + 1u; q += nbid * WG) G.sorBar[q < COOP_MAX_WG ? q : COOP_MAX_WG + 2u] = 0u;
+  if (full) {
+    clear_body(G, bid, nbid);
+    foam_table_body(PP, G, bid, nbid);
+  }
+}
+__global__ void __launch_bounds__(WG) k_tiles_finish(const DParams* __restrict__ PP, const DCols* __restrict__ C, DGrid G, uint32_t full) {
+  tiles_finish_body(PP, C, G, full, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -656,7 +724,7 @@ __device__ __forceinline__ void p2g_tile_body(const DParams* __restrict__ PP, co
     }
     __syncthreads();
   }
-  // fastest particle: one partial per workgroup (k_reduce_stats folds them into
+  // fastest particle: one partial per workgroup (k_p2g_merge folds them into
   // ctl[6]); same-address atomics from every wave would serialise chip-wide
   __shared__ uint32_t wmax[W / 64];
   vmaxBits = wave_max_u32(vmaxBits);
@@ -694,8 +762,22 @@ constexpr BoundaryCells boundary_cells() {
 }
 __constant__ BoundaryCells kBoundary = boundary_cells();
 
+// The last workgroup also folds p2g's per-workgroup partials (p2g ran as many
+// workgroups) into ctl[6], the fastest particle.
 __device__ __forceinline__ void p2g_merge_body(const DGrid& G, uint32_t bid, uint32_t nbid) {
   const uint32_t sc = G.ctl[4];
+  if (bid == nbid - 1u) {
+    __shared__ uint32_t ws[P2G_MERGE_WG / 64];
+    uint32_t m = 0;
+    for (uint32_t i = threadIdx.x; i < nbid; i += P2G_MERGE_WG) m = max(m, G.part[i]);
+    m = wave_max_u32(m);
+    if (lane_id() == 0) ws[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (uint32_t q = 1; q < P2G_MERGE_WG / 64; q++) m = max(m, ws[q]);
+      G.ctl[6] = max(G.ctl[6], m);
+    }
+  }
   for (uint32_t b = bid; b < sc; b += nbid) {
     const uint32_t s = G.slotList[b];
     const uint32_t* nb = G.nbr + s * 27u;
@@ -723,32 +805,27 @@ __device__ __forceinline__ void p2g_merge_body(const DGrid& G, uint32_t bid, uin
 }
 __global__ void __launch_bounds__(P2G_MERGE_WG) k_p2g_merge(DGrid G) { p2g_merge_body(G, blockIdx.x, gridDim.x); }
 
-// statistics partials -> control words: which 0: ctl[6] = max(ctl[6], vmax
-// partials); which 1: ctl[0], ctl[1] = sums of the per-colour fluid partials
-__device__ __forceinline__ void reduce_stats_body(const DGrid& G, uint32_t n, uint32_t which, uint32_t bid, uint32_t nbid) {
-  __shared__ uint32_t ws[2][1024 / 64];
+// classify's per-workgroup fluid counts (n workgroups) into ctl[0] and ctl[1], by
+// one workgroup of WG threads: the last one of normFaces, or k_fluid_counts where
+// a caller stops at classify
+__device__ __forceinline__ void fluid_counts_body(const DGrid& G, uint32_t n) {
+  __shared__ uint32_t ws[2][WG / 64];
   uint32_t a = 0, b = 0;
-  for (uint32_t i = threadIdx.x; i < n; i += 1024) {
-    if (which == 0) a = max(a, G.part[i]);
-    else { a += G.part[2 * i]; b += G.part[2 * i + 1]; }
+  for (uint32_t i = threadIdx.x; i < n; i += WG) {
+    a += G.part[2 * i];
+    b += G.part[2 * i + 1];
   }
-  if (which == 0) a = wave_max_u32(a);
-  else { a = wave_sum_u32(a); b = wave_sum_u32(b); }
+  a = wave_sum_u32(a);
+  b = wave_sum_u32(b);
   if (lane_id() == 0) { ws[0][threadIdx.x >> 6] = a; ws[1][threadIdx.x >> 6] = b; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    uint32_t x = 0, y = 0;
-    for (int q = 0; q < 1024 / 64; q++) {
-      if (which == 0) x = max(x, ws[0][q]);
-      else { x += ws[0][q]; y += ws[1][q]; }
-    }
-    if (which == 0) G.ctl[6] = max(G.ctl[6], x);
-    else { G.ctl[0] = x; G.ctl[1] = y; }
+    for (uint32_t q = 1; q < WG / 64; q++) { a += ws[0][q]; b += ws[1][q]; }
+    G.ctl[0] = a;
+    G.ctl[1] = b;
   }
 }
-__global__ void __launch_bounds__(1024) k_reduce_stats(DGrid G, uint32_t n, uint32_t which) {
-  reduce_stats_body(G, n, which, blockIdx.x, gridDim.x);
-}
+__global__ void __launch_bounds__(WG) k_fluid_counts(DGrid G, uint32_t n) { fluid_counts_body(G, n); }
 
 // ---------------------------------------------------------------------------
 // per active cell kernels: t -> slot slotList[t >> 9], local t & 511 (acell,
@@ -834,6 +911,7 @@ __global__ void __launch_bounds__(WG) k_classify(const DParams* __restrict__ PP,
 __device__ __forceinline__ void norm_faces_body(const DParams* __restrict__ PP, const DCols* __restrict__ C, const DGrid& G,
                                                 uint32_t bid, uint32_t nbid) {
   const DParams& P = *PP;
+  if (bid == nbid - 1u) fluid_counts_body(G, nbid);  // classify ran as many workgroups
   FOR_ACTIVE(G) {
     uint32_t s = G.slotList[t >> 9], local = t & 511u, c = s * 512u + local;
     int3 at = d_slotCoord(P, G.slotTile, s, local);
@@ -863,7 +941,7 @@ __device__ __forceinline__ void norm_faces_body(const DParams* __restrict__ PP, 
     }
   }
 }
-__global__ void k_norm_faces(const DParams* __restrict__ PP, const DCols* __restrict__ C, DGrid G) {
+__global__ void __launch_bounds__(WG) k_norm_faces(const DParams* __restrict__ PP, const DCols* __restrict__ C, DGrid G) {
   norm_faces_body(PP, C, G, blockIdx.x, gridDim.x);
 }
 
@@ -1139,6 +1217,7 @@ __device__ __forceinline__ void sor_pipe_body(const DParams* __restrict__ PP, co
                                               float* __restrict__ pout, uint32_t seq, uint32_t bid, uint32_t nbid) {
   __shared__ SorPipeLds L;
   if (G.sorBar[COOP_MAX_WG] == seq) return;
+  if (bid == 0u && threadIdx.x == 0u) G.sorBar[COOP_MAX_WG + 3] = 0u;  // the path of this solve
   sor_pipe_init(L, threadIdx.x);
   sor_pipe_pass(G, PP->omega, pin, pout, bid, nbid, threadIdx.x, L);
 }
@@ -1589,16 +1668,6 @@ __global__ void __launch_bounds__(COOP_WG) k_sor_resident(const DParams* __restr
   sor_resident_body(PP, G, iters, seq, stream, blockIdx.x, gridDim.x);
 }
 
-// Morton-ordered list of the slots in use (coopList) for the resident SOR
-__global__ void k_coop_flags(const DParams* __restrict__ PP, DGrid G) {
-  uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m < PP->ntiles) G.coopFlags[m] = G.tmap[G.mortonTiles[m]] != ST_NONE ? 1u : 0u;
-}
-__global__ void k_coop_compact(const DParams* __restrict__ PP, DGrid G) {
-  uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m < PP->ntiles && G.coopFlags[m]) G.coopList[G.coopOffs[m]] = G.tmap[G.mortonTiles[m]];
-}
-
 // after an odd number of iterations the result sits in the partner buffer
 __device__ __forceinline__ void copy_tiles_body(const DGrid& G, const float* __restrict__ src, float* __restrict__ dst,
                                                 uint32_t seq, uint32_t bid, uint32_t nbid) {
@@ -1872,9 +1941,6 @@ __device__ __forceinline__ float4 d_foamRow(const DParams& P, float csum) {
 __device__ __forceinline__ void foam_table_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid) {
   for (uint32_t t = bid * blockDim.x + threadIdx.x; t < FOAM_TAB; t += nbid * blockDim.x)
     G.foamTab[t] = d_foamRow(*PP, float(t));
-}
-__global__ void k_foam_table(const DParams* __restrict__ PP, DGrid G) {
-  foam_table_body(PP, G, blockIdx.x, gridDim.x);
 }
 
 template <class GridT>
@@ -2497,35 +2563,17 @@ __global__ void __launch_bounds__(WG) kb_mark_bin(BATCH_ARGS) {
   const DGrid G = T.G;  // local: the body's stores cannot touch it
   mark_bin_body(TP, G, b.blk, b.nblk);
 }
-__global__ void __launch_bounds__(WG) kb_tile_count(BATCH_ARGS) { BATCH_TANK; tile_count_body(TP, T.G, b.blk, b.nblk); }
-__global__ void __launch_bounds__(1024) kb_tile_scan(BATCH_ARGS) {
-  BATCH_TANK;
-  tile_scan_body(T.G, (TP->ntiles + WG - 1u) / WG, b.blk, b.nblk);
-}
-__global__ void __launch_bounds__(WG) kb_tile_scatter(BATCH_ARGS) { BATCH_TANK; tile_scatter_body(TP, T.G, b.blk, b.nblk); }
-__global__ void kb_tile_alloc(BATCH_ARGS) { BATCH_TANK; tile_alloc_body(T.G, b.blk, b.nblk); }
-__global__ void kb_init_new(BATCH_ARGS) { BATCH_TANK; init_new_body(TP, TC, T.G, b.blk, b.nblk); }
-__global__ void kb_nbr(BATCH_ARGS) { BATCH_TANK; nbr_body(TP, T.G, b.blk, b.nblk); }
-// the bin scan: binCount (ntiles + 1 entries) to binStart
-__global__ void __launch_bounds__(WG) kb_scan_blocks(BATCH_ARGS) {
-  BATCH_TANK;
-  scan_blocks_body(T.G.binCount, T.G.binStart, TP->ntiles + 1u, T.G.scanTmp, b.blk, b.nblk);
-}
-__global__ void __launch_bounds__(1024) kb_scan_top(BATCH_ARGS) {
-  BATCH_TANK;
-  const uint32_t n = TP->ntiles + 1u;
-  scan_top_body(T.G.scanTmp, (n + WG * 4u - 1u) / (WG * 4u), T.G.binStart, n, b.blk, b.nblk);
-}
-__global__ void __launch_bounds__(WG) kb_scan_add(BATCH_ARGS) {
-  BATCH_TANK;
-  scan_add_body(T.G.binStart, TP->ntiles + 1u, T.G.scanTmp, nullptr, b.blk, b.nblk);
-}
-__global__ void __launch_bounds__(WG) kb_bin_scatter(BATCH_ARGS) {
+__global__ void __launch_bounds__(WG) kb_tiles_scan(BATCH_ARGS) { BATCH_TANK; tiles_scan_body(TP, T.G); }
+__global__ void __launch_bounds__(WG) kb_tiles_place(BATCH_ARGS) {
   BATCH_TANK;
   const DGrid G = T.G;  // local: the body's stores cannot touch it
-  bin_scatter_body(TP, G, b.blk, b.nblk);
+  tiles_place_body(TP, G, b.blk, b.nblk);
 }
-__global__ void kb_clear(BATCH_ARGS) { BATCH_TANK; clear_body(T.G, b.blk, b.nblk); }
+__global__ void __launch_bounds__(WG) kb_tiles_finish(BATCH_ARGS) {
+  BATCH_TANK;
+  const DGrid G = T.G;
+  tiles_finish_body(TP, TC, G, 1u, b.blk, b.nblk);
+}
 __global__ void __launch_bounds__(WG) kb_p2g_tile(BATCH_ARGS) {
   BATCH_TANK;
   const DGrid G = T.G;  // local: the body's stores cannot touch it
@@ -2537,10 +2585,6 @@ __global__ void __launch_bounds__(P2G_MERGE_WG) kb_p2g_merge(BATCH_ARGS) {
   p2g_merge_body(G, b.blk, b.nblk);
 }
 // reduces the partials of the launch whose block table is `of`
-__global__ void __launch_bounds__(1024) kb_reduce_stats(BATCH_ARGS, const uint32_t* __restrict__ of, uint32_t which) {
-  BATCH_TANK;
-  reduce_stats_body(T.G, of[b.t + 1u] - of[b.t], which, b.blk, b.nblk);
-}
 __global__ void kb_solid_build(BATCH_ARGS) {
   BATCH_TANK;
   const DGrid G = T.G;  // local: the body's stores cannot touch it
@@ -2553,7 +2597,7 @@ __global__ void __launch_bounds__(WG) kb_classify(BATCH_ARGS) {
   const DGrid G = T.G;  // local: the body's stores cannot touch it
   classify_body(TP, G, b.blk, b.nblk);
 }
-__global__ void kb_norm_faces(BATCH_ARGS) { BATCH_TANK; BATCH_STAGED; norm_faces_body(&sP, TC, G, b.blk, b.nblk); }
+__global__ void __launch_bounds__(WG) kb_norm_faces(BATCH_ARGS) { BATCH_TANK; BATCH_STAGED; norm_faces_body(&sP, TC, G, b.blk, b.nblk); }
 __global__ void kb_divergence(BATCH_ARGS) { BATCH_TANK; BATCH_STAGED; divergence_body(&sP, G, b.blk, b.nblk); }
 // one SOR iteration, pres -> pres2 (odd = 0) or back; every tank's range is a
 // multiple of 8 workgroups starting at a multiple of 8, so a workgroup's place
@@ -2563,11 +2607,6 @@ __global__ void __launch_bounds__(WG) kb_sor_pipe(BATCH_ARGS, uint32_t odd) {
   sor_pipe_body(TP, T.G, odd ? T.G.pres2 : T.G.pres, odd ? T.G.pres : T.G.pres2, ST_NONE, b.blk, b.nblk);
 }
 __global__ void kb_copy_tiles(BATCH_ARGS) { BATCH_TANK; copy_tiles_body(T.G, T.G.pres2, T.G.pres, ST_NONE, b.blk, b.nblk); }
-// the path word of the solve just done: one launch per iteration
-__global__ void kb_sor_path(BATCH_ARGS) {
-  BATCH_TANK;
-  if (threadIdx.x == 0 && b.blk == 0) T.G.sorBar[COOP_MAX_WG + 3] = 0u;
-}
 // Batched resident SOR.  The tanks' solves run in one cooperative launch of
 // the resident workgroups (one per CU): each tank gets a range of them, in one
 // of a few phases when all tanks' tiles do not fit in LDS at once, and runs
@@ -2575,36 +2614,8 @@ __global__ void kb_sor_path(BATCH_ARGS) {
 // words).  A tank's workgroups only wait on each other, and every workgroup
 // goes through the phases in order, so a phase never waits on a later one.
 // Per tank active this substep (its range in the first iteration's table is
-// not empty): kb_coop_lists (one 1024-thread workgroup per tank) builds its
-// Morton-ordered slot list, as k_coop_flags / scan / k_coop_compact do, and
-// clears its barrier words; kb_sor_plan (one thread) assigns the workgroups.
-__global__ void __launch_bounds__(1024) kb_coop_lists(const BTank* __restrict__ TT, const uint32_t* __restrict__ act, uint32_t nt) {
-  const uint32_t t = blockIdx.x, tid = threadIdx.x;
-  if (t >= nt || act[t + 1] == act[t]) return;
-  const DGrid G = TT[t].G;
-  const uint32_t ntl = TT[t].P->ntiles;
-  __shared__ uint32_t wsum[1024 / 64];
-  for (uint32_t q = tid; q < COOP_MAX_WG; q += 1024u) G.sorBar[q] = 0u;
-  if (tid == 0u) G.sorBar[COOP_MAX_WG + 2] = 0u;
-  uint32_t base = 0;
-  for (uint32_t m0 = 0; m0 < ntl; m0 += 1024u) {
-    const uint32_t m = m0 + tid;
-    const uint32_t sl = m < ntl ? G.tmap[G.mortonTiles[m]] : ST_NONE;
-    const uint32_t f = sl != ST_NONE ? 1u : 0u;
-    const uint64_t bal = __ballot(f != 0u);
-    const uint32_t inWave = uint32_t(__popcll(bal & lanemask_lt()));
-    if (lane_id() == 0u) wsum[tid >> 6] = uint32_t(__popcll(bal));
-    __syncthreads();
-    uint32_t before = 0, tot = 0;
-    for (uint32_t u = 0; u < 1024u / 64u; u++) {
-      if (u < (tid >> 6)) before += wsum[u];
-      tot += wsum[u];
-    }
-    if (f) G.coopList[base + before + inWave] = sl;
-    base += tot;
-    __syncthreads();
-  }
-}
+// not empty), kb_sor_plan (one thread) assigns the workgroups; tiles_finish has
+// listed its slots in Morton order and cleared its barrier words.
 
 // plan[3 t .. 3 t + 2] = (phase, first workgroup, workgroups) of tank t (phase
 // ST_NONE: no solve), plan[3 nt] = phases.  First fit in tank order, each tank
@@ -2669,7 +2680,6 @@ __global__ void __launch_bounds__(COOP_WG) kb_sor_resident(const BTank* __restri
 }
 
 __global__ void kb_project(BATCH_ARGS) { BATCH_TANK; BATCH_STAGED; project_body(&sP, G, b.blk, b.nblk); }
-__global__ void kb_foam_table(BATCH_ARGS) { BATCH_TANK; foam_table_body(TP, T.G, b.blk, b.nblk); }
 __global__ void __launch_bounds__(WG, 4) kb_g2p_tile(BATCH_ARGS) {
   BATCH_TANK;
   __shared__ DParams sP;
@@ -2689,6 +2699,15 @@ void launch_fill_u32(hipStream_t st, uint32_t* p, size_t n, uint32_t v) {
   hipLaunchKernelGGL(k_fill_u32, dim3(g), dim3(WG), 0, st, p, n, v);
 }
 
+// the tile marks and bin counts to zero, unless tiles_finish left them so
+static void launch_marks_clear(hipStream_t st, const LaunchCtx& L) {
+  if (L.marksClean) return;
+  launch_fill_u32(st, L.G.need, L.ntiles, 0u);
+  launch_fill_u32(st, L.G.binCount, size_t(L.ntiles) + 1, 0u);
+}
+// workgroups of tiles_finish beside the list's: a few hundred words per tile in use at most
+static uint32_t tiles_finish_grid(uint32_t scap) { return std::max<uint32_t>(8u, std::min<uint32_t>(scap, 2048u)); }
+
 static void launch_scan(hipStream_t st, const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* sums, uint32_t* copy) {
   uint32_t nb = gridFor(n, WG * 4);
   hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(WG), 0, st, in, out, n, sums);
@@ -2697,31 +2716,19 @@ static void launch_scan(hipStream_t st, const uint32_t* in, uint32_t* out, uint3
 }
 
 void launch_blocks(hipStream_t st, const LaunchCtx& L) {
-  uint32_t nt = L.ntiles;
+  const uint32_t nt = L.ntiles, nb = scan_blocks_of(nt);
   if (!L.binned) {  // else the last g2p already marked and counted A's positions
-    launch_fill_u32(st, L.G.need, nt, 0u);
-    launch_fill_u32(st, L.G.binCount, size_t(nt) + 1, 0u);
+    launch_marks_clear(st, L);
     if (L.n) hipLaunchKernelGGL(k_mark_bin, dim3(gridFor(L.n, WG)), dim3(WG), 0, st, L.P, L.G);
   }
   // narrow band: last step's tiles holding water by depth, and on a start the
   // tiles the starting water reaches (both before the counters reset)
   if (L.nbOn && L.initStep != 1) hipLaunchKernelGGL(k_nb_mark_phi, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G);
   if (L.initStep) hipLaunchKernelGGL(k_nb_mark_fill, dim3(gridFor(nt, WG)), dim3(WG), 0, st, L.P, L.C, L.G);
-  uint32_t nwg = gridFor(nt, WG);
-  hipLaunchKernelGGL(k_tile_count, dim3(nwg), dim3(WG), 0, st, L.P, L.G);
-  hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(1024), 0, st, L.G, nwg);
-  hipLaunchKernelGGL(k_tile_scatter, dim3(nwg), dim3(WG), 0, st, L.P, L.G);
-  hipLaunchKernelGGL(k_tile_alloc, dim3(std::max<uint32_t>(1u, std::min<uint32_t>(gridFor(nt, WG), 256u))), dim3(WG), 0, st, L.G);
-  hipLaunchKernelGGL(k_init_new, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.C, L.G);
-  hipLaunchKernelGGL(k_nbr, dim3(std::max<uint32_t>(1u, std::min<uint32_t>(gridFor(size_t(L.scap) * 27, WG), 2048u))), dim3(WG), 0, st, L.P, L.G);
+  hipLaunchKernelGGL(k_tiles_scan, dim3(nb), dim3(WG), 0, st, L.P, L.G);
+  hipLaunchKernelGGL(k_tiles_place, dim3(nb + gridFor(L.n, WG * 4)), dim3(WG), 0, st, L.P, L.G);
+  hipLaunchKernelGGL(k_tiles_finish, dim3(nb + tiles_finish_grid(L.scap)), dim3(WG), 0, st, L.P, L.C, L.G, L.full ? 1u : 0u);
   if (L.initStep) hipLaunchKernelGGL(k_nb_phi_init, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.C, L.G);
-  // particle bins: exclusive scan of the counts, then the bin list
-  launch_scan(st, L.G.binCount, L.G.binStart, nt + 1, L.G.scanTmp, nullptr);
-  if (L.n) hipLaunchKernelGGL(k_bin_scatter, dim3(gridFor(L.n, WG)), dim3(WG), 0, st, L.P, L.G);
-}
-
-void launch_clear(hipStream_t st, const LaunchCtx& L) {
-  hipLaunchKernelGGL(k_clear, dim3(512 / WG), dim3(WG), 0, st, L.G);
 }
 
 void launch_p2g(hipStream_t st, const LaunchCtx& L) {
@@ -2732,13 +2739,12 @@ void launch_p2g(hipStream_t st, const LaunchCtx& L) {
   if (L.fullTiles < 2048u) hipLaunchKernelGGL(k_p2g_tile<512>, dim3(L.tileGrid), dim3(512), 0, st, L.P, L.G);
   else hipLaunchKernelGGL(k_p2g_tile<256>, dim3(L.tileGrid), dim3(256), 0, st, L.P, L.G);
   hipLaunchKernelGGL(k_p2g_merge, dim3(L.tileGrid), dim3(P2G_MERGE_WG), 0, st, L.G);
-  hipLaunchKernelGGL(k_reduce_stats, dim3(1), dim3(1024), 0, st, L.G, L.tileGrid, 0u);
 }
 
-void launch_classify(hipStream_t st, const LaunchCtx& L, bool solid) {
+void launch_classify(hipStream_t st, const LaunchCtx& L, bool solid, bool counts) {
   if (solid) hipLaunchKernelGGL(k_solid_build, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.C, L.G);
   hipLaunchKernelGGL(k_classify, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G);
-  hipLaunchKernelGGL(k_reduce_stats, dim3(1), dim3(1024), 0, st, L.G, L.cellGrid, 1u);
+  if (counts) hipLaunchKernelGGL(k_fluid_counts, dim3(1), dim3(WG), 0, st, L.G, L.cellGrid);
   if (L.nbOn) hipLaunchKernelGGL(k_nb_vel, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G);
 }
 
@@ -2806,15 +2812,13 @@ void morton_tiles(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t* out) {
 hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters) {
   hipError_t coopErr = hipSuccess;
   if (L.coopGrid && iters > 0) {
-    // active slots in Morton order, cleared barrier flags, then the whole solve
-    // in one cooperative launch (resident when the tiles fit in LDS, streaming
-    // tile windows otherwise)
-    uint32_t nt = L.ntiles, g = gridFor(nt, WG);
-    hipLaunchKernelGGL(k_coop_flags, dim3(g), dim3(WG), 0, st, L.P, L.G);
-    launch_scan(st, L.G.coopFlags, L.G.coopOffs, nt, L.G.scanTmp, nullptr);
-    hipLaunchKernelGGL(k_coop_compact, dim3(g), dim3(WG), 0, st, L.P, L.G);
-    launch_fill_u32(st, L.G.sorBar, COOP_MAX_WG, 0u);
-    launch_fill_u32(st, L.G.sorBar + COOP_MAX_WG + 2, 1, 0u);
+    // the whole solve in one cooperative launch (resident when the tiles fit in
+    // LDS, streaming tile windows otherwise); the blocks stage has listed the
+    // slots and cleared the streaming mode's barrier words for one solve
+    if (!L.barClean) {
+      launch_fill_u32(st, L.G.sorBar, COOP_MAX_WG, 0u);
+      launch_fill_u32(st, L.G.sorBar + COOP_MAX_WG + 2, 1, 0u);
+    }
     const DParams* P = L.P;
     DGrid G = L.G;
     uint32_t it = uint32_t(iters), seq = L.sorSeq, stream = L.sorStream ? 1u : 0u;
@@ -2832,7 +2836,6 @@ hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters) {
   }
   if (iters & 1)
     hipLaunchKernelGGL(k_copy_tiles, dim3(L.cellGrid), dim3(WG), 0, st, L.G, (const float*)L.G.pres2, L.G.pres, L.sorSeq);
-  launch_fill_u32(st, L.G.sorBar + COOP_MAX_WG + 3, 1, 0u);
   return coopErr;
 }
 
@@ -2858,11 +2861,7 @@ uint32_t g2p_split(uint32_t fullTiles) { return fullTiles < 48u ? 8u : fullTiles
 
 void launch_g2p(hipStream_t st, const LaunchCtx& L) {
   if (!L.n) return;
-  if (L.binNext) {  // the next substep's tile marks and bin counts start here
-    launch_fill_u32(st, L.G.need, L.ntiles, 0u);
-    launch_fill_u32(st, L.G.binCount, size_t(L.ntiles) + 1, 0u);
-  }
-  hipLaunchKernelGGL(k_foam_table, dim3(FOAM_TAB / WG), dim3(WG), 0, st, L.P, L.G);
+  if (L.binNext) launch_marks_clear(st, L);  // the next substep's tile marks and bin counts start here
   const uint32_t split = g2p_split(L.fullTiles);
   uint32_t g = std::min<uint32_t>(L.ntiles * split, 8192u);
   hipLaunchKernelGGL(k_g2p_tile, dim3(g), dim3(WG), 0, st, L.P, L.C, L.G, L.binNext ? 1u : 0u, split);
@@ -2875,6 +2874,8 @@ void launch_unsort(hipStream_t st, const float4* src, const uint32_t* pid, float
 
 // ---------------------------------------------------------------------------
 // batched substep (host side)
+
+size_t scan_word_count(uint32_t ntiles) { return 2u + 5u * size_t(scan_blocks_of(ntiles)); }
 
 size_t batch_table_words(uint32_t nt, uint32_t itersMax) { return size_t(BT_PIPE0 + itersMax) * (nt + 1u); }
 
@@ -2906,24 +2907,19 @@ void batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t itersMax, uint32_
       uint32_t c = 0;
       if (p.n) {
         const uint32_t cell = batch_share(BATCH_CELL_WG, p.scap, scapTot, std::max<uint32_t>(1u, std::min<uint32_t>(p.scap * 2u, 4096u)));
-        const uint32_t nwg = gridFor(p.ntiles, WG), bins = gridFor(size_t(p.ntiles) + 1u, WG);
+        const uint32_t nb = scan_blocks_of(p.ntiles), bins = gridFor(size_t(p.ntiles) + 1u, WG);
         switch (k) {
-          case BT_FILL_MARK: c = p.binned ? 0u : bins; break;
+          case BT_FILL_MARK: c = p.binned || p.marksClean ? 0u : bins; break;
           case BT_MARK: c = p.binned ? 0u : gridFor(p.n, WG); break;
-          case BT_NWG: c = nwg; break;
+          case BT_SCAN: c = nb; break;
+          case BT_PLACE: c = nb + gridFor(p.n, WG * 4u); break;
+          case BT_FINISH: c = nb + batch_share(BATCH_CELL_WG, p.scap, scapTot, tiles_finish_grid(p.scap)); break;
           case BT_ONE: c = 1u; break;
-          case BT_ALLOC: c = std::max<uint32_t>(1u, std::min<uint32_t>(nwg, 256u)); break;
           case BT_CELL: c = cell; break;
-          case BT_NBR: c = std::max<uint32_t>(1u, std::min<uint32_t>(gridFor(size_t(p.scap) * 27u, WG), 2048u)); break;
-          case BT_SCAN: c = gridFor(size_t(p.ntiles) + 1u, WG * 4u); break;
-          case BT_PART: c = gridFor(p.n, WG); break;
           case BT_TILE: c = batch_share(BATCH_TILE_WG, p.scap, scapTot, std::max<uint32_t>(1u, std::min<uint32_t>(p.scap, 8192u))); break;
-          case BT_ONE_N: c = 1u; break;
           case BT_SOLID: c = p.solid ? cell : 0u; break;
           case BT_COPY: c = (p.iters & 1u) ? cell : 0u; break;
-          case BT_FOAM: c = FOAM_TAB / WG; break;
           case BT_G2P: c = batch_share(BATCH_TILE_WG, p.ntiles + 1u, binTot, std::min<uint32_t>((p.ntiles + 1u) * p.split, 8192u)); break;
-          case BT_FILL_NEXT: c = bins; break;
           default: {
             // SOR: the tank's share of the resident workgroups by pool size,
             // whole groups of 8, at least one group and at most one workgroup
@@ -2950,36 +2946,25 @@ bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, co
   auto tot = [&](uint32_t k) { return htab[k * w + nt]; };
 #define BLAUNCH(kern, k, threads, ...) \
   if (tot(k)) hipLaunchKernelGGL(kern, dim3(tot(k)), dim3(threads), 0, st, dT, tab(k), nt, ##__VA_ARGS__)
-  // blocks: marks and bins (unless the last g2p made them), tile allocation,
-  // neighbour slots, bin scan and bin list
+  // blocks: marks and bins (unless the last g2p made them), the tile bookkeeping
+  // and what it clears
   BLAUNCH(kb_fill_bins, BT_FILL_MARK, WG);
   BLAUNCH(kb_mark_bin, BT_MARK, WG);
-  BLAUNCH(kb_tile_count, BT_NWG, WG);
-  BLAUNCH(kb_tile_scan, BT_ONE, 1024);
-  BLAUNCH(kb_tile_scatter, BT_NWG, WG);
-  BLAUNCH(kb_tile_alloc, BT_ALLOC, WG);
-  BLAUNCH(kb_init_new, BT_CELL, WG);
-  BLAUNCH(kb_nbr, BT_NBR, WG);
-  BLAUNCH(kb_scan_blocks, BT_SCAN, WG);
-  BLAUNCH(kb_scan_top, BT_ONE, 1024);
-  BLAUNCH(kb_scan_add, BT_SCAN, WG);
-  BLAUNCH(kb_bin_scatter, BT_PART, WG);
-  // clear, p2g
-  BLAUNCH(kb_clear, BT_CELL, WG);
+  BLAUNCH(kb_tiles_scan, BT_SCAN, WG);
+  BLAUNCH(kb_tiles_place, BT_PLACE, WG);
+  BLAUNCH(kb_tiles_finish, BT_FINISH, WG);
+  // p2g
   BLAUNCH(kb_p2g_tile, BT_TILE, WG);
   BLAUNCH(kb_p2g_merge, BT_TILE, P2G_MERGE_WG);
-  BLAUNCH(kb_reduce_stats, BT_ONE_N, 1024, tab(BT_TILE), 0u);
   // classify, normFaces, divergence
   BLAUNCH(kb_solid_build, BT_SOLID, WG);
   BLAUNCH(kb_classify, BT_CELL, WG);
-  BLAUNCH(kb_reduce_stats, BT_ONE, 1024, tab(BT_CELL), 1u);
   BLAUNCH(kb_norm_faces, BT_CELL, WG);
   BLAUNCH(kb_divergence, BT_CELL, WG);
   // pressure: the resident solves of all tanks in one cooperative launch, or
   // one launch per iteration (ping-pong between pres and pres2)
   bool resident = false;
   if (coopGrid && dPlan && itersMax) {
-    hipLaunchKernelGGL(kb_coop_lists, dim3(nt), dim3(1024), 0, st, dT, tab(BT_PIPE0), nt);
     hipLaunchKernelGGL(kb_sor_plan, dim3(1), dim3(64), 0, st, dT, tab(BT_PIPE0), nt, coopGrid, dPlan);
     const BTank* a0 = dT;
     const uint32_t* a1 = dPlan;
@@ -2991,12 +2976,9 @@ bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, co
   if (!resident) {
     for (uint32_t it = 0; it < itersMax; it++) BLAUNCH(kb_sor_pipe, uint32_t(BT_PIPE0) + it, WG, it & 1u);
     BLAUNCH(kb_copy_tiles, BT_COPY, WG);
-    BLAUNCH(kb_sor_path, BT_ONE, 64);
   }
   // project, g2p (which marks and bins the next substep)
   BLAUNCH(kb_project, BT_CELL, WG);
-  BLAUNCH(kb_fill_bins, BT_FILL_NEXT, WG);
-  BLAUNCH(kb_foam_table, BT_FOAM, WG);
   BLAUNCH(kb_g2p_tile, BT_G2P, WG);
 #undef BLAUNCH
   return resident;
