@@ -177,6 +177,7 @@ struct Sim {
     L.scap = scap;
     L.cellGrid = std::max<uint32_t>(1u, std::min<uint32_t>(scap * 2u, 4096u));
     L.tileGrid = std::max<uint32_t>(1u, std::min<uint32_t>(scap, 8192u));
+    L.faceGrid = std::max<uint32_t>(1u, std::min<uint32_t>(scap * 2u, 8192u));
     L.pipeGrid = pipeOverride ? pipeOverride : std::min<uint32_t>((scap + 7u) & ~7u, sorResident);  // whole groups of 8 (one per XCD)
     L.coopGrid = sorMode == 1u ? 0u : coopGrid;
     L.sorStream = sorMode == 2u;
@@ -214,6 +215,7 @@ int allocSlots(Sim* s, uint32_t n) {
   if ((rc = dalloc(&s->G.slotList, n))) return rc;
   if ((rc = dalloc(&s->G.nbr, size_t(n) * 27))) return rc;
   if ((rc = dalloc(&s->G.nbrL, size_t(n) * 27))) return rc;
+  if ((rc = dalloc(&s->G.tileRec, size_t(n) * 3))) return rc;
   if ((rc = dalloc(&s->G.coopList, n))) return rc;
   if ((rc = dalloc(&s->G.sorHalo, size_t(n) * 2 * 6 * 32))) return rc;
   // tag 0 is never a half-sweep's tag, so no entry looks written before it is
@@ -224,7 +226,7 @@ int allocSlots(Sim* s, uint32_t n) {
 void freeSlotArrays(DGrid& g) {
   dfree(g.cnt); dfree(g.ctype); dfree(g.pres); dfree(g.pres2); dfree(g.rhs); dfree(g.sten);
   dfree(g.accV); dfree(g.accW); dfree(g.p2gHalo); dfree(g.velG);
-  dfree(g.slotTile); dfree(g.fstack); dfree(g.slotList); dfree(g.nbr); dfree(g.nbrL);
+  dfree(g.slotTile); dfree(g.fstack); dfree(g.slotList); dfree(g.nbr); dfree(g.nbrL); dfree(g.tileRec);
   dfree(g.coopList); dfree(g.sorHalo);
 }
 void freeSlots(Sim* s) { freeSlotArrays(s->G); }
@@ -1170,7 +1172,7 @@ int st_grow(void* p, uint32_t n) {
   DGrid keep = s->G;
   s->G.cnt = nullptr; s->G.ctype = nullptr; s->G.pres = nullptr; s->G.pres2 = nullptr; s->G.rhs = nullptr; s->G.sten = nullptr;
   s->G.accV = nullptr; s->G.accW = nullptr; s->G.p2gHalo = nullptr; s->G.velG = nullptr; s->G.slotTile = nullptr; s->G.fstack = nullptr;
-  s->G.slotList = nullptr; s->G.nbr = nullptr; s->G.nbrL = nullptr; s->G.coopList = nullptr; s->G.sorHalo = nullptr;
+  s->G.slotList = nullptr; s->G.nbr = nullptr; s->G.nbrL = nullptr; s->G.tileRec = nullptr; s->G.coopList = nullptr; s->G.sorHalo = nullptr;
   int rc = allocSlots(s, n);
   if (rc) { freeSlots(s); s->G = keep; return rc; }
   // the wg scratch and grid sizes follow the pool
@@ -1187,6 +1189,7 @@ int st_grow(void* p, uint32_t n) {
   HIPCHK(hipMemcpy(s->G.slotTile, keep.slotTile, size_t(old) * 4, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.fstack, keep.fstack, size_t(old) * 4, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.slotList, keep.slotList, size_t(old) * 4, hipMemcpyDeviceToDevice));
+  HIPCHK(hipMemcpy(s->G.tileRec, keep.tileRec, size_t(old) * 48, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.coopList, keep.coopList, size_t(old) * 4, hipMemcpyDeviceToDevice));
   rc = zeroSlots(s, old, n);
   if (rc) return rc;

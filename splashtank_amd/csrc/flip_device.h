@@ -99,6 +99,7 @@ struct DGrid {
   uint32_t* slotList;
   uint32_t* nbr;       // per slot: slots of the 27 tiles around it (0 none, WSLOT_OUT outside)
   uint32_t* nbrL;      // the same rows in slotList order (row b for slotList[b])
+  uint4* tileRec;      // three per slotList entry: slot, first cell (x, y, z), slots across the faces x-, x+, y-, y+, z-, z+ (0: none)
   uint32_t* wg;        // per scan block: new and kept tiles before it
   uint32_t* part;      // per-workgroup statistics partials (vmax; fluid cells per colour)
   uint32_t* ctl;       // control words, as in the reference's ctl

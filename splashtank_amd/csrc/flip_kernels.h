@@ -27,6 +27,7 @@ struct LaunchCtx {
   uint32_t scap;
   uint32_t cellGrid;  // workgroups of grid-stride loops over active cells
   uint32_t tileGrid;  // workgroups of loops with one workgroup per tile in use
+  uint32_t faceGrid;  // workgroups of the cell kernels that walk tiles in use (normFaces, divergence, project)
   uint32_t pipeGrid;  // persistent SOR workgroups (about eight per CU)
   uint32_t coopGrid;  // resident-SOR workgroups (one per CU), 0 when cooperative launches are unavailable
   uint32_t sorSeq;    // sequence number of this pressure solve
