@@ -121,6 +121,7 @@ struct Sim {
   uint32_t lcap = 0;
   uint32_t sorResident = 2048;  // SOR workgroups resident at once on this device
   uint32_t coopGrid = 0;        // resident-SOR workgroups (0: not available)
+  uint32_t sorTiles = 0;        // resident workgroups of the one-per-tile solve (0: not available)
   uint32_t sorSeq = 0;          // pressure solves so far
   uint32_t sorTag = 1;          // tag of the next substep's first halo exchange (0 is never used)
   uint32_t sorMode = 0;         // this step's pressure path (st_params.sor_mode, a tuned choice for 3)
@@ -181,6 +182,8 @@ struct Sim {
     L.pipeGrid = pipeOverride ? pipeOverride : std::min<uint32_t>((scap + 7u) & ~7u, sorResident);  // whole groups of 8 (one per XCD)
     L.coopGrid = sorMode == 1u ? 0u : coopGrid;
     L.sorStream = sorMode == 2u;
+    L.sorTiles = sorTiles;
+    L.sorTag = 0u;
     L.sorSeq = sorSeq;
     L.full = !onlyTiles;
     L.marksClean = marksClean;
@@ -216,17 +219,23 @@ int allocSlots(Sim* s, uint32_t n) {
   if ((rc = dalloc(&s->G.nbr, size_t(n) * 27))) return rc;
   if ((rc = dalloc(&s->G.nbrL, size_t(n) * 27))) return rc;
   if ((rc = dalloc(&s->G.tileRec, size_t(n) * 3))) return rc;
+  if ((rc = dalloc(&s->G.slotPos, n))) return rc;
+  if ((rc = dalloc(&s->G.posFluid, size_t(n) * 2 + 16))) return rc;  // read 16 bytes at a time
+  HIPCHK(hipMemsetAsync(s->G.posFluid, 0, size_t(n) * 2 + 16, s->st));
+  s->G.tileCap = std::min<uint32_t>(n, SOR_TILES_MAX);
+  if ((rc = dalloc(&s->G.sorTileW, size_t(s->G.tileCap) * 1024))) return rc;
+  HIPCHK(hipMemsetAsync(s->G.sorTileW, 0, size_t(s->G.tileCap) * 1024 * sizeof(uint64_t), s->st));
   if ((rc = dalloc(&s->G.coopList, n))) return rc;
   if ((rc = dalloc(&s->G.sorHalo, size_t(n) * 2 * 6 * 32))) return rc;
   // tag 0 is never a half-sweep's tag, so no entry looks written before it is
-  HIPCHK(hipMemset(s->G.sorHalo, 0, size_t(n) * 2 * 6 * 32 * sizeof(uint64_t)));
+  HIPCHK(hipMemsetAsync(s->G.sorHalo, 0, size_t(n) * 2 * 6 * 32 * sizeof(uint64_t), s->st));
   return ST_OK;
 }
 
 void freeSlotArrays(DGrid& g) {
   dfree(g.cnt); dfree(g.ctype); dfree(g.pres); dfree(g.pres2); dfree(g.rhs); dfree(g.sten);
   dfree(g.accV); dfree(g.accW); dfree(g.p2gHalo); dfree(g.velG);
-  dfree(g.slotTile); dfree(g.fstack); dfree(g.slotList); dfree(g.nbr); dfree(g.nbrL); dfree(g.tileRec);
+  dfree(g.slotTile); dfree(g.fstack); dfree(g.slotList); dfree(g.nbr); dfree(g.nbrL); dfree(g.tileRec); dfree(g.slotPos); dfree(g.posFluid); dfree(g.sorTileW);
   dfree(g.coopList); dfree(g.sorHalo);
 }
 void freeSlots(Sim* s) { freeSlotArrays(s->G); }
@@ -385,6 +394,22 @@ static float quietBelow(double c, float dt, float sens) {
   return f;
 }
 
+// Every exchange of a one-launch solve carries its own tag: a solve reserves
+// 2 iters + 2 (a batched step's through its parameter block, which each step
+// uploads anew).  When the counter would wrap, the words are cleared first so that
+// no old tag can match.
+uint32_t reserveTags(Sim* s) {
+  const uint32_t need = 2u * uint32_t(s->iters) + 2u;
+  if (s->sorTag > 0xffffffffu - need) {
+    launch_fill_u32(s->st, reinterpret_cast<uint32_t*>(s->G.sorHalo), size_t(s->scap) * 2 * 6 * 32 * 2, 0u);
+    launch_fill_u32(s->st, reinterpret_cast<uint32_t*>(s->G.sorTileW), size_t(s->G.tileCap) * 1024 * 2, 0u);
+    s->sorTag = 1;
+  }
+  const uint32_t t = s->sorTag;
+  s->sorTag += need;
+  return t;
+}
+
 int prepStep(Sim* s, const st_params* o, DParams& Pout, DCols& C) {
   if (s->N == 0) return fail(ST_ERR_STATE, "st_begin_step: no particles (step() does nothing when N = 0)");
   if (o->ocean_on && o->nwave > ST_OCEAN_MAX_WAVES) return fail(ST_ERR_ARG, "st_begin_step: nwave above ST_OCEAN_MAX_WAVES");
@@ -516,20 +541,8 @@ int prepStep(Sim* s, const st_params* o, DParams& Pout, DCols& C) {
   }
   s->extrapOnStep = o->only_tiles ? 0u : o->extrap_layers;
   s->iters = std::max(1, int(o->iters));
-  {
-    // Every halo exchange of a resident solve carries its own tag, taken from
-    // this block (so each replay of a captured substep gets new ones): the
-    // step reserves 2 iters + 2.  When the counter would wrap, the entries are
-    // cleared first so that no old tag can match.
-    const uint32_t need = 2u * uint32_t(s->iters) + 2u;
-    if (s->sorTag > 0xffffffffu - need) {
-      launch_fill_u32(s->st, reinterpret_cast<uint32_t*>(s->G.sorHalo), size_t(s->scap) * 2 * 6 * 32 * 2, 0u);
-      s->sorTag = 1;
-    }
-    P.sorTag = s->sorTag;
-    P.iters = uint32_t(s->iters);
-    s->sorTag += need;
-  }
+  P.sorTag = reserveTags(s);
+  P.iters = uint32_t(s->iters);
   Pout = P;
   size_t ncAll = std::min<size_t>(s->ncTotal, ST_MAX_COLS);
   std::memcpy(C.c, s->cf.data(), ncAll * 32 * sizeof(float));
@@ -588,6 +601,7 @@ int runStage(Sim* s, int stage, bool alone = false) {
     case ST_STAGE_PRESSURE:
       if (full) {
         L.sorSeq = ++s->sorSeq;
+        if (L.coopGrid) L.sorTag = reserveTags(s);
         if (launch_pressure(st, L, s->iters) != hipSuccess) s->coopGrid = 0;  // per-iteration launches from now on
         s->barClean = false;
       }
@@ -733,7 +747,7 @@ struct Batch {
   std::vector<Sim*> tanks;
   uint32_t sorResident = 2048;   // SOR workgroups of a batched iteration, over all tanks
   uint32_t coopGrid = 0;         // resident workgroups of the one-launch batched SOR (0: launches per iteration)
-  uint32_t* dPlan = nullptr;     // its per-tank workgroup plan (3 nt + 1 words)
+  uint32_t* dPlan = nullptr;     // its per-tank workgroup plan (batch_plan_words)
   uint32_t lastResident = 0;     // the last substep's SOR ran in the one launch
   // ring of step slots: tank records, parameter blocks, collider records, block
   // tables (host pinned and device), each reusable once its upload is done
@@ -893,6 +907,7 @@ int st_create(const st_opts* o, void** out) {
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, o->device));
     s->sorResident = sor_resident_grid(uint32_t(cus));
     s->coopGrid = sor_coop_grid(uint32_t(cus));
+    s->sorTiles = s->coopGrid ? sor_tiles_grid(uint32_t(cus)) : 0u;
   }
   double rt = o->ratio > 0 ? o->ratio : 2.0;
   rt = std::max(1.4, std::min(4.0, rt));
@@ -932,7 +947,7 @@ int st_create(const st_opts* o, void** out) {
       (rc = dalloc(&s->G.tmap, s->ntiles)) || (rc = dalloc(&s->G.need, s->ntiles)) || (rc = dalloc(&s->G.newList, size_t(s->ntiles) * 2)) ||
       (rc = dalloc(&s->G.wg, scan_word_count(s->ntiles))) || (rc = dalloc(&s->G.ctl, 16)) || (rc = allocSlots(s, s->scap)) ||
       (rc = dalloc(&s->G.part, 2 * 8192 + 64)) || (rc = dalloc(&s->G.foamTab, FOAM_TAB)) ||
-      (rc = dalloc(&s->G.mortonTiles, s->ntiles)) || (rc = dalloc(&s->G.sorBar, COOP_MAX_WG + 4)) ||
+      (rc = dalloc(&s->G.mortonTiles, s->ntiles)) || (rc = dalloc(&s->G.sorBar, COOP_MAX_WG + 5)) ||
       (rc = dalloc(&s->dSlots, RING))) {
     destroySim(s);
     return rc;
@@ -959,8 +974,8 @@ int st_create(const st_opts* o, void** out) {
   if (hipMemcpy(s->G.fstack, st.data(), size_t(s->scap) * 4, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(s->G.tmap, tm.data(), size_t(s->ntiles) * 4, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(s->G.mortonTiles, mort.data(), size_t(s->ntiles) * 4, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemset(s->G.sorBar, 0, (COOP_MAX_WG + 4) * 4) != hipSuccess ||
-      hipMemset(s->G.scanW, 0, scan_word_count(s->ntiles) * 8) != hipSuccess ||
+      hipMemsetAsync(s->G.sorBar, 0, (COOP_MAX_WG + 5) * 4, s->st) != hipSuccess ||
+      hipMemsetAsync(s->G.scanW, 0, scan_word_count(s->ntiles) * 8, s->st) != hipSuccess ||
       hipMemcpy(s->G.ctl, ctl, 64, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(s->G.pos, 0, M * 16) != hipSuccess || hipMemset(s->G.vel, 0, M * 16) != hipSuccess ||
       hipMemset(s->G.need, 0, size_t(s->ntiles) * 4) != hipSuccess) {
@@ -1172,7 +1187,8 @@ int st_grow(void* p, uint32_t n) {
   DGrid keep = s->G;
   s->G.cnt = nullptr; s->G.ctype = nullptr; s->G.pres = nullptr; s->G.pres2 = nullptr; s->G.rhs = nullptr; s->G.sten = nullptr;
   s->G.accV = nullptr; s->G.accW = nullptr; s->G.p2gHalo = nullptr; s->G.velG = nullptr; s->G.slotTile = nullptr; s->G.fstack = nullptr;
-  s->G.slotList = nullptr; s->G.nbr = nullptr; s->G.nbrL = nullptr; s->G.tileRec = nullptr; s->G.coopList = nullptr; s->G.sorHalo = nullptr;
+  s->G.slotList = nullptr; s->G.nbr = nullptr; s->G.nbrL = nullptr; s->G.tileRec = nullptr; s->G.slotPos = nullptr; s->G.posFluid = nullptr;
+  s->G.sorTileW = nullptr; s->G.coopList = nullptr; s->G.sorHalo = nullptr;
   int rc = allocSlots(s, n);
   if (rc) { freeSlots(s); s->G = keep; return rc; }
   // the wg scratch and grid sizes follow the pool
@@ -1189,6 +1205,8 @@ int st_grow(void* p, uint32_t n) {
   HIPCHK(hipMemcpy(s->G.slotTile, keep.slotTile, size_t(old) * 4, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.fstack, keep.fstack, size_t(old) * 4, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.slotList, keep.slotList, size_t(old) * 4, hipMemcpyDeviceToDevice));
+  HIPCHK(hipMemcpy(s->G.slotPos, keep.slotPos, size_t(old) * 4, hipMemcpyDeviceToDevice));
+  HIPCHK(hipMemcpy(s->G.posFluid, keep.posFluid, size_t(old) * 2, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.tileRec, keep.tileRec, size_t(old) * 48, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.coopList, keep.coopList, size_t(old) * 4, hipMemcpyDeviceToDevice));
   rc = zeroSlots(s, old, n);
@@ -1724,7 +1742,7 @@ int st_batch_create(void* const* sims, uint32_t n, void** out) {
   b->sorResident = b->tanks[0]->sorResident;
   b->coopGrid = b->tanks[0]->coopGrid;
   b->plan.resize(n);
-  if (b->coopGrid && dalloc(&b->dPlan, size_t(n) * 3 + 1) != ST_OK) {
+  if (b->coopGrid && dalloc(&b->dPlan, batch_plan_words(n)) != ST_OK) {
     (void)hipGetLastError();
     b->coopGrid = 0;  // launches per iteration
   }
@@ -1774,7 +1792,12 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
   DCols* hC = (DCols*)(h + b->offC);
   uint32_t* hTab = (uint32_t*)(h + b->offTab);
   uint32_t full = 0;
-  for (const Sim* s : b->tanks) full += s->fullTiles();
+  uint32_t most = 0;  // tiles the tanks can have in use
+  for (const Sim* s : b->tanks) {
+    if (!s->N) continue;
+    full += s->fullTiles();
+    most += std::min(s->ntiles, s->scap - 1u);
+  }
   const uint32_t split = g2p_split(full);
   for (uint32_t t = 0; t < nt; t++) {
     Sim* s = b->tanks[t];
@@ -1801,8 +1824,11 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
   HIPCHK(hipEventRecord(b->ev[k], b->st));
   b->ringPos++;
   if (!graph) {
-    b->lastResident = launch_batch_step(b->st, (const BTank*)d, (const uint32_t*)(d + b->offTab), hTab, nt, itersMax, b->coopGrid,
-                                        b->dPlan) ? 1u : 0u;
+    // a cap on the one-launch solve (st_batch_sor_grid) caps the one-per-tile form too
+    const Sim* s0 = b->tanks[0];
+    const uint32_t tiles = b->coopGrid < s0->coopGrid ? std::min(b->coopGrid, s0->sorTiles) : s0->sorTiles;
+    b->lastResident = launch_batch_step(b->st, (const BTank*)d, (const uint32_t*)(d + b->offTab), hTab, nt, itersMax, b->coopGrid, tiles,
+                                        most, full, b->dPlan) ? 1u : 0u;
   } else {
     // the block tables fix every launch's grid and kernel choice; the tank
     // records, parameters and tables are read from the graph slot at run time.
@@ -1817,7 +1843,7 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
       HIPCHK(hipGraphLaunch(hit->exec, b->st));
     } else {
       HIPCHK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
-      launch_batch_step(b->st, (const BTank*)d, (const uint32_t*)(d + b->offTab), hTab, nt, itersMax, 0u, nullptr);
+      launch_batch_step(b->st, (const BTank*)d, (const uint32_t*)(d + b->offTab), hTab, nt, itersMax, 0u, 0u, 0u, 0u, nullptr);
       hipError_t le = hipGetLastError();
       hipGraph_t g = nullptr;
       hipError_t ce = hipStreamEndCapture(b->st, &g);
@@ -1890,7 +1916,7 @@ int st_batch_sor_grid(void* p, uint32_t workgroups) {
   if (workgroups && !b->dPlan) {
     if (!most) return fail(ST_ERR_STATE, "st_batch_sor_grid: cooperative launches are not available on this device");
     HIPCHK(hipSetDevice(b->dev));
-    int rc = dalloc(&b->dPlan, b->tanks.size() * 3 + 1);
+    int rc = dalloc(&b->dPlan, batch_plan_words(uint32_t(b->tanks.size())));
     if (rc) return rc;
   }
   // a tank that streams tile windows runs four pipelines per workgroup over

@@ -99,6 +99,10 @@ struct DGrid {
   uint32_t* slotList;
   uint32_t* nbr;       // per slot: slots of the 27 tiles around it (0 none, WSLOT_OUT outside)
   uint32_t* nbrL;      // the same rows in slotList order (row b for slotList[b])
+  uint32_t* slotPos;   // per slot in use: its place in slotList
+  uint8_t* posFluid;   // per slotList entry and half (cells below 256, the others): whether it holds fluid (divergence)
+  uint64_t* sorTileW;  // exchange words of the one-per-tile SOR: two buffers of tileCap x 512 (value low, tag high)
+  uint32_t tileCap;    // slotList entries sorTileW has room for
   uint4* tileRec;      // three per slotList entry: slot, first cell (x, y, z), slots across the faces x-, x+, y-, y+, z-, z+ (0: none)
   uint32_t* wg;        // per scan block: new and kept tiles before it
   uint32_t* part;      // per-workgroup statistics partials (vmax; fluid cells per colour)

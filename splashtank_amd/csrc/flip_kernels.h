@@ -12,11 +12,14 @@
 // resident SOR: workgroup size, tiles resident per workgroup, and the largest
 // grid its barrier serves (sorBar holds COOP_MAX_WG epochs, then the sequence
 // number of the last solve it finished, a count of barrier time-outs, the
-// barrier's release word and the path of the last solve: 0 one launch per
-// iteration, 1 resident, 2 streaming)
+// barrier's release word, the path of the last solve: 0 one launch per
+// iteration, 1 resident, 2 streaming, and the sequence number of the last solve
+// with a workgroup per tile)
 #define COOP_WG 1024
 #define COOP_TMAX 54
 #define COOP_MAX_WG 1024
+// most tiles in use of the one-per-tile solve: its exchange words are numbered in 20 bits
+#define SOR_TILES_MAX 2048u
 
 struct LaunchCtx {
   const DParams* P;
@@ -30,6 +33,8 @@ struct LaunchCtx {
   uint32_t faceGrid;  // workgroups of the cell kernels that walk tiles in use (normFaces, divergence, project)
   uint32_t pipeGrid;  // persistent SOR workgroups (about eight per CU)
   uint32_t coopGrid;  // resident-SOR workgroups (one per CU), 0 when cooperative launches are unavailable
+  uint32_t sorTiles;  // workgroups of the one-per-tile solve resident at once (0: not available)
+  uint32_t sorTag;    // tag of this solve's first exchange
   uint32_t sorSeq;    // sequence number of this pressure solve
   bool sorStream;     // the cooperative solve streams tile windows even when the tiles fit in LDS
   bool full;          // the whole substep follows the blocks stage (not a tile-only step)
@@ -91,11 +96,14 @@ size_t batch_table_words(uint32_t nt, uint32_t itersMax);
 void batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t itersMax, uint32_t sorResident, uint32_t* tab);
 // every stage of one substep for all tanks, one launch per kernel: dT and dtab
 // are the device copies of the tank records and tables, htab the host copy
-// coopGrid > 0 (and a plan buffer of 3 nt + 1 words): the SOR of every tank in
-// one cooperative launch of that many resident workgroups, else (or when the
+// coopGrid > 0 (and a plan buffer of batch_plan_words): the SOR of every tank in
+// one cooperative launch, with a workgroup per fluid tile where the device holds
+// that many (sorTiles; most: tiles the tanks can have in use, full: tiles their
+// particles would fill) or of coopGrid resident workgroups, else (or when the
 // launch is refused) one launch per iteration; returns whether it ran resident
+inline size_t batch_plan_words(uint32_t nt) { return size_t(nt) * 4u + 2u; }
 bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, const uint32_t* htab, uint32_t nt, uint32_t itersMax,
-                       uint32_t coopGrid, uint32_t* dPlan);
+                       uint32_t coopGrid, uint32_t sorTiles, uint32_t most, uint32_t full, uint32_t* dPlan);
 
 void launch_fill_u32(hipStream_t st, uint32_t* p, size_t n, uint32_t v);
 void launch_blocks(hipStream_t st, const LaunchCtx& L);
@@ -116,6 +124,8 @@ hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters);
 uint32_t sor_resident_grid(uint32_t cus);
 // workgroups of the resident SOR (one per CU when it fits there), 0 if it does not
 uint32_t sor_coop_grid(uint32_t cus);
+// workgroups of the one-per-tile SOR resident at once (at most SOR_TILES_MAX), 0 if none fits
+uint32_t sor_tiles_grid(uint32_t cus);
 // tile indices in Morton order of their (ti, tj, tk) coordinates
 void morton_tiles(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t* out);
 void launch_project(hipStream_t st, const LaunchCtx& L);

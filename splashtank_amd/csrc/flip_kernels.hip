@@ -381,7 +381,9 @@ __device__ __forceinline__ void tiles_place_body(const DParams* __restrict__ PP,
   for (uint32_t q = 0; q < 4u; q++) {
     if (!nd[q]) continue;
     if (slot[q] != ST_NONE) {
-      G.slotList[kept + min(k, nalloc)] = slot[q];
+      const uint32_t at = kept + min(k, nalloc);
+      G.slotList[at] = slot[q];
+      G.slotPos[slot[q]] = at;
       kept++;
       continue;
     }
@@ -392,6 +394,7 @@ __device__ __forceinline__ void tiles_place_body(const DParams* __restrict__ PP,
       G.tmap[t] = s;
       G.slotTile[s] = t;
       G.slotList[kept + k] = s;
+      G.slotPos[s] = kept + k;
     }
     k++;
   }
@@ -922,7 +925,7 @@ __global__ void __launch_bounds__(WG) k_classify(const DParams* __restrict__ PP,
 // the slot across that face: no tile map lookups and no divisions per cell, and a
 // cell's three faces move in one 12-byte access.  Bound by HBM and, in divergence,
 // by its twelve loads per cell; before, by the lookups.  At 256^3 (10,245 tiles, 5.2 M
-// cells): normFaces 104 -> 64 us (4.3 TB/s), divergence 77 -> 60, project 79 -> 46.
+// cells): normFaces 104 -> 65 us (4.2 TB/s), divergence 77 -> 57, project 79 -> 48.
 struct TileAt {
   uint32_t s;                       // slot
   int32_t x, y, z;                  // the tile's first cell
@@ -1011,12 +1014,15 @@ __device__ __forceinline__ float gv0R(const DGrid& G, uint32_t f) { return st_u2
 #define STEN_FLUID 0x80u
 
 // divergence (wgsl-solver.js:106-123); also records the SOR stencil of the cell,
-// which depends only on the cell types fixed by classify.
+// which depends only on the cell types fixed by classify, and whether each half
+// tile holds fluid.
 __device__ __forceinline__ void divergence_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid) {
   const DParams& P = *PP;
   FOR_TILES(G, T, l) {
     const uint32_t c = T.s * 512u + l;
     const uint32_t ct = G.ctype[c];
+    const int any = __syncthreads_or((ct & 0xffu) == 1u);
+    if (threadIdx.x == 0) G.posFluid[u_] = any ? 1u : 0u;
     if ((ct & 0xffu) != 1u) {
       G.rhs[c] = 0.0f;
       G.sten[c] = 0;
@@ -1510,7 +1516,7 @@ static_assert(kCoopLdsBytes + 256 <= 160 * 1024, "the resident solve's LDS fits 
 // The resident solve of one sim by its workgroups w = 0 .. ng-1 (the whole
 // launch for one sim, or its range of a batched launch).
 __device__ __forceinline__ void sor_resident_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t iters, uint32_t seq,
-                                                  uint32_t stream, uint32_t w, uint32_t ng) {
+                                                  uint32_t tag0, uint32_t stream, uint32_t w, uint32_t ng) {
   __shared__ __align__(16) unsigned char smem[kCoopLdsBytes];
   __shared__ uint32_t nFor;
   __shared__ float ytab[8];
@@ -1518,7 +1524,6 @@ __device__ __forceinline__ void sor_resident_body(const DParams* __restrict__ PP
   const uint32_t nact = G.ctl[4], tid = threadIdx.x;
   if (nact == 0u || ng > COOP_MAX_WG) return;
   const float omega = PP->omega;
-  const uint32_t tag0 = PP->sorTag;
   if (tid == 0u) sFail = 0u;
   if (stream || nact > ng * COOP_TMAX) {
     // Streaming mode, for more tiles than fit in LDS: four tile pipelines of 256
@@ -1724,8 +1729,328 @@ __device__ __forceinline__ void sor_resident_body(const DParams* __restrict__ PP
   }
 }
 __global__ void __launch_bounds__(COOP_WG) k_sor_resident(const DParams* __restrict__ PP, DGrid G, uint32_t iters,
-                                                          uint32_t seq, uint32_t stream) {
-  sor_resident_body(PP, G, iters, seq, stream, blockIdx.x, gridDim.x);
+                                                          uint32_t seq, uint32_t tag0, uint32_t stream) {
+  if (G.sorBar[COOP_MAX_WG + 4] == seq) return;  // k_sor_tiles did this solve
+  sor_resident_body(PP, G, iters, seq, tag0, stream, blockIdx.x, gridDim.x);
+}
+
+// Tile SOR: the whole solve in one cooperative launch with a workgroup per tile,
+// where the tiles in use that hold fluid are no more than the workgroups the device
+// holds at once (TS_WAVES per CU, 1792 on 256 CUs).  The resident solve above exchanges faces after each colour, and
+// with a few tiles per CU that exchange (about 2.4 us) is nearly all of its time.
+// Here each workgroup also relaxes the cells around its tile that its own cells
+// depend on within two iterations, so it exchanges once per two iterations: 16^3
+// window in LDS; red cells up to distance 3 (city block distance from the tile),
+// black up to 2, red up to 1, then the tile's black cells; 2372 cell updates for
+// 1024.  Every cell is relaxed from the same inputs with the same arithmetic as
+// where it belongs, so the copies agree bit for bit and the iterate is the
+// reference's.  Tiles without fluid hold zeros throughout and take no part.
+// Measured (pressure stage): 64^3 dam break, 160 fluid tiles, 40 iterations 222 -> 88
+// us; 128^3 splash, 1223 fluid tiles, 80 iterations 457 -> 338; 16^3, 4 fluid tiles, 30
+// iterations 173 -> 67.  Per exchange at 64^3 the sweeps take 1.4 us and the exchange
+// 1.6; at seven workgroups per CU the sweeps' instructions bound it.
+//
+// Exchange g (g = 0 carries the start pressure): a workgroup publishes its tile's
+// 512 values as 64-bit words (value, tag of the exchange) in buffer g & 1 and polls
+// the words it needs in its neighbours' until their tags match.  It overwrites
+// buffer g only after it has read exchange g + 1 of every neighbour it exchanges
+// with, which they publish after reading exchange g; whether two tiles exchange
+// depends on both holding fluid alone, so the waiting is mutual.
+#define TS_WAVES 7  // workgroups per CU it is built for: what fits in LDS (20.8 KB each)
+#define TS_Y 20  // row pitch: the four same-colour cells of eight rows fall on 32 different banks
+#define TS_Z 320
+#define TS_W3 (16 * TS_Z)
+#define TS_NRED 980    // red cells within distance 3: 256, 192, 240, 292 at distances 0 .. 3
+#define TS_NBLACK 688  // black cells within distance 2: 256, 192, 240
+#define TS_NPOLL 1604  // words polled per exchange: black at distances 1 .. 4, red at 2 and 3 (red at 1 is our own result)
+#define TS_NPOLL0 192  // exchange 0 also: red at distance 1
+#define TS_KPOLL ((TS_NPOLL + WG - 1) / WG)
+struct TileCells {
+  uint16_t red[TS_NRED], black[TS_NBLACK], poll[TS_NPOLL + TS_NPOLL0];  // x + 16 y + 256 z in the window
+};
+constexpr int ts_out(int w) { return w < 4 ? 4 - w : (w > 11 ? w - 11 : 0); }
+constexpr TileCells tile_cells() {
+  TileCells t{};
+  int nr = 0, nb = 0;
+  for (int d = 0; d < 4; d++)
+    for (int z = 0; z < 16; z++)
+      for (int y = 0; y < 16; y++) {
+        const int dyz = ts_out(y) + ts_out(z);
+        if (dyz > d) continue;
+        for (int x = 0; x < 16; x++) {
+          if (ts_out(x) + dyz != d) continue;
+          const uint16_t i = uint16_t(x + 16 * (y + 16 * z));
+          if (((x + y + z) & 1) == 0) t.red[nr++] = i;
+          else if (d < 3) t.black[nb++] = i;
+        }
+      }
+  // by the tile they lie in, then in its order, so that neighbouring lanes poll neighbouring words
+  int np = 0, n0 = TS_NPOLL;
+  for (int q = 0; q < 27; q++) {
+    const int x0 = q % 3 == 0 ? 0 : (q % 3 == 1 ? 4 : 12), x1 = q % 3 == 0 ? 4 : (q % 3 == 1 ? 12 : 16);
+    const int y0 = q / 3 % 3 == 0 ? 0 : (q / 3 % 3 == 1 ? 4 : 12), y1 = q / 3 % 3 == 0 ? 4 : (q / 3 % 3 == 1 ? 12 : 16);
+    const int z0 = q / 9 == 0 ? 0 : (q / 9 == 1 ? 4 : 12), z1 = q / 9 == 0 ? 4 : (q / 9 == 1 ? 12 : 16);
+    for (int z = z0; z < z1; z++)
+      for (int y = y0; y < y1; y++)
+        for (int x = x0; x < x1; x++) {
+          const int d = ts_out(x) + ts_out(y) + ts_out(z);
+          const bool black = ((x + y + z) & 1) != 0;
+          const uint16_t i = uint16_t(x + 16 * (y + 16 * z));
+          if (d >= 1 && d <= (black ? 4 : 3)) {
+            if (!black && d == 1) t.poll[n0++] = i;
+            else t.poll[np++] = i;
+          }
+        }
+  }
+  return t;
+}
+constexpr TileCells kTileCellsHost = tile_cells();
+static_assert(kTileCellsHost.red[TS_NRED - 1] != 0 && kTileCellsHost.black[TS_NBLACK - 1] != 0 && kTileCellsHost.poll[TS_NPOLL - 1] != 0 &&
+                  kTileCellsHost.poll[TS_NPOLL + TS_NPOLL0 - 1] != 0,
+              "the lists are full");
+__constant__ TileCells kTileCells = kTileCellsHost;
+
+// window index -> which of the 27 tiles (nbr order) and the local cell in it
+__device__ __forceinline__ uint32_t ts_tile(uint32_t i) {
+  const uint32_t x = i & 15u, y = (i >> 4) & 15u, z = i >> 8;
+  return ((x + 4u) >> 3) + 3u * ((y + 4u) >> 3) + 9u * ((z + 4u) >> 3);
+}
+__device__ __forceinline__ uint32_t ts_local(uint32_t i) {
+  const uint32_t x = i & 15u, y = (i >> 4) & 15u, z = i >> 8;
+  return ((x + 4u) & 7u) + 8u * (((y + 4u) & 7u) + 8u * ((z + 4u) & 7u));
+}
+__device__ __forceinline__ uint32_t ts_window(uint32_t i) { return (i & 15u) + TS_Y * ((i >> 4) & 15u) + TS_Z * (i >> 8); }
+// N cells of one colour: a = byte offset in the window | stencil byte << 16 (0: not
+// fluid, kept; its offset is any inner cell's).  coop_cell's arithmetic, all N
+// cells' loads and steps side by side: a thread's chain of one cell after another
+// was most of a sweep's time (2.5 us for the four sweeps of an exchange).
+template <uint32_t N>
+__device__ __forceinline__ void ts_relax(float* sp, const uint32_t* a, const float* rhs, float omega, const float* ytab) {
+  float pc[N], sum[N], out[N];
+  float* p[N];
+  uint32_t st[N];
+  bool slow = false;
+#pragma unroll
+  for (uint32_t j = 0; j < N; j++) {
+    p[j] = reinterpret_cast<float*>(reinterpret_cast<char*>(sp) + (a[j] & 0xffffu));
+    st[j] = a[j] >> 16;
+    const float n0 = p[j][-1], n1 = p[j][1], n2 = p[j][-TS_Y], n3 = p[j][TS_Y], n4 = p[j][-TS_Z], n5 = p[j][TS_Z];
+    pc[j] = p[j][0];
+    float t = 0.0f;
+    t = t + n0;
+    t = t + n1;
+    t = t + n2;
+    t = t + n3;
+    t = t + n4;
+    t = t + n5;
+    sum[j] = t;
+  }
+#pragma unroll
+  for (uint32_t j = 0; j < N; j++) {
+    const uint32_t nns = st[j] & 7u;
+    const float v = rhs[j] + sum[j], n = float(nns), y = ytab[nns];
+    const float q = v * y;
+    const float r = fmaf(-q, n, v);
+    const float pg = fmaf(r, y, q);
+    const uint32_t ua = st_f2u(v) & 0x7fffffffu;
+    slow = slow || (nns != 0u && !(ua - 0x01800000u < 0x7e000000u));
+    out[j] = pc[j] + omega * (pg - pc[j]);
+    if (nns == 0u) out[j] = 0.0f;
+  }
+  if (slow) {  // a quotient outside st_div_small's range: the division
+#pragma unroll
+    for (uint32_t j = 0; j < N; j++) {
+      const uint32_t nns = st[j] & 7u;
+      const float v = rhs[j] + sum[j];
+      const uint32_t ua = st_f2u(v) & 0x7fffffffu;
+      if (nns != 0u && !(ua - 0x01800000u < 0x7e000000u)) {
+        const float pg = v / float(nns);
+        out[j] = pc[j] + omega * (pg - pc[j]);
+      }
+    }
+  }
+#pragma unroll
+  for (uint32_t j = 0; j < N; j++)
+    if (st[j]) p[j][0] = out[j];
+}
+
+// Which of the eight tiles in use from 8 threadIdx.x (places in slotList, at most
+// SOR_TILES_MAX) hold fluid: two flag bytes each.
+__device__ __forceinline__ uint32_t ts_fluid8(const DGrid& G, uint32_t nact) {
+  static_assert(SOR_TILES_MAX == 8u * WG, "eight tiles per thread");
+  const uint32_t b0 = threadIdx.x * 8u;
+  uint4 f = make_uint4(0u, 0u, 0u, 0u);
+  if (b0 < nact) f = *reinterpret_cast<const uint4*>(G.posFluid + 2u * b0);
+  const uint32_t h[4] = {f.x, f.y, f.z, f.w};
+  uint32_t m = 0;
+  for (uint32_t k = 0; k < 8u; k++)
+    if (b0 + k < nact && ((h[k >> 1] >> (16u * (k & 1u))) & 0xffffu)) m |= 1u << k;
+  return m;
+}
+// The w-th tile in use that holds fluid (its place in slotList), or ST_NONE when
+// there are no more; *total = how many there are.
+__device__ __forceinline__ uint32_t ts_find(const DGrid& G, uint32_t nact, uint32_t w, uint32_t* total) {
+  __shared__ uint32_t sB;
+  const uint32_t b0 = threadIdx.x * 8u;
+  uint32_t m = ts_fluid8(G, nact);
+  if (threadIdx.x == 0) sB = ST_NONE;
+  uint64_t tot;
+  const uint64_t before = wg_scan_u64(uint64_t(__popc(m)), &tot);
+  const uint32_t at = w - uint32_t(before);
+  if (w >= uint32_t(before) && at < uint32_t(__popc(m))) {
+    for (uint32_t k = 0; k < at; k++) m &= m - 1u;
+    sB = b0 + uint32_t(__ffs((int)m)) - 1u;
+  }
+  __syncthreads();
+  *total = uint32_t(tot);
+  return sB;
+}
+
+// The solve of one tile: b its place in slotList (ts_find).
+__device__ __forceinline__ void sor_tile_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t iters, uint32_t tag0, uint32_t b) {
+  __shared__ float sp[TS_W3];
+  __shared__ uint32_t sSlot[27], sPos[27];
+  __shared__ float ytab[8];
+  __shared__ uint32_t sFail;
+  const uint32_t tid = threadIdx.x;
+  const float omega = PP->omega;
+  // this thread's cells (position tid + 256 j of each list) and polled words
+  uint32_t ra[4], ba[3], pa[TS_KPOLL];
+  float rr[4], br[3];
+#pragma unroll
+  for (uint32_t j = 0; j < 4u; j++) ra[j] = tid + j * WG < TS_NRED ? kTileCells.red[tid + j * WG] : ST_NONE;
+#pragma unroll
+  for (uint32_t j = 0; j < 3u; j++) ba[j] = tid + j * WG < TS_NBLACK ? kTileCells.black[tid + j * WG] : ST_NONE;
+#pragma unroll
+  for (uint32_t j = 0; j < TS_KPOLL; j++) pa[j] = tid + j * WG < TS_NPOLL ? kTileCells.poll[tid + j * WG] : ST_NONE;
+  uint32_t p0 = tid < TS_NPOLL0 ? kTileCells.poll[TS_NPOLL + tid] : ST_NONE;
+  if (tid < 27u) {
+    const uint32_t ns = G.nbrL[b * 27u + tid];
+    uint32_t pos = ST_NONE;
+    if (!sor_missing(ns)) {
+      pos = G.slotPos[ns];
+      if (*reinterpret_cast<const uint16_t*>(G.posFluid + 2u * pos) == 0u) pos = ST_NONE;
+    }
+    sSlot[tid] = ns;
+    sPos[tid] = pos;
+  }
+  if (tid < 8u) ytab[tid] = (tid >= 1u && tid <= 6u) ? 1.0f / float(tid) : 0.0f;
+  if (tid == 0u) sFail = 0u;
+  for (uint32_t q = tid; q < TS_W3; q += WG) sp[q] = 0.0f;
+  __syncthreads();
+  const uint32_t x = (tid & 7u) + 4u, y = ((tid >> 3) & 7u) + 4u, z = (tid >> 6) + 4u, own = x + TS_Y * y + TS_Z * z;
+  constexpr uint32_t half = 4u * TS_Z;  // cells tid and tid + 256 of the tile
+  float* pres = G.pres + size_t(sSlot[13]) * 512u;
+  sp[own] = pres[tid];
+  sp[own + half] = pres[tid + 256u];
+  // rhs and stencil of the cells, in registers for the whole solve
+  auto item = [&](uint32_t& a, float& rhs) {
+    const uint32_t i = a, q = i == ST_NONE ? 13u : ts_tile(i);
+    const bool in = i != ST_NONE && sPos[q] != ST_NONE;
+    const uint32_t c = (in ? sSlot[q] : sSlot[13]) * 512u + (in ? ts_local(i) : 0u), st = G.sten[c];
+    rhs = G.rhs[c];
+    a = in && (st & STEN_FLUID) ? ts_window(i) * 4u | (st << 16) : own * 4u;
+  };
+#pragma unroll
+  for (uint32_t j = 0; j < 4u; j++) item(ra[j], rr[j]);
+#pragma unroll
+  for (uint32_t j = 0; j < 3u; j++) item(ba[j], br[j]);
+  // a polled word: its place in the buffer (20 bits) | its cell in the window << 20
+  auto pollAt = [&](uint32_t i) {
+    const uint32_t p = i == ST_NONE ? ST_NONE : sPos[ts_tile(i)];
+    return p == ST_NONE ? ST_NONE : (p * 512u + ts_local(i)) | (i << 20);
+  };
+#pragma unroll
+  for (uint32_t j = 0; j < TS_KPOLL; j++) pa[j] = pollAt(pa[j]);
+  p0 = pollAt(p0);
+  __syncthreads();
+  const size_t bufN = size_t(G.tileCap) * 512u;
+  auto publish = [&](uint32_t g) {
+    uint64_t* buf = G.sorTileW + (g & 1u) * bufN + b * 512u;
+    const uint64_t t = uint64_t(tag0 + g) << 32;
+    __hip_atomic_store(&buf[tid], t | __float_as_uint(sp[own]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&buf[tid + 256u], t | __float_as_uint(sp[own + half]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  auto poll = [&](uint32_t g, auto n, const uint32_t* at) {
+    constexpr uint32_t K = decltype(n)::value;
+    const uint64_t* buf = G.sorTileW + (g & 1u) * bufN;
+    const uint32_t tag = tag0 + g;
+    uint64_t v[K];
+#pragma unroll
+    for (uint32_t j = 0; j < K; j++)
+      v[j] = at[j] == ST_NONE ? uint64_t(tag) << 32
+                              : __hip_atomic_load(&buf[at[j] & 0xfffffu], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (uint32_t spins = 0;; spins++) {
+      bool ready = true;
+#pragma unroll
+      for (uint32_t j = 0; j < K; j++) ready = ready && uint32_t(v[j] >> 32) == tag;
+      if (ready) break;
+      if (spins >= COOP_SPIN_LIMIT) {
+        sFail = 1u;
+        break;
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < K; j++)
+        if (uint32_t(v[j] >> 32) != tag) v[j] = __hip_atomic_load(&buf[at[j] & 0xfffffu], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < K; j++)
+      if (at[j] != ST_NONE) sp[ts_window(at[j] >> 20)] = __uint_as_float(uint32_t(v[j]));
+  };
+  publish(0u);
+  poll(0u, std::integral_constant<uint32_t, 1>{}, &p0);
+  poll(0u, std::integral_constant<uint32_t, TS_KPOLL>{}, pa);
+  __syncthreads();
+  for (uint32_t it = 0, g = 0;;) {
+    if (sFail) {  // a neighbour's words never came: give up the solve (counted)
+      if (tid == 0u) atomicAdd(&G.sorBar[COOP_MAX_WG + 1], 1u);
+      return;
+    }
+    // what derives from the items and polled words (addresses, divisors) is worked
+    // out again each time rather than held in registers for the whole solve
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; j++) asm volatile("" : "+v"(ra[j]));
+#pragma unroll
+    for (uint32_t j = 0; j < 3u; j++) asm volatile("" : "+v"(ba[j]));
+    const uint32_t n = min(2u, iters - it);
+    if (n == 2u) {
+      ts_relax<4>(sp, ra, rr, omega, ytab);
+      __syncthreads();
+      ts_relax<3>(sp, ba, br, omega, ytab);
+      __syncthreads();
+    }
+    if (tid < 192u) ts_relax<2>(sp, ra, rr, omega, ytab);  // red within distance 1: the first 448
+    else ts_relax<1>(sp, ra, rr, omega, ytab);
+    __syncthreads();
+    ts_relax<1>(sp, ba, br, omega, ytab);  // the tile's black cells
+    __syncthreads();
+    it += n;
+    if (it >= iters) break;
+    g++;
+    publish(g);
+    // a word takes about a microsecond to reach memory: a poll sent at once comes back
+    // without it and the next costs another round trip (exchange 2.1 -> 1.6 us at 160
+    // fluid tiles, 3.4 -> 2.8 at 480)
+    __builtin_amdgcn_s_sleep(20);
+    poll(g, std::integral_constant<uint32_t, TS_KPOLL>{}, pa);
+    __syncthreads();
+  }
+  pres[tid] = sp[own];
+  pres[tid + 256u] = sp[own + half];
+}
+// seq: marks the solve as done (the resident launch that follows where the tiles in
+// use may exceed the workgroups then has nothing to do)
+__global__ void __launch_bounds__(WG, TS_WAVES) k_sor_tiles(const DParams* __restrict__ PP, DGrid G, uint32_t iters, uint32_t tag0, uint32_t seq) {
+  const uint32_t nact = G.ctl[4], w = blockIdx.x;
+  if (nact > G.tileCap) return;
+  uint32_t total;
+  const uint32_t b = ts_find(G, nact, w, &total);
+  if (total > gridDim.x) return;
+  if (w == 0u && threadIdx.x == 0u) {
+    G.sorBar[COOP_MAX_WG + 4] = seq;
+    G.sorBar[COOP_MAX_WG + 3] = 1u;
+  }
+  if (b != ST_NONE) sor_tile_body(PP, G, iters, tag0, b);
 }
 
 // after an odd number of iterations the result sits in the partner buffer
@@ -2685,15 +3010,67 @@ __global__ void kb_copy_tiles(BATCH_ARGS) { BATCH_TANK; copy_tiles_body(T.G, T.G
 // not empty), kb_sor_plan (one thread) assigns the workgroups; tiles_finish has
 // listed its slots in Morton order and cleared its barrier words.
 
+// Batched tile SOR: plan words after the phases' count, 3 nt + 1: whether the
+// launch below did the solves, 3 nt + 2 + t: fluid tiles of tank t (ST_NONE: too
+// many tiles in use to look).
+__global__ void __launch_bounds__(WG) kb_sor_counts(const BTank* __restrict__ TT, const uint32_t* __restrict__ act, uint32_t nt,
+                                                    uint32_t* __restrict__ plan) {
+  const uint32_t t = blockIdx.x;
+  const DGrid G = TT[t].G;
+  const uint32_t nact = act[t + 1] != act[t] ? G.ctl[4] : 0u;
+  uint64_t tot = ST_NONE;
+  if (nact <= G.tileCap) (void)wg_scan_u64(uint64_t(__popc(ts_fluid8(G, nact))), &tot);
+  if (threadIdx.x == 0) {
+    plan[3u * nt + 2u + t] = uint32_t(tot);
+    if (t == 0u) plan[3u * nt + 1u] = 0u;
+  }
+}
+// every tank's solve with a workgroup per fluid tile, where they all fit at once
+__global__ void __launch_bounds__(WG, TS_WAVES) kb_sor_tiles(const BTank* __restrict__ TT, const uint32_t* __restrict__ act, uint32_t nt,
+                                                             uint32_t* __restrict__ plan) {
+  static_assert(ST_BATCH_MAX <= WG, "a thread per tank");
+  __shared__ uint32_t sT, sW;
+  const uint32_t tid = threadIdx.x, w = blockIdx.x;
+  const uint32_t cnt = tid < nt ? plan[3u * nt + 2u + tid] : 0u;
+  if (tid == 0u) sT = ST_NONE;
+  uint64_t tot;
+  const uint64_t before = wg_scan_u64(cnt, &tot);
+  if (tot > gridDim.x) return;
+  if (w == 0u) {
+    if (tid == 0u) plan[3u * nt + 1u] = 1u;
+    if (tid < nt && act[tid + 1u] != act[tid]) TT[tid].G.sorBar[COOP_MAX_WG + 3] = 1u;
+  }
+  if (w >= uint32_t(before) && w < uint32_t(before) + cnt) {
+    sT = tid;
+    sW = w - uint32_t(before);
+  }
+  __syncthreads();
+  const uint32_t t = sT;
+  if (t == ST_NONE) return;
+  const DGrid G = TT[t].G;
+  const DParams* P = TT[t].P;
+  uint32_t total;
+  const uint32_t b = ts_find(G, G.ctl[4], sW, &total);
+  if (b != ST_NONE) sor_tile_body(P, G, P->iters, P->sorTag, b);
+}
+
 // plan[3 t .. 3 t + 2] = (phase, first workgroup, workgroups) of tank t (phase
 // ST_NONE: no solve), plan[3 nt] = phases.  First fit in tank order, each tank
 // at least the workgroups its tiles need in LDS (all `grid` when even those
 // are too few: it then streams); a phase's spare workgroups go to its tanks in
 // proportion to their tiles.  A tank that streams is alone in its phase with
 // all `grid` workgroups (at least 2, which its tile pipelines need).
-__global__ void kb_sor_plan(const BTank* __restrict__ TT, const uint32_t* __restrict__ act, uint32_t nt, uint32_t grid,
-                            uint32_t* __restrict__ plan) {
+__global__ void __launch_bounds__(WG) kb_sor_plan(const BTank* __restrict__ TT, const uint32_t* __restrict__ act, uint32_t nt, uint32_t grid,
+                                                  uint32_t tiled, uint32_t* __restrict__ plan) {
+  // the tanks' tile counts, loaded side by side (one thread after the other took 17 us for 16 tanks)
+  __shared__ uint32_t sAct[WG];
+  if (threadIdx.x < nt) sAct[threadIdx.x] = act[threadIdx.x + 1u] != act[threadIdx.x] ? TT[threadIdx.x].G.ctl[4] : 0u;
+  __syncthreads();
   if (threadIdx.x != 0u || blockIdx.x != 0u) return;
+  if (tiled && plan[3 * nt + 1]) {  // kb_sor_tiles did the solves
+    plan[3 * nt] = 0u;
+    return;
+  }
   uint32_t phase = 0, used = 0, first = 0;
   uint64_t tiles = 0;
   auto close = [&](uint32_t endT) {  // spread the spare workgroups of the phase over tanks [first, endT)
@@ -2701,7 +3078,7 @@ __global__ void kb_sor_plan(const BTank* __restrict__ TT, const uint32_t* __rest
     uint32_t at = 0;
     for (uint32_t q = first; q < endT; q++) {
       if (plan[3 * q] != phase) continue;
-      const uint32_t nact = TT[q].G.ctl[4];
+      const uint32_t nact = sAct[q];
       const uint32_t extra = tiles ? uint32_t(uint64_t(spare) * nact / tiles) : 0u;
       plan[3 * q + 1] = at;
       plan[3 * q + 2] += extra;
@@ -2712,7 +3089,7 @@ __global__ void kb_sor_plan(const BTank* __restrict__ TT, const uint32_t* __rest
     plan[3 * t] = ST_NONE;
     plan[3 * t + 1] = 0u;
     plan[3 * t + 2] = 0u;
-    const uint32_t nact = act[t + 1] != act[t] ? TT[t].G.ctl[4] : 0u;
+    const uint32_t nact = sAct[t];
     if (nact == 0u) continue;
     const uint32_t need = min(grid, (nact + COOP_TMAX - 1u) / COOP_TMAX);
     if (used + need > grid) {
@@ -2742,7 +3119,7 @@ __global__ void __launch_bounds__(COOP_WG) kb_sor_resident(const BTank* __restri
       if (plan[3 * q] == p && w >= plan[3 * q + 1] && w < plan[3 * q + 1] + plan[3 * q + 2]) t = q;
     if (t == ST_NONE) continue;
     const BTank& B = TT[t];
-    sor_resident_body(B.P, B.G, B.P->iters, 0u, 0u, w - plan[3 * t + 1], plan[3 * t + 2]);
+    sor_resident_body(B.P, B.G, B.P->iters, 0u, B.P->sorTag, 0u, w - plan[3 * t + 1], plan[3 * t + 2]);
     __syncthreads();  // the LDS of this phase's tank is free again
   }
 }
@@ -2861,6 +3238,15 @@ uint32_t sor_coop_grid(uint32_t cus) {
   return std::min<uint32_t>(cus, COOP_MAX_WG);
 }
 
+uint32_t sor_tiles_grid(uint32_t cus) {
+  int nb = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sor_tiles, WG, 0) != hipSuccess || nb < 1) return 0u;
+  return std::min<uint32_t>(cus * uint32_t(nb), SOR_TILES_MAX);
+}
+// Whether the fluid tiles probably fit: about a fifth more than the particles would
+// fill (1223 for 1050 at the 128^3 splash).  A miss costs an idle launch (5 us).
+static bool sor_tiles_likely(uint32_t fullTiles, uint32_t grid) { return fullTiles + fullTiles / 5u <= grid; }
+
 void morton_tiles(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t* out) {
   auto spread = [](uint64_t v) {  // bit i of v to bit 3i
     uint64_t r = 0;
@@ -2889,8 +3275,17 @@ hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters) {
     }
     const DParams* P = L.P;
     DGrid G = L.G;
-    uint32_t it = uint32_t(iters), seq = L.sorSeq, stream = L.sorStream ? 1u : 0u;
-    void* args[] = {(void*)&P, (void*)&G, (void*)&it, (void*)&seq, (void*)&stream};
+    uint32_t it = uint32_t(iters), seq = L.sorSeq, tag = L.sorTag, stream = L.sorStream ? 1u : 0u;
+    // a workgroup per tile where every tile in use has one: at most `most` tiles are
+    // in use, and about as many as the particles would fill, and their neighbours
+    const uint32_t most = std::min<uint32_t>(L.ntiles, L.scap - 1u);
+    if (!stream && L.sorTiles && (most <= L.sorTiles || sor_tiles_likely(L.fullTiles, L.sorTiles))) {
+      void* args[] = {(void*)&P, (void*)&G, (void*)&it, (void*)&tag, (void*)&seq};
+      coopErr = hipLaunchCooperativeKernel((const void*)k_sor_tiles, dim3(std::min(most, L.sorTiles)), dim3(WG), args, 0, st);
+      if (coopErr == hipSuccess && most <= L.sorTiles) return hipSuccess;
+      if (coopErr != hipSuccess) (void)hipGetLastError();  // the launch below does the solve
+    }
+    void* args[] = {(void*)&P, (void*)&G, (void*)&it, (void*)&seq, (void*)&tag, (void*)&stream};
     coopErr = hipLaunchCooperativeKernel((const void*)k_sor_resident, dim3(L.coopGrid), dim3(COOP_WG), args, 0, st);
     if (coopErr == hipSuccess) return hipSuccess;
     (void)hipGetLastError();  // the per-iteration launches below do the solve
@@ -3008,7 +3403,7 @@ void batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t itersMax, uint32_
 }
 
 bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, const uint32_t* htab, uint32_t nt, uint32_t itersMax,
-                       uint32_t coopGrid, uint32_t* dPlan) {
+                       uint32_t coopGrid, uint32_t sorTiles, uint32_t most, uint32_t full, uint32_t* dPlan) {
   const size_t w = size_t(nt) + 1u;
   auto tab = [&](uint32_t k) { return dtab + k * w; };
   auto tot = [&](uint32_t k) { return htab[k * w + nt]; };
@@ -3033,12 +3428,23 @@ bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, co
   // one launch per iteration (ping-pong between pres and pres2)
   bool resident = false;
   if (coopGrid && dPlan && itersMax) {
-    hipLaunchKernelGGL(kb_sor_plan, dim3(1), dim3(64), 0, st, dT, tab(BT_PIPE0), nt, coopGrid, dPlan);
     const BTank* a0 = dT;
+    const uint32_t* actTab = tab(BT_PIPE0);
+    const bool tiles = sorTiles && (most <= sorTiles || sor_tiles_likely(full, sorTiles));
+    bool done = false;
+    if (tiles) {
+      hipLaunchKernelGGL(kb_sor_counts, dim3(nt), dim3(WG), 0, st, dT, actTab, nt, dPlan);
+      uint32_t* plan = dPlan;
+      void* args[] = {(void*)&a0, (void*)&actTab, (void*)&nt, (void*)&plan};
+      done = hipLaunchCooperativeKernel((const void*)kb_sor_tiles, dim3(std::max(1u, std::min(most, sorTiles))), dim3(WG), args, 0, st) == hipSuccess;
+      if (!done) (void)hipGetLastError();
+      done = done && most <= sorTiles;  // else the launches below do the solve where it did not fit
+    }
+    if (!done) hipLaunchKernelGGL(kb_sor_plan, dim3(1), dim3(WG), 0, st, dT, actTab, nt, coopGrid, tiles ? 1u : 0u, dPlan);
     const uint32_t* a1 = dPlan;
     uint32_t a2 = nt;
     void* args[] = {(void*)&a0, (void*)&a1, (void*)&a2};
-    resident = hipLaunchCooperativeKernel((const void*)kb_sor_resident, dim3(coopGrid), dim3(COOP_WG), args, 0, st) == hipSuccess;
+    resident = done || hipLaunchCooperativeKernel((const void*)kb_sor_resident, dim3(coopGrid), dim3(COOP_WG), args, 0, st) == hipSuccess;
     if (!resident) (void)hipGetLastError();  // the launches per iteration below do the solve
   }
   if (!resident) {
