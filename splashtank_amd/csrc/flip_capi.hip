@@ -864,7 +864,7 @@ int allocTape(Sim* s, AdjTape& T) {
   return ST_OK;
 }
 
-#define D2D(dst, src, n) HIPCHK(hipMemcpyAsync((dst), (src), (n) * sizeof(*(src)), hipMemcpyDeviceToDevice, s->st))
+#define D2D(list, dst, src, n) (list).add((dst), (src), (n) * sizeof(*(src)))
 
 }  // namespace
 
@@ -1953,9 +1953,12 @@ int st_snapshot_create(void* p, void** out) {
     freeSnap(q);
     return rc;
   }
-  D2D(q->pos, s->G.pos, M); D2D(q->vel, s->G.vel, M); D2D(q->pid, s->G.pid, M); D2D(q->tmap, s->G.tmap, s->ntiles);
-  D2D(q->slotTile, s->G.slotTile, s->scap); D2D(q->fstack, s->G.fstack, s->scap); D2D(q->slotList, s->G.slotList, s->scap);
-  D2D(q->ctl, s->G.ctl, 16); D2D(q->ctype, s->G.ctype, C); D2D(q->pres, s->G.pres, C);
+  CopyList L;
+  D2D(L, q->pos, s->G.pos, M); D2D(L, q->vel, s->G.vel, M); D2D(L, q->pid, s->G.pid, M); D2D(L, q->tmap, s->G.tmap, s->ntiles);
+  D2D(L, q->slotTile, s->G.slotTile, s->scap); D2D(L, q->fstack, s->G.fstack, s->scap); D2D(L, q->slotList, s->G.slotList, s->scap);
+  D2D(L, q->ctl, s->G.ctl, 16); D2D(L, q->ctype, s->G.ctype, C); D2D(L, q->pres, s->G.pres, C);
+  launch_copies(s->st, L);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s->st));
   q->N = s->N; q->scap = s->scap; q->seed = s->seed; q->tm = s->tm;
   *out = q;
@@ -1969,9 +1972,12 @@ int st_snapshot_restore(void* p, void* snap) {
   if (q->scap != s->scap) return fail(ST_ERR_STATE, "st_snapshot_restore: the pool has grown since the snapshot");
   HIPCHK(hipSetDevice(s->dev));
   size_t M = s->maxn, C = size_t(s->scap) * 512u;
-  D2D(s->G.pos, q->pos, M); D2D(s->G.vel, q->vel, M); D2D(s->G.pid, q->pid, M); D2D(s->G.tmap, q->tmap, s->ntiles);
-  D2D(s->G.slotTile, q->slotTile, s->scap); D2D(s->G.fstack, q->fstack, s->scap); D2D(s->G.slotList, q->slotList, s->scap);
-  D2D(s->G.ctl, q->ctl, 16); D2D(s->G.ctype, q->ctype, C); D2D(s->G.pres, q->pres, C);
+  CopyList L;
+  D2D(L, s->G.pos, q->pos, M); D2D(L, s->G.vel, q->vel, M); D2D(L, s->G.pid, q->pid, M); D2D(L, s->G.tmap, q->tmap, s->ntiles);
+  D2D(L, s->G.slotTile, q->slotTile, s->scap); D2D(L, s->G.fstack, q->fstack, s->scap); D2D(L, s->G.slotList, q->slotList, s->scap);
+  D2D(L, s->G.ctl, q->ctl, 16); D2D(L, s->G.ctype, q->ctype, C); D2D(L, s->G.pres, q->pres, C);
+  launch_copies(s->st, L);
+  HIPCHK(hipGetLastError());
   s->N = q->N; s->seed = q->seed; s->tm = q->tm;
   s->solidDirty = true;  // the restored cell types hold the collider bits of the records then
   s->binned = false;  // marks and bins are rebuilt from the restored positions
@@ -2203,27 +2209,31 @@ int st_adj_record(void* adj, const st_params* prm) {
   }
   AdjTape& T = a->tapes[a->depth];
   size_t M = s->maxn, C = size_t(s->scap) * 512u;
-  D2D(T.pos, s->G.pos, M); D2D(T.vel, s->G.vel, M); D2D(T.pid, s->G.pid, M); D2D(T.tmap0, s->G.tmap, s->ntiles);
+  CopyList before;
+  D2D(before, T.pos, s->G.pos, M); D2D(before, T.vel, s->G.vel, M); D2D(before, T.pid, s->G.pid, M); D2D(before, T.tmap0, s->G.tmap, s->ntiles);
+  launch_copies(s->st, before);
   int rc = st_begin_step(s, prm);
   if (rc) return rc;
   T.n = s->N;
   T.iters = uint32_t(s->iters);
-  D2D(T.P, &s->cur->P, 1);
-  D2D(T.C, &s->cur->C, 1);
   T.sdf = s->G.sdf;
   a->sdfSig[a->depth] = s->sdfSig;
   a->sdfAt[a->depth] = s->G.sdf;
   a->ncols[a->depth] = ncol;
   for (int k = 0; k < ST_STAGE_COUNT; k++) {
     if ((rc = runStage(s, k))) return rc;
+    CopyList L;
     if (k == ST_STAGE_BLOCKS) {
-      D2D(T.tmap, s->G.tmap, s->ntiles); D2D(T.slotTile, s->G.slotTile, s->scap); D2D(T.slotList, s->G.slotList, s->scap);
-      D2D(T.binStart, s->G.binStart, size_t(s->ntiles) + 2); D2D(T.binIdx, s->G.binIdx, M);
+      D2D(L, T.P, &s->cur->P, 1); D2D(L, T.C, &s->cur->C, 1);
+      D2D(L, T.tmap, s->G.tmap, s->ntiles); D2D(L, T.slotTile, s->G.slotTile, s->scap); D2D(L, T.slotList, s->G.slotList, s->scap);
+      D2D(L, T.binStart, s->G.binStart, size_t(s->ntiles) + 2); D2D(L, T.binIdx, s->G.binIdx, M);
     }
-    if (k == ST_STAGE_P2G) D2D(T.accWraw, s->G.accW, C * 3);
-    if (k == ST_STAGE_CLASSIFY) D2D(T.ctype, s->G.ctype, C);
-    if (k == ST_STAGE_DIVERGENCE) D2D(T.sten, s->G.sten, C);
-    if (k == ST_STAGE_PROJECT) { D2D(T.accVfin, s->G.accV, C * 3); D2D(T.accWfin, s->G.accW, C * 3); D2D(T.ctl, s->G.ctl, 16); }
+    if (k == ST_STAGE_P2G) D2D(L, T.accWraw, s->G.accW, C * 3);
+    if (k == ST_STAGE_PROJECT) {  // the cell types and stencils are classify's and divergence's still
+      D2D(L, T.accVfin, s->G.accV, C * 3); D2D(L, T.accWfin, s->G.accW, C * 3); D2D(L, T.ctl, s->G.ctl, 16);
+      D2D(L, T.ctype, s->G.ctype, C); D2D(L, T.sten, s->G.sten, C);
+    }
+    launch_copies(s->st, L);
   }
   a->depth++;
   return ST_OK;

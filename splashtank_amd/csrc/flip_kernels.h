@@ -105,6 +105,18 @@ inline size_t batch_plan_words(uint32_t nt) { return size_t(nt) * 4u + 2u; }
 bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, const uint32_t* htab, uint32_t nt, uint32_t itersMax,
                        uint32_t coopGrid, uint32_t sorTiles, uint32_t most, uint32_t full, uint32_t* dPlan);
 
+// device-to-device copies made by one launch: whole words, starts aligned to 16
+// bytes (allocations are), at most COPY_LIST_MAX
+#define COPY_LIST_MAX 12
+struct CopyList {
+  void* dst[COPY_LIST_MAX];
+  const void* src[COPY_LIST_MAX];
+  size_t bytes[COPY_LIST_MAX];
+  uint32_t first[COPY_LIST_MAX + 1] = {0};  // first workgroup of each copy
+  uint32_t n = 0;
+  void add(void* d, const void* s, size_t nbytes);
+};
+void launch_copies(hipStream_t st, const CopyList& L);
 void launch_fill_u32(hipStream_t st, uint32_t* p, size_t n, uint32_t v);
 void launch_blocks(hipStream_t st, const LaunchCtx& L);
 void launch_p2g(hipStream_t st, const LaunchCtx& L);
