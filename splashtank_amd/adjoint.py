@@ -22,11 +22,24 @@ import torch
 from . import capi, scenes
 
 
-def _f4(a: torch.Tensor) -> np.ndarray:
-    x = a.detach().to("cpu", torch.float32).numpy()
-    out = np.zeros((x.shape[0], 4), np.float32)
-    out[:, :3] = x[:, :3]
-    return out
+def _put(dst: torch.Tensor, a: torch.Tensor):
+    """The first three columns of `a` into the (n, 4) host rows `dst`, 0 in the
+    fourth; a device tensor is padded there and crosses in one copy."""
+    a = a.detach()
+    if a.is_cuda:
+        t = torch.zeros(dst.shape, dtype=torch.float32, device=a.device)
+        t[:, :3] = a[:, :3]
+        dst.copy_(t)
+    else:
+        dst[:, :3] = a[:, :3]
+        dst[:, 3] = 0.0
+
+
+def _take(src: torch.Tensor, device, dtype) -> torch.Tensor:
+    """A new (n, 3) tensor of the host rows `src`."""
+    if torch.device(device).type == "cuda":
+        return src.to(device)[:, :3].to(dtype).contiguous()
+    return src[:, :3].to(dtype, copy=True).contiguous().to(device)
 
 
 def pose_weights(times, t: float, smooth: bool = True) -> np.ndarray:
@@ -104,6 +117,11 @@ class Rollout:
         self.cols = list(cols)
         self.t0 = float(t0)
         self.keys = [None] * len(self.cols)
+        # kept for the rollout's life: two (n, 4) pinned host buffers that states and
+        # gradients cross through, and the adjoint context with its tapes
+        self._rows = None
+        self._adj = None
+        self._adj_slots = 0
         self._sdf = np.concatenate([c.data for c in self.cols]) if self.cols else np.zeros(0, np.float32)
 
     def __call__(self, pos0: torch.Tensor, vel0: torch.Tensor, *keys: torch.Tensor):
@@ -130,33 +148,53 @@ class Rollout:
         self.sim.set_colliders(np.concatenate(recs), self._sdf, 1)
         return ws
 
-    def forward_raw(self, pos0: np.ndarray, vel0: np.ndarray, keep_snaps: bool = False):
-        """Run the substeps; return final (pos, vel) as (N, 3) float32 arrays."""
+    def _host_rows(self, n: int):
+        if self._rows is None or self._rows.shape[1] < n:
+            self._rows = torch.zeros((2, n, 4), dtype=torch.float32, pin_memory=torch.cuda.is_available())
+        return self._rows[0, :n], self._rows[1, :n]
+
+    def _run(self, n: int, keep_snaps: bool):
+        """Run the substeps from the state in the host rows, which then hold the
+        final one (id order); returns the snapshots."""
+        p4, v4 = self._host_rows(n)
         self.base.restore()
-        p4 = np.zeros((pos0.shape[0], 4), np.float32)
-        v4 = np.zeros_like(p4)
-        p4[:, :3] = pos0[:, :3]
-        v4[:, :3] = vel0[:, :3]
-        self.sim.upload(p4, v4)
+        self.sim._call("upload_particles", self.sim.h, 0, n, p4.data_ptr(), v4.data_ptr())
         snaps = []
         for s in range(self.nsteps):
             if keep_snaps and s % self.every == 0:
                 snaps.append(capi.SnapshotC(self.sim))
             self._colliders(s)
             self.sim.step(self.prm)
-        pos = self.sim.dump("pos")[:, :3].copy()
-        vel = self.sim.dump("vel")[:, :3].copy()
-        return pos, vel, snaps
+        self.sim._call("dump", self.sim.h, capi.DUMP["pos"], p4.data_ptr(), n * 16)
+        self.sim._call("dump", self.sim.h, capi.DUMP["vel"], v4.data_ptr(), n * 16)
+        return snaps
 
-    def backward_raw(self, snaps, g_pos: np.ndarray, g_vel: np.ndarray):
-        """Gradient of the initial (pos, vel), and of the key positions of each
-        keyed collider, from that of the final state."""
-        adj = capi.AdjointC(self.sim, self.every)
+    def forward_raw(self, pos0: np.ndarray, vel0: np.ndarray, keep_snaps: bool = False):
+        """Run the substeps; return final (pos, vel) as (N, 3) float32 arrays."""
+        n = pos0.shape[0]
+        p4, v4 = (q.numpy() for q in self._host_rows(n))
+        p4[:, :3] = pos0[:, :3]
+        v4[:, :3] = vel0[:, :3]
+        p4[:, 3] = 0.0
+        v4[:, 3] = 0.0
+        snaps = self._run(n, keep_snaps)
+        return p4[:, :3].copy(), v4[:, :3].copy(), snaps
+
+    def _reverse(self, n: int, snaps):
+        """Reverse the recorded segments from the final state's gradient in the host
+        rows, which then hold the initial state's; returns the key gradients."""
+        gp, gv = self._host_rows(n)
+        if self._adj is None or self._adj_slots != self.sim.dims.scap:
+            self._drop_adjoint()
+            self._adj = capi.AdjointC(self.sim, self.every)
+            self._adj_slots = self.sim.dims.scap
+        adj = self._adj
         gkeys = [np.zeros((len(c.times), 3)) for c in self.cols]
         try:
-            adj.seed(g_pos, g_vel)
             for k in reversed(range(len(snaps))):
                 snaps[k].restore()
+                if k == len(snaps) - 1:  # with this pass's particle count, whatever ran since
+                    adj._call("seed", gp.data_ptr(), gv.data_ptr())
                 first = k * self.every
                 seg = min(self.every, self.nsteps - first)
                 ws = []
@@ -169,12 +207,31 @@ class Rollout:
                         g = adj.col_grad(len(self.cols)).astype(np.float64)
                         for q, (wc, wv) in enumerate(ws[s]):
                             gkeys[q] += np.outer(wc, g[q, 0:3]) + np.outer(wv, g[q, 3:6])
-            gp, gv = adj.grad()
-            return gp, gv, gkeys
-        finally:
-            adj.close()
+            if snaps:
+                adj._call("grad", gp.data_ptr(), gv.data_ptr())
+        except Exception:
+            self._drop_adjoint()  # it may hold tapes of substeps that were not reversed
+            raise
+        return gkeys
+
+    def backward_raw(self, snaps, g_pos: np.ndarray, g_vel: np.ndarray):
+        """Gradient of the initial (pos, vel), and of the key positions of each
+        keyed collider, from that of the final state."""
+        n = self.sim.count()
+        gp, gv = (q.numpy() for q in self._host_rows(n))
+        for dst, src in ((gp, g_pos), (gv, g_vel)):
+            dst[:, :3] = np.asarray(src, np.float32).reshape(n, -1)[:, :3]
+            dst[:, 3] = 0.0
+        gkeys = self._reverse(n, snaps)
+        return gp[:, :3].copy(), gv[:, :3].copy(), gkeys
+
+    def _drop_adjoint(self):
+        if self._adj is not None:
+            self._adj.close()
+            self._adj = None
 
     def close(self):
+        self._drop_adjoint()
         self.base.close()
         self.sim.close()
 
@@ -183,27 +240,31 @@ class _RolloutFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, pos0, vel0, ro: Rollout, *keys):
         ro.set_keys([k.detach().to("cpu", torch.float64).numpy() for k in keys])
-        pos, vel, snaps = ro.forward_raw(_f4(pos0)[:, :3], _f4(vel0)[:, :3], keep_snaps=True)
+        p4, v4 = ro._host_rows(pos0.shape[0])
+        _put(p4, pos0)
+        _put(v4, vel0)
+        snaps = ro._run(pos0.shape[0], True)
         ctx.ro = ro
         ctx.snaps = snaps
         ctx.keys = [k.detach().to("cpu", torch.float64).numpy() for k in keys]
         ctx.kmeta = [(k.device, k.dtype) for k in keys]
         ctx.dev = pos0.device
         ctx.dtype = pos0.dtype
-        return (torch.from_numpy(pos).to(pos0.device, pos0.dtype), torch.from_numpy(vel).to(vel0.device, vel0.dtype))
+        return _take(p4, pos0.device, pos0.dtype), _take(v4, vel0.device, vel0.dtype)
 
     @staticmethod
     def backward(ctx, g_pos, g_vel):
         n = g_pos.shape[0]
-        gp = np.zeros((n, 3), np.float32) if g_pos is None else g_pos.detach().to("cpu", torch.float32).numpy()
-        gv = np.zeros((n, 3), np.float32) if g_vel is None else g_vel.detach().to("cpu", torch.float32).numpy()
+        gp, gv = ctx.ro._host_rows(n)
+        _put(gp, g_pos)
+        _put(gv, g_vel)
         ctx.ro.set_keys(ctx.keys)
-        dp, dv, dk = ctx.ro.backward_raw(ctx.snaps, gp, gv)
+        dk = ctx.ro._reverse(n, ctx.snaps)
         for q in ctx.snaps:
             q.close()
         ctx.snaps = []
         gk = [torch.from_numpy(g).to(dev, dt) for g, (dev, dt) in zip(dk, ctx.kmeta)]
-        return (torch.from_numpy(dp).to(ctx.dev, ctx.dtype), torch.from_numpy(dv).to(ctx.dev, ctx.dtype), None, *gk)
+        return (_take(gp, ctx.dev, ctx.dtype), _take(gv, ctx.dev, ctx.dtype), None, *gk)
 
 
 def splat_density(pos: torch.Tensor, origin, h: float, dims) -> torch.Tensor:

@@ -1250,6 +1250,19 @@ int st_dump_size(void* p, int32_t what, size_t* bytes) {
 int st_dump(void* p, int32_t what, void* dst, size_t bytes) {
   Sim* s = getSim(p);
   if (!s || !dst) return fail(ST_ERR_ARG, "st_dump: null argument");
+  if (what == ST_DUMP_POS || what == ST_DUMP_VEL) {  // put in id order on the device, copied straight into dst
+    if (bytes < size_t(s->N) * 16) return fail(ST_ERR_ARG, "st_dump: buffer too small");
+    if (!s->N) return ST_OK;
+    HIPCHK(hipSetDevice(s->dev));
+    uint32_t* bad = s->G.wg + scan_word_count(s->ntiles) - 1u;  // a word of the tile scan's scratch past its use
+    uint32_t isBad = 0;
+    launch_unsort_checked(s->st, what == ST_DUMP_POS ? s->G.pos : s->G.vel, s->G.pid, s->G.scratch4, s->N, bad);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(&isBad, bad, 4, hipMemcpyDeviceToHost, s->st));
+    HIPCHK(hipMemcpyAsync(dst, s->G.scratch4, size_t(s->N) * 16, hipMemcpyDeviceToHost, s->st));
+    HIPCHK(hipStreamSynchronize(s->st));
+    return isBad ? fail(ST_ERR_STATE, "st_dump: particle id out of range") : ST_OK;
+  }
   size_t need = 0;
   int rc = st_dump_size(p, what, &need);
   if (rc) return rc;
@@ -1282,21 +1295,6 @@ int st_dump(void* p, int32_t what, void* dst, size_t bytes) {
     case ST_DUMP_ACCW: case ST_DUMP_FACEO: return perCell(s->G.accW, 3);
     case ST_DUMP_VELG: return perCell(s->G.velG, 3);
     case ST_DUMP_TMAP: std::memcpy(o, tm.data(), tm.size() * 4); return ST_OK;
-    case ST_DUMP_POS:
-    case ST_DUMP_VEL: {
-      if (!s->N) return ST_OK;
-      // id order: out[pid[i]] = field[i]
-      std::vector<float> f(size_t(s->N) * 4);
-      std::vector<uint32_t> id(s->N);
-      HIPCHK(hipMemcpy(f.data(), what == ST_DUMP_POS ? (const void*)s->G.pos : (const void*)s->G.vel, f.size() * 4, hipMemcpyDeviceToHost));
-      HIPCHK(hipMemcpy(id.data(), s->G.pid, id.size() * 4, hipMemcpyDeviceToHost));
-      float* out = (float*)o;
-      for (size_t i = 0; i < s->N; i++) {
-        if (id[i] >= s->N) return fail(ST_ERR_STATE, "st_dump: particle id out of range");
-        std::memcpy(out + size_t(id[i]) * 4, f.data() + i * 4, 16);
-      }
-      return ST_OK;
-    }
   }
   return fail(ST_ERR_ARG, "st_dump: unknown field");
 }

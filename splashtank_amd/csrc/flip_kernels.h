@@ -145,6 +145,8 @@ void launch_g2p(hipStream_t st, const LaunchCtx& L);
 // g2p workgroups per tile for particles that would fill this many tiles
 uint32_t g2p_split(uint32_t fullTiles);
 void launch_unsort(hipStream_t st, const float4* src, const uint32_t* pid, float4* out, uint32_t n);
+// the same with *bad set when an id is not below n (that particle is left out)
+void launch_unsort_checked(hipStream_t st, const float4* src, const uint32_t* pid, float4* out, uint32_t n, uint32_t* bad);
 // the live view: what one packing needs (positions quantised to 16 bits across the box)
 struct ViewParams {
   float x0, y0, z0, kx, ky, kz, vs, foamLife;  // kx = 65535 / (x1 - x0), ...

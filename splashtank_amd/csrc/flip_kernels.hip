@@ -3356,6 +3356,20 @@ void launch_g2p(hipStream_t st, const LaunchCtx& L) {
   hipLaunchKernelGGL(k_g2p_tile, dim3(g), dim3(WG), 0, st, L.P, L.C, L.G, L.binNext ? 1u : 0u, split);
 }
 
+// the same with every id checked against n: *bad is set for one out of range
+__global__ void k_unsort_checked(const float4* __restrict__ src, const uint32_t* __restrict__ pid, float4* __restrict__ out, uint32_t n,
+                                 uint32_t* __restrict__ bad) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t id = pid[i];
+  if (id < n) out[id] = src[i];
+  else *bad = 1u;
+}
+void launch_unsort_checked(hipStream_t st, const float4* src, const uint32_t* pid, float4* out, uint32_t n, uint32_t* bad) {
+  launch_fill_u32(st, bad, 1, 0u);
+  if (n) hipLaunchKernelGGL(k_unsort_checked, dim3(gridFor(n, WG)), dim3(WG), 0, st, src, pid, out, n, bad);
+}
+
 void CopyList::add(void* d, const void* s, size_t nbytes) {
   if (!nbytes) return;
   dst[n] = d;
