@@ -191,6 +191,7 @@ struct Sim {
     L.binned = binned;
     L.binNext = !nbOn;  // the narrow band's reseed moves particles after g2p
     L.nbOn = nbOn;
+    L.ocean = hp.ocean != 0;
     L.initStep = initStep;
     L.smax = sprayCap;
     L.fullTiles = fullTiles();
@@ -526,6 +527,10 @@ int prepStep(Sim* s, const st_params* o, DParams& Pout, DCols& C) {
     P.oease = 1.0f - st_expf(-8.0f * P.dt);
     for (uint32_t k = 0; k < P.nwave; k++)
       for (int q = 0; q < 8; q++) P.waves[k * 2 + q / 4][q % 4] = o->waves[k * 8 + q];
+    for (uint32_t k = 0; k < P.nwave; k++) {
+      const float kk = std::fmax(P.waves[k * 2 + 1][1], 1.0e-4f), D = std::fmax(P.odepth, 1.0e-3f);
+      P.waves[k * 2 + 1][2] = std::fmax(1.0f - st_expf(-2.0f * kk * D), 1.0e-4f);
+    }
   }
   // opt-in modes (no counterpart in the reference)
   if (o->extrap_layers > ST_EXTRAP_MAX) return fail(ST_ERR_ARG, "st_params.extrap_layers: at most ST_EXTRAP_MAX layers");

@@ -58,7 +58,8 @@ struct DParams {
   // squared lengths of vn - vo (v0 - vo) at or below which g2p's impact (turb)
   // quotient cannot exceed 15 (0.35), so both are 0 there
   float impS2, turbS2;
-  float waves[64][4]; // per wave two rows: (kx, kz, amplitude, angular frequency), (phase, wavenumber, 0, 0)
+  float waves[64][4]; // per wave two rows: (kx, kz, amplitude, angular frequency), (phase, wavenumber,
+                      // 1 - exp(-2 k depth) as d_oceanVel divides by it, 0)
 };
 
 // Collider records: 8 float4 per collider (gpu.js:3-4): (sdf offset, nx, ny, nz),
@@ -313,26 +314,33 @@ __device__ __forceinline__ float d_oceanEta(const DParams& P, float x, float z) 
   return P.olevel + e;
 }
 // water velocity under the waves; the height is stretched so the crest gets the
-// surface value (Wheeler stretching)
-__device__ __forceinline__ float3 d_oceanVel(const DParams& P, float3 p) {
+// surface value (Wheeler stretching).  eta: the surface height at the point's
+// (x, z); angle(k, sn, cs): sine and cosine of wave k's phase there
+template <class AngleT>
+__device__ __forceinline__ float3 d_oceanVelAt(const DParams& P, float y, float eta, AngleT angle) {
   const float D = fmaxf(P.odepth, 1.0e-3f);
-  const float eta = d_oceanEta(P, p.x, p.z);
-  const float ys = st_clampf((p.y - P.oy0) * D / fmaxf(D + eta - P.olevel, 0.1f * D), 0.0f, D);
+  const float ys = st_clampf((y - P.oy0) * D / fmaxf(D + eta - P.olevel, 0.1f * D), 0.0f, D);
   float3 v = make_float3(0.0f, 0.0f, 0.0f);
   for (uint32_t k = 0; k < P.nwave; k++) {
     const float* A = P.waves[k * 2u];
     const float* B = P.waves[k * 2u + 1u];
     const float kk = fmaxf(B[1], 1.0e-4f);
     float sn, cs;
-    st_sincosf_wide(A[0] * p.x + A[1] * p.z - A[3] * P.otime + B[0], &sn, &cs);
+    angle(k, &sn, &cs);
     const float e1 = st_expf(kk * (ys - D));
     const float e2 = st_expf(-kk * (ys + D));
-    const float dn = fmaxf(1.0f - st_expf(-2.0f * kk * D), 1.0e-4f);
+    const float dn = B[2];  // depends on the wave alone: the host's
     const float aw = A[2] * A[3];
     const float hc = aw * (e1 + e2) / dn * cs / kk;
     v = f3add(v, make_float3(hc * A[0], aw * (e1 - e2) / dn * sn, hc * A[1]));
   }
   return v;
+}
+__device__ __forceinline__ float3 d_oceanVel(const DParams& P, float3 p) {
+  return d_oceanVelAt(P, p.y, d_oceanEta(P, p.x, p.z), [&](uint32_t k, float* sn, float* cs) {
+    const float* A = P.waves[k * 2u];
+    st_sincosf_wide(A[0] * p.x + A[1] * p.z - A[3] * P.otime + P.waves[k * 2u + 1u][0], sn, cs);
+  });
 }
 // 1 at the side walls, 0 at the layer's width in from them (0 without the ocean)
 __device__ __forceinline__ float d_layerW(const DParams& P, float3 p) {

@@ -43,6 +43,7 @@ struct LaunchCtx {
   bool binned;        // blocks: need, binCount and binKey already hold A's marks and bins
   bool binNext;       // g2p: mark and bin the positions it writes, for the next substep
   bool nbOn;          // narrow band on this step
+  bool ocean;         // ocean side boundary on this step
   uint32_t initStep;  // narrow-band start: 1 restart, 2 water added, 0 none
   uint32_t smax;      // whitewater slots (host copy of P->smax)
   uint32_t fullTiles; // tiles the particles would fill (n / particles of a full tile), for launch shapes

@@ -964,8 +964,50 @@ __device__ __forceinline__ uint32_t type_at(const DParams& P, const DGrid& G, in
     if (const TileAt T = tile_at(G, u_ >> 1); true)                    \
       if (const uint32_t l = threadIdx.x + (u_ & 1u) * 256u; true)
 
+// The ocean's waves over a half tile's columns.  The cells of a column share x and z,
+// hence the sine and cosine of every wave's phase and the surface height, which are
+// most of what a face's ocean velocity costs (24 waves, two sincos each): they are
+// worked out once per column and axis, not for each of its eight faces twice.
+// normFaces 108 -> 57 us and the starting fill 139 -> 59 us with 24 waves at 72^3 (421
+// tiles); bound by the exponentials and divisions that remain per face.
+#define OC_COLS 96  // 3 axes x (8 x 4) columns
+#define OC_WAVES 32
+struct OceanCols {
+  float2 sc[OC_WAVES][OC_COLS];  // (sine, cosine)
+  float eta[OC_COLS];
+};
+__device__ __forceinline__ uint32_t oc_col(uint32_t axis, uint32_t l) { return axis * 32u + (l & 7u) + 8u * ((l >> 6) & 3u); }
+// for the half tile that holds local cell l0 (0 or 256) of tile T; the whole workgroup calls it
+__device__ __forceinline__ void ocean_cols(const DParams& P, const TileAt& T, uint32_t l0, OceanCols& oc) {
+  __syncthreads();  // the last half tile's readers are done
+  for (uint32_t q = threadIdx.x; q < P.nwave * OC_COLS; q += WG) {
+    const uint32_t k = q / OC_COLS, col = q - k * OC_COLS, axis = col >> 5;
+    const float x = P.x0 + (float(T.x + int32_t(col & 7u)) + (axis == 0u ? 0.0f : 0.5f)) * P.h;
+    const float z = P.z0 + (float(T.z + int32_t((l0 >> 6) + ((col >> 3) & 3u))) + (axis == 2u ? 0.0f : 0.5f)) * P.h;
+    const float* A = P.waves[k * 2u];
+    float sn, cs;
+    st_sincosf_wide(A[0] * x + A[1] * z - A[3] * P.otime + P.waves[k * 2u + 1u][0], &sn, &cs);
+    oc.sc[k][col] = make_float2(sn, cs);
+  }
+  __syncthreads();
+  if (threadIdx.x < OC_COLS) {  // d_oceanEta's sum
+    float e = 0.0f;
+    for (uint32_t k = 0; k < P.nwave; k++) e = e + P.waves[k * 2u][2] * oc.sc[k][threadIdx.x].y;
+    oc.eta[threadIdx.x] = P.olevel + e;
+  }
+  __syncthreads();
+}
+__device__ __forceinline__ float oc_vel(const DParams& P, const OceanCols& oc, uint32_t col, float y, uint32_t axis) {
+  return f3get(d_oceanVelAt(P, y, oc.eta[col], [&](uint32_t k, float* sn, float* cs) {
+    const float2 v = oc.sc[k][col];
+    *sn = v.x;
+    *cs = v.y;
+  }), axis);
+}
+
 // normBody / normFaces (wgsl-solver.js:75-105).  counted: classify's workgroups,
 // whose fluid counts the last workgroup adds up
+template <bool OCEAN>
 __device__ __forceinline__ void norm_faces_body(const DParams* __restrict__ PP, const DCols* __restrict__ C, const DGrid& G,
                                                 uint32_t counted, uint32_t bid, uint32_t nbid) {
   const DParams& P = *PP;
@@ -976,6 +1018,7 @@ __device__ __forceinline__ void norm_faces_body(const DParams* __restrict__ PP, 
     const uint32_t th = type_at(P, G, at.x, at.y, at.z, c);
     const uint32_t cl[3] = {nb_down(T.s, T.xm, l, 0u), nb_down(T.s, T.ym, l, 3u), nb_down(T.s, T.zm, l, 6u)};
     Face3 fv = face3(G.accV, c), fw = face3(G.accW, c);
+    uint32_t waves = 0u;  // axes whose face is the ocean's moving wall
 #pragma unroll
     for (uint32_t axis = 0; axis < 3; axis++) {
       const int3 lo = make_int3(at.x - (axis == 0 ? 1 : 0), at.y - (axis == 1 ? 1 : 0), at.z - (axis == 2 ? 1 : 0));
@@ -989,22 +1032,33 @@ __device__ __forceinline__ void norm_faces_body(const DParams* __restrict__ PP, 
         int32_t ci = -1;
         if (tl == 2u && d_inDom(P, lo)) ci = int32_t((G.ctype[cl[axis]] >> 8) & 0xffu) - 1;
         if (ci < 0 && th == 2u && d_inDom(P, at)) ci = int32_t((G.ctype[c] >> 8) & 0xffu) - 1;
-        float3 fp = d_facePos(P, at, axis);
-        if (ci >= 0) sv = f3get(d_colSurfVel(C, uint32_t(ci), fp), axis);
-        else if (P.ocean != 0u && ((tl == 2u && d_inDom(P, lo)) || (th == 2u && d_inDom(P, at))))
-          sv = f3get(d_oceanVel(P, fp), axis);  // the ocean's moving wall
+        if (ci >= 0) sv = f3get(d_colSurfVel(C, uint32_t(ci), d_facePos(P, at, axis)), axis);
+        else if (OCEAN && ((tl == 2u && d_inDom(P, lo)) || (th == 2u && d_inDom(P, at)))) waves |= 1u << axis;
         v = sv;
         old = sv;
       }
       fw.a[axis] = (int32_t)st_f2u(old);
       fv.a[axis] = (int32_t)st_f2u(v);
     }
+    if constexpr (OCEAN) {
+      __shared__ OceanCols oc;
+      if (__syncthreads_or(waves != 0u)) {
+        ocean_cols(P, T, l & 256u, oc);
+#pragma unroll
+        for (uint32_t axis = 0; axis < 3; axis++)
+          if ((waves >> axis) & 1u) {
+            const float v = oc_vel(P, oc, oc_col(axis, l), d_facePos(P, at, axis).y, axis);
+            fw.a[axis] = fv.a[axis] = (int32_t)st_f2u(v);
+          }
+      }
+    }
     face3_put(G.accW, c, fw);
     face3_put(G.accV, c, fv);
   }
 }
+template <bool OCEAN>
 __global__ void __launch_bounds__(WG) k_norm_faces(const DParams* __restrict__ PP, const DCols* __restrict__ C, DGrid G, uint32_t counted) {
-  norm_faces_body(PP, C, G, counted, blockIdx.x, gridDim.x);
+  norm_faces_body<OCEAN>(PP, C, G, counted, blockIdx.x, gridDim.x);
 }
 
 __device__ __forceinline__ float gvR(const DGrid& G, uint32_t f) { return st_u2f((uint32_t)G.accV[f]); }
@@ -2567,7 +2621,8 @@ __device__ __forceinline__ float3 d_velGVec(const DParams& P, const DGrid& G, fl
 
 // signed distance in cells to the starting water: boxes, spheres, water volumes and
 // the ocean (wgsl-core.js:228-238)
-__device__ __forceinline__ float d_fillPhi(const DParams& P, const DCols* __restrict__ C, const float* __restrict__ sdf, float3 x) {
+// (eta: the ocean's surface height at x, when it is on)
+__device__ __forceinline__ float d_fillPhi(const DParams& P, const DCols* __restrict__ C, const float* __restrict__ sdf, float3 x, float eta) {
   float dd = 1.0e9f;
   for (uint32_t k = 0; k < P.nfill; k++) {
     const float* A = P.fills[k * 2];
@@ -2586,7 +2641,7 @@ __device__ __forceinline__ float d_fillPhi(const DParams& P, const DCols* __rest
     d_sdfEval(C, sdf, k, x, phi, wn);
     dd = fminf(dd, phi);
   }
-  if (P.ocean != 0u) dd = fminf(dd, x.y - d_oceanEta(P, x.x, x.z));
+  if (P.ocean != 0u) dd = fminf(dd, x.y - eta);
   return dd * P.ih;
 }
 // depth at a point from the cell centres around it, collider cells left out
@@ -2638,35 +2693,39 @@ __global__ void k_nb_mark_fill(const DParams* __restrict__ PP, const DCols* __re
   float3 tc = make_float3(float(t % P.tx), float(tt % P.ty), float(tt / P.ty));
   tc = f3add(f3mul(tc, 8.0f), make_float3(4.0f, 4.0f, 4.0f));
   float3 q = f3add(make_float3(P.x0, P.y0, P.z0), f3mul(tc, P.h));
-  if (d_fillPhi(P, C, G.sdf, q) < 9.0f) G.need[t] = 1u;
+  if (d_fillPhi(P, C, G.sdf, q, P.ocean != 0u ? d_oceanEta(P, q.x, q.z) : 0.0f) < 9.0f) G.need[t] = 1u;
 }
 // phiInitAll (wgsl-narrowband.js:21-35)
-__device__ __forceinline__ void nb_phi_init_body(const DParams* __restrict__ PP, const DCols* __restrict__ C,
-                                                 const DGrid& G, uint32_t bid, uint32_t nbid) {
+template <bool OCEAN>
+__global__ void __launch_bounds__(WG) k_nb_phi_init(const DParams* __restrict__ PP, const DCols* __restrict__ C, DGrid G) {
   const DParams& P = *PP;
-  FOR_ACTIVE(G) {
-    uint32_t s = G.slotList[t >> 9], local = t & 511u, c = s * 512u + local;
-    int3 p = d_slotCoord(P, G.slotTile, s, local);
-    float ph = st_clampf(d_fillPhi(P, C, G.sdf, d_cellCenter(P, p.x, p.y, p.z)), -7.9f, 7.9f);
+  const uint32_t bid = blockIdx.x, nbid = gridDim.x;
+  FOR_TILES(G, T, l) {
+    const uint32_t c = T.s * 512u + l;
+    const int3 p = make_int3(T.x + int32_t(l & 7u), T.y + int32_t((l >> 3) & 7u), T.z + int32_t(l >> 6));
+    const float3 x = d_cellCenter(P, p.x, p.y, p.z);
+    float eta = 0.0f, v[3] = {0.0f, 0.0f, 0.0f};  // at rest, or moving with the waves under the ocean's surface
+    if constexpr (OCEAN) {
+      __shared__ OceanCols oc;
+      ocean_cols(P, T, l & 256u, oc);
+      eta = oc.eta[oc_col(1u, l)];  // the y faces' columns are the cell centres'
+      if (P.nbInit == 1u) {
+#pragma unroll
+        for (uint32_t ax = 0; ax < 3; ax++) {
+          const float y = d_facePos(P, p, ax).y;
+          if (y < oc.eta[oc_col(ax, l)]) v[ax] = oc_vel(P, oc, oc_col(ax, l), y, ax);
+        }
+      }
+    }
+    float ph = st_clampf(d_fillPhi(P, C, G.sdf, x, eta), -7.9f, 7.9f);
     if (ph < 0.0f) ph = fminf(ph, -1.5f);
     if (!d_inDom(P, p)) ph = 8.0f;
     uint32_t ct = G.ctype[c];
     if (P.nbInit == 2u) ph = fminf(ph, d_phiOfBits(ct));
     G.ctype[c] = d_phiPutBits(ct, ph);
-    if (P.nbInit == 1u) {  // at rest, or moving with the waves under the ocean's surface
-      for (uint32_t ax = 0; ax < 3; ax++) {
-        float v = 0.0f;
-        if (P.ocean != 0u) {
-          float3 fp = d_facePos(P, p, ax);
-          if (fp.y < d_oceanEta(P, fp.x, fp.z)) v = f3get(d_oceanVel(P, fp), ax);
-        }
-        G.velG[c * 3 + ax] = v;
-      }
-    }
+    if (P.nbInit == 1u)
+      for (uint32_t ax = 0; ax < 3; ax++) G.velG[c * 3 + ax] = v[ax];
   }
-}
-__global__ void k_nb_phi_init(const DParams* __restrict__ PP, const DCols* __restrict__ C, DGrid G) {
-  nb_phi_init_body(PP, C, G, blockIdx.x, gridDim.x);
 }
 // nbPhi (wgsl-narrowband.js:39-49): depth carried by the kept grid velocity
 __device__ __forceinline__ void nb_phi_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid) {
@@ -2829,33 +2888,40 @@ __device__ __forceinline__ float d_hash1(uint32_t n0) {
   x ^= x >> 16; x *= 0x7feb352du; x ^= x >> 15; x *= 0x846ca68bu; x ^= x >> 16;
   return float(x) * 2.3283064e-10f;
 }
-// nbSpawn (wgsl-narrowband.js:135-149): fill the short cells from the dead slots
-__global__ void k_nb_spawn(const DParams* __restrict__ PP, DGrid G, const uint32_t* __restrict__ needA,
+// nbSpawn (wgsl-narrowband.js:135-149): fill the short cells from the dead slots.
+// A workgroup takes WG cells and hands their new particles to its threads one by
+// one (each finds its cell by a search in the cells' starts): a short cell wants up
+// to 64, and one thread after another making a cell's left the others idle (217 ->
+// 27 us in the ocean, whose boundary cells are refilled each substep).
+__global__ void __launch_bounds__(WG) k_nb_spawn(const DParams* __restrict__ PP, DGrid G, const uint32_t* __restrict__ needA,
                            const uint32_t* __restrict__ needStart, const uint32_t* __restrict__ entIdx,
                            const uint32_t* __restrict__ deadList, const uint32_t* __restrict__ deadCount, uint32_t ncap) {
   const DParams& P = *PP;
-  uint32_t tot = G.ctl[4] * 512u, ndead = *deadCount, avail = min(ndead, P.lcap), nent = entIdx[ncap];
-  uint32_t maxe = P.lcap / 2u;
-  for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < tot; t += gridDim.x * blockDim.x) {
-    uint32_t need = needA[t];
-    if (!need) continue;
-    uint32_t e = entIdx[t];
-    if (e >= maxe) continue;
-    uint32_t base = needStart[t];
+  __shared__ uint32_t sStart[WG];
+  const uint32_t tot = G.ctl[4] * 512u, ndead = *deadCount, avail = min(ndead, P.lcap), nent = entIdx[ncap];
+  const uint32_t maxe = P.lcap / 2u;
+  for (uint32_t t0 = blockIdx.x * WG; t0 < tot; t0 += gridDim.x * WG) {  // tot is whole workgroups
+    const uint32_t mine = t0 + threadIdx.x, need0 = needA[mine];
+    __syncthreads();
+    sStart[threadIdx.x] = needStart[mine];
     // nbReset / nbSpawn's ctl[10]: the needs of the entries the spawn served, summed
-    if (e + 1u == min(nent, maxe)) G.ctl[10] = base + need;
-    uint32_t s = G.slotList[t >> 9], local = t & 511u;
-    int3 p = d_slotCoord(P, G.slotTile, s, local);
-    float3 cp = make_float3(float(uint32_t(p.x) & 0xffffu), float(uint32_t(p.y) & 0xffffu), float(uint32_t(p.z) & 0xffffu));
-    for (uint32_t m = 0; m < need; m++) {
-      uint32_t k = base + m;
-      if (k >= avail) break;
-      uint32_t i = deadList[k];
-      uint32_t hh = (e * 9781u + m * 6271u + 17u) ^ (P.seed * 2654435761u);
-      float3 x = f3add(make_float3(P.x0, P.y0, P.z0),
-                       f3mul(f3add(cp, make_float3(d_hash1(hh + 1u), d_hash1(hh + 2u), d_hash1(hh + 3u))), P.h));
-      float3 v = d_velGVec(P, G, x);
-      if (d_layerW(P, x) > 0.25f) v = d_oceanVel(P, x);
+    if (need0 && entIdx[mine] + 1u == min(nent, maxe)) G.ctl[10] = needStart[mine] + need0;
+    __syncthreads();
+    const uint32_t first = sStart[0], end = min(needStart[t0 + WG], avail);
+    for (uint32_t k = first + threadIdx.x; k < end; k += WG) {
+      uint32_t lo = 0u;  // the last cell that starts at or before k
+      for (uint32_t h = WG / 2u; h; h >>= 1)
+        if (sStart[lo + h] <= k) lo += h;
+      const uint32_t t = t0 + lo, m = k - sStart[lo], e = entIdx[t];
+      if (e >= maxe) continue;
+      const uint32_t s = G.slotList[t >> 9], local = t & 511u;
+      const int3 p = d_slotCoord(P, G.slotTile, s, local);
+      const float3 cp = make_float3(float(uint32_t(p.x) & 0xffffu), float(uint32_t(p.y) & 0xffffu), float(uint32_t(p.z) & 0xffffu));
+      const uint32_t i = deadList[k];
+      const uint32_t hh = (e * 9781u + m * 6271u + 17u) ^ (P.seed * 2654435761u);
+      const float3 x = f3add(make_float3(P.x0, P.y0, P.z0),
+                             f3mul(f3add(cp, make_float3(d_hash1(hh + 1u), d_hash1(hh + 2u), d_hash1(hh + 3u))), P.h));
+      const float3 v = d_layerW(P, x) > 0.25f ? d_oceanVel(P, x) : d_velGVec(P, G, x);
       G.pos[i] = make_float4(x.x, x.y, x.z, fminf(f3len(v), 63.0f));
       G.vel[i] = make_float4(v.x, v.y, v.z, 0.0f);
     }
@@ -3015,7 +3081,7 @@ __global__ void __launch_bounds__(WG) kb_classify(BATCH_ARGS) {
 __global__ void __launch_bounds__(WG) kb_norm_faces(BATCH_ARGS, const uint32_t* __restrict__ cells) {
   BATCH_TANK;
   BATCH_STAGED;
-  norm_faces_body(&sP, TC, G, cells[b.t + 1u] - cells[b.t], b.blk, b.nblk);
+  norm_faces_body<false>(&sP, TC, G, cells[b.t + 1u] - cells[b.t], b.blk, b.nblk);  // a batch has no ocean
 }
 __global__ void __launch_bounds__(WG) kb_divergence(BATCH_ARGS) { BATCH_TANK; BATCH_STAGED; divergence_body(&sP, G, b.blk, b.nblk); }
 // one SOR iteration, pres -> pres2 (odd = 0) or back; every tank's range is a
@@ -3199,7 +3265,8 @@ void launch_blocks(hipStream_t st, const LaunchCtx& L) {
   hipLaunchKernelGGL(k_tiles_scan, dim3(nb), dim3(WG), 0, st, L.P, L.G);
   hipLaunchKernelGGL(k_tiles_place, dim3(nb + gridFor(L.n, WG * 4)), dim3(WG), 0, st, L.P, L.G);
   hipLaunchKernelGGL(k_tiles_finish, dim3(nb + tiles_finish_grid(L.scap)), dim3(WG), 0, st, L.P, L.C, L.G, L.full ? 1u : 0u);
-  if (L.initStep) hipLaunchKernelGGL(k_nb_phi_init, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.C, L.G);
+  if (L.initStep && L.ocean) hipLaunchKernelGGL(k_nb_phi_init<true>, dim3(L.faceGrid), dim3(WG), 0, st, L.P, L.C, L.G);
+  else if (L.initStep) hipLaunchKernelGGL(k_nb_phi_init<false>, dim3(L.faceGrid), dim3(WG), 0, st, L.P, L.C, L.G);
 }
 
 void launch_p2g(hipStream_t st, const LaunchCtx& L) {
@@ -3242,7 +3309,8 @@ void launch_reseed(hipStream_t st, const LaunchCtx& L, const NbScratch& S) {
 }
 
 void launch_norm_faces(hipStream_t st, const LaunchCtx& L) {
-  hipLaunchKernelGGL(k_norm_faces, dim3(L.faceGrid), dim3(WG), 0, st, L.P, L.C, L.G, L.cellGrid);
+  if (L.ocean) hipLaunchKernelGGL(k_norm_faces<true>, dim3(L.faceGrid), dim3(WG), 0, st, L.P, L.C, L.G, L.cellGrid);
+  else hipLaunchKernelGGL(k_norm_faces<false>, dim3(L.faceGrid), dim3(WG), 0, st, L.P, L.C, L.G, L.cellGrid);
 }
 
 void launch_divergence(hipStream_t st, const LaunchCtx& L) {
