@@ -768,6 +768,7 @@ struct Batch {
   // captured kernels read, and the captured substeps by their block tables
   uint8_t* dGraph = nullptr;
   struct Captured {
+    bool passes;
     std::vector<uint32_t> tab;
     hipGraphExec_t exec;
   };
@@ -1818,7 +1819,7 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
     pl.marksClean = s->marksClean;
     pl.solid = s->solidDirty;
   }
-  batch_tables(b->plan.data(), nt, itersMax, b->sorResident, hTab);
+  const bool passes = batch_tables(b->plan.data(), nt, full, itersMax, b->sorResident, hTab);
   HIPCHK(hipMemcpyAsync(d, h, b->offTab + batch_table_words(nt, itersMax) * 4u, hipMemcpyHostToDevice, b->st));
   if (!b->evUsed[k]) {
     HIPCHK(hipEventCreateWithFlags(&b->ev[k], hipEventDisableTiming));
@@ -1831,22 +1832,22 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
     const Sim* s0 = b->tanks[0];
     const uint32_t tiles = b->coopGrid < s0->coopGrid ? std::min(b->coopGrid, s0->sorTiles) : s0->sorTiles;
     b->lastResident = launch_batch_step(b->st, (const BTank*)d, (const uint32_t*)(d + b->offTab), hTab, nt, itersMax, b->coopGrid, tiles,
-                                        most, full, b->dPlan) ? 1u : 0u;
+                                        most, full, passes, b->dPlan) ? 1u : 0u;
   } else {
     // the block tables fix every launch's grid and kernel choice; the tank
     // records, parameters and tables are read from the graph slot at run time.
-    // The SOR takes one launch per iteration in a graph: a captured
+    // The SOR takes a launch per iteration or two in a graph: a captured
     // cooperative launch is not scheduled as one when other streams run.
     b->lastResident = 0u;
     const size_t words = batch_table_words(nt, itersMax);
     Batch::Captured* hit = nullptr;
     for (auto& g : b->graphs)
-      if (g.tab.size() == words && std::memcmp(g.tab.data(), hTab, words * 4u) == 0) hit = &g;
+      if (g.passes == passes && g.tab.size() == words && std::memcmp(g.tab.data(), hTab, words * 4u) == 0) hit = &g;
     if (hit) {
       HIPCHK(hipGraphLaunch(hit->exec, b->st));
     } else {
       HIPCHK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
-      launch_batch_step(b->st, (const BTank*)d, (const uint32_t*)(d + b->offTab), hTab, nt, itersMax, 0u, 0u, 0u, 0u, nullptr);
+      launch_batch_step(b->st, (const BTank*)d, (const uint32_t*)(d + b->offTab), hTab, nt, itersMax, 0u, 0u, 0u, 0u, passes, nullptr);
       hipError_t le = hipGetLastError();
       hipGraph_t g = nullptr;
       hipError_t ce = hipStreamEndCapture(b->st, &g);
@@ -1855,6 +1856,7 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
         return fail(ST_ERR_HIP, std::string("st_batch_step_n: capture: ") + hipGetErrorString(le != hipSuccess ? le : ce));
       }
       Batch::Captured c;
+      c.passes = passes;
       c.tab.assign(hTab, hTab + words);
       hipError_t ie = hipGraphInstantiate(&c.exec, g, nullptr, nullptr, 0);
       (void)hipGraphDestroy(g);

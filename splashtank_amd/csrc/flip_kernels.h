@@ -87,24 +87,27 @@ struct BTankPlan {
 };
 // Block tables of a batched substep: table k holds nt + 1 workgroup starts, one
 // range per tank (empty where the tank has no work in that launch).  Table
-// BT_PIPE0 + it belongs to SOR iteration it.
+// BT_PIPE0 + it belongs to SOR iteration (or pass) it.
 enum BatchTable {
   BT_FILL_MARK, BT_MARK, BT_SCAN, BT_PLACE, BT_FINISH, BT_ONE, BT_CELL,
   BT_TILE, BT_SOLID, BT_COPY, BT_G2P, BT_PIPE0
 };
 size_t batch_table_words(uint32_t nt, uint32_t itersMax);
-// fills the tables (host copy); sorResident = SOR workgroups resident at once
-void batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t itersMax, uint32_t sorResident, uint32_t* tab);
+// fills the tables (host copy); full: tiles the tanks' particles would fill,
+// sorResident = SOR workgroups resident at once; returns whether SOR launches that
+// are not one cooperative launch take two iterations each
+bool batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t full, uint32_t itersMax, uint32_t sorResident, uint32_t* tab);
 // every stage of one substep for all tanks, one launch per kernel: dT and dtab
 // are the device copies of the tank records and tables, htab the host copy
 // coopGrid > 0 (and a plan buffer of batch_plan_words): the SOR of every tank in
 // one cooperative launch, with a workgroup per fluid tile where the device holds
-// that many (sorTiles; most: tiles the tanks can have in use, full: tiles their
-// particles would fill) or of coopGrid resident workgroups, else (or when the
-// launch is refused) one launch per iteration; returns whether it ran resident
+// that many (sorTiles; most: tiles the tanks can have in use) or of coopGrid
+// resident workgroups, else (or when the launch is refused) one launch per
+// iteration, or per two where `passes` (batch_tables); returns whether it ran
+// resident
 inline size_t batch_plan_words(uint32_t nt) { return size_t(nt) * 4u + 2u; }
 bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, const uint32_t* htab, uint32_t nt, uint32_t itersMax,
-                       uint32_t coopGrid, uint32_t sorTiles, uint32_t most, uint32_t full, uint32_t* dPlan);
+                       uint32_t coopGrid, uint32_t sorTiles, uint32_t most, uint32_t full, bool passes, uint32_t* dPlan);
 
 // device-to-device copies made by one launch: whole words, starts aligned to 16
 // bytes (allocations are), at most COPY_LIST_MAX

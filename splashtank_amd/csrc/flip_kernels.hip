@@ -1332,18 +1332,17 @@ __device__ __forceinline__ void sor_pipe_pass(const DGrid& G, float omega, const
 }
 
 // One red-black iteration per launch (the grid a multiple of 8 workgroups, as
-// many as are resident), skipped when the resident solve has done this stage.
+// many as are resident).
 __device__ __forceinline__ void sor_pipe_body(const DParams* __restrict__ PP, const DGrid& G, const float* __restrict__ pin,
-                                              float* __restrict__ pout, uint32_t seq, uint32_t bid, uint32_t nbid) {
+                                              float* __restrict__ pout, uint32_t bid, uint32_t nbid) {
   __shared__ SorPipeLds L;
-  if (G.sorBar[COOP_MAX_WG] == seq) return;
   if (bid == 0u && threadIdx.x == 0u) G.sorBar[COOP_MAX_WG + 3] = 0u;  // the path of this solve
   sor_pipe_init(L, threadIdx.x);
   sor_pipe_pass(G, PP->omega, pin, pout, bid, nbid, threadIdx.x, L);
 }
 __global__ void __launch_bounds__(WG) k_sor_pipe(const DParams* __restrict__ PP, DGrid G, const float* __restrict__ pin,
-                                                 float* __restrict__ pout, uint32_t seq) {
-  sor_pipe_body(PP, G, pin, pout, seq, blockIdx.x, gridDim.x);
+                                                 float* __restrict__ pout) {
+  sor_pipe_body(PP, G, pin, pout, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1581,7 +1580,7 @@ __device__ __forceinline__ void sor_resident_body(const DParams* __restrict__ PP
   if (tid == 0u) sFail = 0u;
   if (stream || nact > ng * COOP_TMAX) {
     // Streaming mode, for more tiles than fit in LDS: four tile pipelines of 256
-    // threads per workgroup run the per-iteration pass (as k_sor_pipe, virtual
+    // threads per workgroup run the per-iteration pass (virtual
     // workgroup g * grid + w), with a grid barrier between iterations.
     const uint32_t g = tid >> 8, gt = tid & 255u;
     SorPipeLds& L = reinterpret_cast<SorPipeLds*>(smem)[g];
@@ -1960,6 +1959,45 @@ __device__ __forceinline__ uint32_t ts_find(const DGrid& G, uint32_t nact, uint3
   return sB;
 }
 
+// The 27 tiles around tile b of slotList (lanes 0 .. 26): their slots, and their
+// places in slotList where they hold fluid (else ST_NONE).
+__device__ __forceinline__ void ts_around(const DGrid& G, uint32_t b, uint32_t* sSlot, uint32_t* sPos) {
+  if (threadIdx.x < 27u) {
+    const uint32_t ns = G.nbrL[b * 27u + threadIdx.x];
+    uint32_t pos = ST_NONE;
+    if (!sor_missing(ns)) {
+      pos = G.slotPos[ns];
+      if (*reinterpret_cast<const uint16_t*>(G.posFluid + 2u * pos) == 0u) pos = ST_NONE;
+    }
+    sSlot[threadIdx.x] = ns;
+    sPos[threadIdx.x] = pos;
+  }
+}
+// a cell of the lists: a = its place in the window (ST_NONE: none) becomes its byte
+// offset and stencil byte as ts_relax takes them, with its rhs
+__device__ __forceinline__ void ts_item(const DGrid& G, const uint32_t* sSlot, const uint32_t* sPos, uint32_t own, uint32_t& a, float& rhs) {
+  const uint32_t i = a, q = i == ST_NONE ? 13u : ts_tile(i);
+  const bool in = i != ST_NONE && sPos[q] != ST_NONE;
+  const uint32_t c = (in ? sSlot[q] : sSlot[13]) * 512u + (in ? ts_local(i) : 0u), st = G.sten[c];
+  rhs = G.rhs[c];
+  a = in && (st & STEN_FLUID) ? ts_window(i) * 4u | (st << 16) : own * 4u;
+}
+// the sweeps of n iterations (1 or 2) on the window
+__device__ __forceinline__ void ts_sweeps(float* sp, uint32_t n, const uint32_t* ra, const float* rr, const uint32_t* ba, const float* br,
+                                          float omega, const float* ytab) {
+  if (n == 2u) {
+    ts_relax<4>(sp, ra, rr, omega, ytab);
+    __syncthreads();
+    ts_relax<3>(sp, ba, br, omega, ytab);
+    __syncthreads();
+  }
+  if (threadIdx.x < 192u) ts_relax<2>(sp, ra, rr, omega, ytab);  // red within distance 1: the first 448
+  else ts_relax<1>(sp, ra, rr, omega, ytab);
+  __syncthreads();
+  ts_relax<1>(sp, ba, br, omega, ytab);  // the tile's black cells
+  __syncthreads();
+}
+
 // The solve of one tile: b its place in slotList (ts_find).
 __device__ __forceinline__ void sor_tile_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t iters, uint32_t tag0, uint32_t b) {
   __shared__ float sp[TS_W3];
@@ -1978,16 +2016,7 @@ __device__ __forceinline__ void sor_tile_body(const DParams* __restrict__ PP, co
 #pragma unroll
   for (uint32_t j = 0; j < TS_KPOLL; j++) pa[j] = tid + j * WG < TS_NPOLL ? kTileCells.poll[tid + j * WG] : ST_NONE;
   uint32_t p0 = tid < TS_NPOLL0 ? kTileCells.poll[TS_NPOLL + tid] : ST_NONE;
-  if (tid < 27u) {
-    const uint32_t ns = G.nbrL[b * 27u + tid];
-    uint32_t pos = ST_NONE;
-    if (!sor_missing(ns)) {
-      pos = G.slotPos[ns];
-      if (*reinterpret_cast<const uint16_t*>(G.posFluid + 2u * pos) == 0u) pos = ST_NONE;
-    }
-    sSlot[tid] = ns;
-    sPos[tid] = pos;
-  }
+  ts_around(G, b, sSlot, sPos);
   if (tid < 8u) ytab[tid] = (tid >= 1u && tid <= 6u) ? 1.0f / float(tid) : 0.0f;
   if (tid == 0u) sFail = 0u;
   for (uint32_t q = tid; q < TS_W3; q += WG) sp[q] = 0.0f;
@@ -1998,17 +2027,10 @@ __device__ __forceinline__ void sor_tile_body(const DParams* __restrict__ PP, co
   sp[own] = pres[tid];
   sp[own + half] = pres[tid + 256u];
   // rhs and stencil of the cells, in registers for the whole solve
-  auto item = [&](uint32_t& a, float& rhs) {
-    const uint32_t i = a, q = i == ST_NONE ? 13u : ts_tile(i);
-    const bool in = i != ST_NONE && sPos[q] != ST_NONE;
-    const uint32_t c = (in ? sSlot[q] : sSlot[13]) * 512u + (in ? ts_local(i) : 0u), st = G.sten[c];
-    rhs = G.rhs[c];
-    a = in && (st & STEN_FLUID) ? ts_window(i) * 4u | (st << 16) : own * 4u;
-  };
 #pragma unroll
-  for (uint32_t j = 0; j < 4u; j++) item(ra[j], rr[j]);
+  for (uint32_t j = 0; j < 4u; j++) ts_item(G, sSlot, sPos, own, ra[j], rr[j]);
 #pragma unroll
-  for (uint32_t j = 0; j < 3u; j++) item(ba[j], br[j]);
+  for (uint32_t j = 0; j < 3u; j++) ts_item(G, sSlot, sPos, own, ba[j], br[j]);
   // a polled word: its place in the buffer (20 bits) | its cell in the window << 20
   auto pollAt = [&](uint32_t i) {
     const uint32_t p = i == ST_NONE ? ST_NONE : sPos[ts_tile(i)];
@@ -2067,17 +2089,7 @@ __device__ __forceinline__ void sor_tile_body(const DParams* __restrict__ PP, co
 #pragma unroll
     for (uint32_t j = 0; j < 3u; j++) asm volatile("" : "+v"(ba[j]));
     const uint32_t n = min(2u, iters - it);
-    if (n == 2u) {
-      ts_relax<4>(sp, ra, rr, omega, ytab);
-      __syncthreads();
-      ts_relax<3>(sp, ba, br, omega, ytab);
-      __syncthreads();
-    }
-    if (tid < 192u) ts_relax<2>(sp, ra, rr, omega, ytab);  // red within distance 1: the first 448
-    else ts_relax<1>(sp, ra, rr, omega, ytab);
-    __syncthreads();
-    ts_relax<1>(sp, ba, br, omega, ytab);  // the tile's black cells
-    __syncthreads();
+    ts_sweeps(sp, n, ra, rr, ba, br, omega, ytab);
     it += n;
     if (it >= iters) break;
     g++;
@@ -2107,18 +2119,90 @@ __global__ void __launch_bounds__(WG, TS_WAVES) k_sor_tiles(const DParams* __res
   if (b != ST_NONE) sor_tile_body(PP, G, iters, tag0, b);
 }
 
-// after an odd number of iterations the result sits in the partner buffer
-__device__ __forceinline__ void copy_tiles_body(const DGrid& G, const float* __restrict__ src, float* __restrict__ dst,
-                                                uint32_t seq, uint32_t bid, uint32_t nbid) {
-  if (G.sorBar[COOP_MAX_WG] == seq) return;
+// Where the solve cannot be one cooperative launch (graph replays, sor_mode 1) and
+// the tiles are few (sor_passes_few): a launch per two iterations, the same windows
+// read from one pressure buffer and the tiles written to the other.  Tiles without
+// fluid are never read (they stand for zeros) nor written.
+// Bounds: the launch (about 3 us) and the window's three dependent loads.  Per
+// iteration, one launch each before: 16^3 tank 4.65 -> 3.93 us, 64^3 4.88 -> 4.01,
+// 96^3 (particles of 415 full tiles) 5.84 -> 5.24; at 128^3 (1050) the windows'
+// extra cells cost more than the launches they save, 7.4 -> 7.8, and at 256^3
+// 27 -> 32: there k_sor_pipe.
+// The launches of a solve are even in number, so that the result ends in pres: two
+// iterations each, and one each in the last two or three where the count asks for
+// it.  A solve of one iteration takes k_sor_pipe.
+__host__ __device__ __forceinline__ uint32_t sor_pass_doubles(uint32_t iters) { return (iters >> 1) - (((iters + (iters & 1u)) >> 1) & 1u); }
+__host__ __device__ __forceinline__ uint32_t sor_passes(uint32_t iters) { return iters - sor_pass_doubles(iters); }
+static bool sor_passes_few(uint32_t fullTiles, uint32_t iters) { return iters >= 2u && fullTiles < 700u; }
+__device__ __forceinline__ void sor_pass_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t iters, uint32_t pass, uint32_t bid,
+                                              uint32_t nbid) {
+  __shared__ float sp[TS_W3];
+  __shared__ uint32_t sSlot[27], sPos[27];
+  __shared__ float ytab[8];
+  const uint32_t tid = threadIdx.x, nact = G.ctl[4], n = pass < sor_pass_doubles(iters) ? 2u : 1u;
+  const float omega = PP->omega;
+  const float* pin = (pass & 1u) ? G.pres2 : G.pres;
+  float* pout = (pass & 1u) ? G.pres : G.pres2;
+  if (bid == 0u && tid == 0u) G.sorBar[COOP_MAX_WG + 3] = 0u;  // the path of this solve
+  if (tid < 8u) ytab[tid] = (tid >= 1u && tid <= 6u) ? 1.0f / float(tid) : 0.0f;
+  const uint32_t x = (tid & 7u) + 4u, y = ((tid >> 3) & 7u) + 4u, z = (tid >> 6) + 4u, own = x + TS_Y * y + TS_Z * z;
+  constexpr uint32_t half = 4u * TS_Z;
+  for (uint32_t b = bid; b < nact; b += nbid) {
+    if (*reinterpret_cast<const uint16_t*>(G.posFluid + 2u * b) == 0u) continue;
+    uint32_t ra[4], ba[3], pa[TS_KPOLL];
+    float rr[4], br[3];
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; j++) ra[j] = tid + j * WG < TS_NRED ? kTileCells.red[tid + j * WG] : ST_NONE;
+#pragma unroll
+    for (uint32_t j = 0; j < 3u; j++) ba[j] = tid + j * WG < TS_NBLACK ? kTileCells.black[tid + j * WG] : ST_NONE;
+#pragma unroll
+    for (uint32_t j = 0; j < TS_KPOLL; j++) pa[j] = tid + j * WG < TS_NPOLL ? kTileCells.poll[tid + j * WG] : ST_NONE;
+    const uint32_t p0 = tid < TS_NPOLL0 ? kTileCells.poll[TS_NPOLL + tid] : ST_NONE;
+    __syncthreads();  // the last tile's window is free
+    ts_around(G, b, sSlot, sPos);
+    for (uint32_t q = tid; q < TS_W3; q += WG) sp[q] = 0.0f;
+    __syncthreads();
+    auto fetch = [&](uint32_t i) {
+      const uint32_t q = i == ST_NONE ? 13u : ts_tile(i);
+      return i != ST_NONE && sPos[q] != ST_NONE ? pin[sSlot[q] * 512u + ts_local(i)] : 0.0f;
+    };
+    float v[TS_KPOLL];
+#pragma unroll
+    for (uint32_t j = 0; j < TS_KPOLL; j++) v[j] = fetch(pa[j]);
+    const float v0 = fetch(p0);
+    const size_t at = size_t(sSlot[13]) * 512u;
+    const float own0 = pin[at + tid], own1 = pin[at + tid + 256u];
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; j++) ts_item(G, sSlot, sPos, own, ra[j], rr[j]);
+#pragma unroll
+    for (uint32_t j = 0; j < 3u; j++) ts_item(G, sSlot, sPos, own, ba[j], br[j]);
+#pragma unroll
+    for (uint32_t j = 0; j < TS_KPOLL; j++)
+      if (pa[j] != ST_NONE) sp[ts_window(pa[j])] = v[j];
+    if (p0 != ST_NONE) sp[ts_window(p0)] = v0;
+    sp[own] = own0;
+    sp[own + half] = own1;
+    __syncthreads();
+    ts_sweeps(sp, n, ra, rr, ba, br, omega, ytab);
+    pout[at + tid] = sp[own];
+    pout[at + tid + 256u] = sp[own + half];
+  }
+}
+__global__ void __launch_bounds__(WG, TS_WAVES) k_sor_pass(const DParams* __restrict__ PP, DGrid G, uint32_t iters, uint32_t pass) {
+  sor_pass_body(PP, G, iters, pass, blockIdx.x, gridDim.x);
+}
+
+// after an odd number of single iterations the result sits in the partner buffer
+__device__ __forceinline__ void copy_tiles_body(const DGrid& G, const float* __restrict__ src, float* __restrict__ dst, uint32_t bid,
+                                                uint32_t nbid) {
   uint32_t tot = G.ctl[4] * 512u;
   for (uint32_t t = bid * blockDim.x + threadIdx.x; t < tot; t += nbid * blockDim.x) {
     uint32_t c = G.slotList[t >> 9] * 512u + (t & 511u);
     dst[c] = src[c];
   }
 }
-__global__ void k_copy_tiles(DGrid G, const float* __restrict__ src, float* __restrict__ dst, uint32_t seq) {
-  copy_tiles_body(G, src, dst, seq, blockIdx.x, gridDim.x);
+__global__ void k_copy_tiles(DGrid G, const float* __restrict__ src, float* __restrict__ dst) {
+  copy_tiles_body(G, src, dst, blockIdx.x, gridDim.x);
 }
 
 // projBody / project (wgsl-solver.js:165-180)
@@ -3084,14 +3168,19 @@ __global__ void __launch_bounds__(WG) kb_norm_faces(BATCH_ARGS, const uint32_t* 
   norm_faces_body<false>(&sP, TC, G, cells[b.t + 1u] - cells[b.t], b.blk, b.nblk);  // a batch has no ocean
 }
 __global__ void __launch_bounds__(WG) kb_divergence(BATCH_ARGS) { BATCH_TANK; BATCH_STAGED; divergence_body(&sP, G, b.blk, b.nblk); }
-// one SOR iteration, pres -> pres2 (odd = 0) or back; every tank's range is a
-// multiple of 8 workgroups starting at a multiple of 8, so a workgroup's place
-// within its tank keeps the XCD it runs on
+// one SOR iteration, pres -> pres2 (odd = 0) or back, or pass `pass` of the few-tile
+// form; every tank's range is a multiple of 8 workgroups starting at a multiple of
+// 8, so a workgroup's place within its tank keeps the XCD it runs on
 __global__ void __launch_bounds__(WG) kb_sor_pipe(BATCH_ARGS, uint32_t odd) {
   BATCH_TANK;
-  sor_pipe_body(TP, T.G, odd ? T.G.pres2 : T.G.pres, odd ? T.G.pres : T.G.pres2, ST_NONE, b.blk, b.nblk);
+  sor_pipe_body(TP, T.G, odd ? T.G.pres2 : T.G.pres, odd ? T.G.pres : T.G.pres2, b.blk, b.nblk);
 }
-__global__ void kb_copy_tiles(BATCH_ARGS) { BATCH_TANK; copy_tiles_body(T.G, T.G.pres2, T.G.pres, ST_NONE, b.blk, b.nblk); }
+__global__ void __launch_bounds__(WG, TS_WAVES) kb_sor_pass(BATCH_ARGS, uint32_t pass) {
+  BATCH_TANK;
+  const DGrid G = T.G;
+  sor_pass_body(TP, G, TP->iters, pass, b.blk, b.nblk);
+}
+__global__ void kb_copy_tiles(BATCH_ARGS) { BATCH_TANK; copy_tiles_body(T.G, T.G.pres2, T.G.pres, b.blk, b.nblk); }
 // Batched resident SOR.  The tanks' solves run in one cooperative launch of
 // the resident workgroups (one per CU): each tank gets a range of them, in one
 // of a few phases when all tanks' tiles do not fit in LDS at once, and runs
@@ -3384,15 +3473,19 @@ hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters) {
     if (coopErr == hipSuccess) return hipSuccess;
     (void)hipGetLastError();  // the per-iteration launches below do the solve
   }
-  // one iteration per launch, ping-pong between the two pressure buffers; an
-  // odd count leaves the result in pres2 and it is copied back.
+  // one or two iterations a launch, ping-pong between the two pressure buffers; an
+  // odd count of single ones leaves the result in pres2 and it is copied back
+  if (sor_passes_few(L.fullTiles, uint32_t(iters))) {
+    for (uint32_t k = 0; k < sor_passes(uint32_t(iters)); k++)
+      hipLaunchKernelGGL(k_sor_pass, dim3(L.pipeGrid), dim3(WG), 0, st, L.P, L.G, uint32_t(iters), k);
+    return coopErr;
+  }
   for (int it = 0; it < iters; it++) {
     const float* pin = (it & 1) ? L.G.pres2 : L.G.pres;
     float* pout = (it & 1) ? L.G.pres : L.G.pres2;
-    hipLaunchKernelGGL(k_sor_pipe, dim3(L.pipeGrid), dim3(WG), 0, st, L.P, L.G, pin, pout, L.sorSeq);
+    hipLaunchKernelGGL(k_sor_pipe, dim3(L.pipeGrid), dim3(WG), 0, st, L.P, L.G, pin, pout);
   }
-  if (iters & 1)
-    hipLaunchKernelGGL(k_copy_tiles, dim3(L.cellGrid), dim3(WG), 0, st, L.G, (const float*)L.G.pres2, L.G.pres, L.sorSeq);
+  if (iters & 1) hipLaunchKernelGGL(k_copy_tiles, dim3(L.cellGrid), dim3(WG), 0, st, L.G, (const float*)L.G.pres2, L.G.pres);
   return coopErr;
 }
 
@@ -3474,10 +3567,12 @@ static uint32_t batch_share(uint64_t total, uint64_t part, uint64_t whole, uint3
   return uint32_t(std::max<uint64_t>(1u, std::min<uint64_t>(c, most)));
 }
 
-void batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t itersMax, uint32_t sorResident, uint32_t* tab) {
+bool batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t full, uint32_t itersMax, uint32_t sorResident, uint32_t* tab) {
   uint64_t scapTot = 0, binTot = 0;
+  bool passes = true;
   for (uint32_t t = 0; t < nt; t++)
     if (plan[t].n) {
+      passes = passes && sor_passes_few(full, plan[t].iters);
       scapTot += plan[t].scap;
       binTot += plan[t].ntiles + 1u;
     }
@@ -3501,13 +3596,13 @@ void batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t itersMax, uint32_
           case BT_CELL: c = cell; break;
           case BT_TILE: c = batch_share(BATCH_TILE_WG, p.scap, scapTot, std::max<uint32_t>(1u, std::min<uint32_t>(p.scap, 8192u))); break;
           case BT_SOLID: c = p.solid ? cell : 0u; break;
-          case BT_COPY: c = (p.iters & 1u) ? cell : 0u; break;
+          case BT_COPY: c = !passes && (p.iters & 1u) ? cell : 0u; break;
           case BT_G2P: c = batch_share(BATCH_TILE_WG, p.ntiles + 1u, binTot, std::min<uint32_t>((p.ntiles + 1u) * p.split, 8192u)); break;
           default: {
             // SOR: the tank's share of the resident workgroups by pool size,
             // whole groups of 8, at least one group and at most one workgroup
             // per slot (rounded up to 8)
-            if (k - uint32_t(BT_PIPE0) >= p.iters) break;
+            if (k - uint32_t(BT_PIPE0) >= (passes ? sor_passes(p.iters) : p.iters)) break;
             const uint32_t most = (p.scap + 7u) & ~7u;
             uint32_t share = uint32_t((uint64_t(sorResident) * p.scap + scapTot - 1u) / scapTot);
             share = (share + 7u) & ~7u;
@@ -3520,10 +3615,11 @@ void batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t itersMax, uint32_
     }
     s[nt] = acc;
   }
+  return passes;
 }
 
 bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, const uint32_t* htab, uint32_t nt, uint32_t itersMax,
-                       uint32_t coopGrid, uint32_t sorTiles, uint32_t most, uint32_t full, uint32_t* dPlan) {
+                       uint32_t coopGrid, uint32_t sorTiles, uint32_t most, uint32_t full, bool passes, uint32_t* dPlan) {
   const size_t w = size_t(nt) + 1u;
   auto tab = [&](uint32_t k) { return dtab + k * w; };
   auto tot = [&](uint32_t k) { return htab[k * w + nt]; };
@@ -3568,7 +3664,11 @@ bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, co
     if (!resident) (void)hipGetLastError();  // the launches per iteration below do the solve
   }
   if (!resident) {
-    for (uint32_t it = 0; it < itersMax; it++) BLAUNCH(kb_sor_pipe, uint32_t(BT_PIPE0) + it, WG, it & 1u);
+    if (passes) {
+      for (uint32_t k = 0; k < sor_passes(itersMax); k++) BLAUNCH(kb_sor_pass, uint32_t(BT_PIPE0) + k, WG, k);
+    } else {
+      for (uint32_t it = 0; it < itersMax; it++) BLAUNCH(kb_sor_pipe, uint32_t(BT_PIPE0) + it, WG, it & 1u);
+    }
     BLAUNCH(kb_copy_tiles, BT_COPY, WG);
   }
   // project, g2p (which marks and bins the next substep)
