@@ -2470,7 +2470,7 @@ __device__ __forceinline__ void foam_table_body(const DParams* __restrict__ PP, 
     G.foamTab[t] = d_foamRow(*PP, float(t));
 }
 
-template <class GridT>
+template <bool OCEAN, class GridT>
 __device__ __forceinline__ void g2p_particle(const DParams& P, const DCols* __restrict__ C, const DGrid& G, const GridT& g,
                                              bool storage, float4 p4, float4 v04, float4& po, float4& vo4) {
   const float* __restrict__ sdf = G.sdf;
@@ -2483,7 +2483,7 @@ __device__ __forceinline__ void g2p_particle(const DParams& P, const DCols* __re
   float3 fl = f3add(v0, f3sub(vn, vo));
   float3 v = make_float3(st_mixf(vn.x, fl.x, P.flip), st_mixf(vn.y, fl.y, P.flip), st_mixf(vn.z, fl.z, P.flip));
   float lw = 0.0f;
-  if (P.ocean != 0u) {  // near the ocean's boundary, ease into the waves (wgsl-solver.js:218)
+  if constexpr (OCEAN) {  // near the ocean's boundary, ease into the waves (wgsl-solver.js:218)
     lw = d_layerW(P, p);
     if (lw > 0.0f) {
       const float s = st_clampf(lw * 2.0f, 0.0f, 1.0f);
@@ -2520,7 +2520,7 @@ __device__ __forceinline__ void g2p_particle(const DParams& P, const DCols* __re
   if (air != 0.0f) spray = air * (0.25f + 0.75f * st_clampf(f3len(v) / 4.0f, 0.0f, 1.0f));
   float foam = v04.w * ft.z;
   foam = fmaxf(foam, fmaxf(spray * 0.9f, fmaxf(impact, turb * 0.8f)));
-  if (P.ocean != 0u) foam = foam * (1.0f - st_clampf(lw * 2.0f, 0.0f, 1.0f));  // easing is not churning (wgsl-solver.js:248)
+  if constexpr (OCEAN) foam = foam * (1.0f - st_clampf(lw * 2.0f, 0.0f, 1.0f));  // easing is not churning (wgsl-solver.js:248)
   float3 gust = make_float3(0.0f, 0.0f, 0.0f);
   if (P.q7 > 0.0f && P.q4 > 0.0f && (!fast || shield < 0.9f)) {
     float3 gp = f3mul(p, 0.55f);
@@ -2588,6 +2588,7 @@ __device__ __forceinline__ void g2p_emit(const DParams& P, const DGrid& G, uint3
   if (keys) bin_mark(P, G, k, valid, po);
 }
 
+template <bool OCEAN>
 __device__ __forceinline__ void g2p_tile_body(const DParams* __restrict__ PP, const DCols* __restrict__ C, const DGrid& G,
                                               uint32_t keys, uint32_t split, uint32_t bid, uint32_t nbid) {
   const DParams& P = *PP;
@@ -2624,7 +2625,7 @@ __device__ __forceinline__ void g2p_tile_body(const DParams* __restrict__ PP, co
         bool valid = k < end;
         uint32_t i = valid ? G.binIdx[k] : 0u;
         float4 po = make_float4(0.f, -1.0e6f, 0.f, 0.f), vo = po;
-        if (valid) g2p_particle(P, C, G, gg, false, G.pos[i], G.vel[i], po, vo);
+        if (valid) g2p_particle<OCEAN>(P, C, G, gg, false, G.pos[i], G.vel[i], po, vo);
         g2p_emit(P, G, keys, k, i, valid, po, vo);
       }
       continue;
@@ -2667,15 +2668,18 @@ __device__ __forceinline__ void g2p_tile_body(const DParams* __restrict__ PP, co
       bool valid = k < end;
       uint32_t i = valid ? G.binIdx[k] : 0u;
       float4 po = make_float4(0.f, -1.0e6f, 0.f, 0.f), vo = po;
-      if (valid) g2p_particle(P, C, G, wg, true, G.pos[i], G.vel[i], po, vo);
+      if (valid) g2p_particle<OCEAN>(P, C, G, wg, true, G.pos[i], G.vel[i], po, vo);
       g2p_emit(P, G, keys, k, i, valid, po, vo);
     }
     __syncthreads();
   }
 }
-__global__ void __launch_bounds__(WG) k_g2p_tile(const DParams* __restrict__ PP, const DCols* __restrict__ C, DGrid G,
+// Five waves per SIMD, as many as the window leaves room for: 1051 -> 1032 us at 33.5
+// million particles (four waves, 100 registers: 1139).
+template <bool OCEAN>
+__global__ void __launch_bounds__(WG, 5) k_g2p_tile(const DParams* __restrict__ PP, const DCols* __restrict__ C, DGrid G,
                                                  uint32_t keys, uint32_t split) {
-  g2p_tile_body(PP, C, G, keys, split, blockIdx.x, gridDim.x);
+  g2p_tile_body<OCEAN>(PP, C, G, keys, split, blockIdx.x, gridDim.x);
 }
 
 // kept grid velocity at a point, all three components (wgsl-core.js:185-197)
@@ -3093,25 +3097,17 @@ typedef const DCols __attribute__((address_space(4))) ConstDCols;
   __builtin_assume_dereferenceable(&T, sizeof(BTank));      \
   __builtin_assume_dereferenceable(TP, sizeof(DParams));    \
   __builtin_assume_dereferenceable(TC, sizeof(DCols))
-// For g2p the tank's parameter block is copied into LDS once per workgroup:
-// read through the pointer above, the compiler cannot treat it as invariant
-// there and reads its words with vector loads at each use; from LDS they are
-// cheap.  (The other kernels read few words, and their grids can be large.)
-__device__ __forceinline__ void batch_stage_params(DParams& dst, const DParams* __restrict__ src) {
-  static_assert(sizeof(DParams) % 4 == 0, "word copy");
-  for (uint32_t q = threadIdx.x; q < sizeof(DParams) / 4; q += blockDim.x)
-    reinterpret_cast<uint32_t*>(&dst)[q] = reinterpret_cast<const uint32_t*>(src)[q];
-  __syncthreads();
-}
-
-// The cell kernels (one pass per cell of the tank's tiles in use) store into the
-// grid between their reads of the parameter block and the grid's pointers.  Read
-// through the tank table, neither can be proven unaffected by those stores, so
-// each would be loaded again (with vector loads) after every store; the LDS copy
-// of the block and a local copy of the pointers are loaded once.
-#define BATCH_STAGED            \
-  __shared__ DParams sP;        \
-  batch_stage_params(sP, TP);   \
+// For g2p and the cell kernels, local copies of the tank's parameter block and grid
+// pointers: they store into the grid between their reads of both, and read through
+// the tank table neither can be proven unaffected by those stores, so each word
+// would be loaded again (with vector loads) after every store.  A batch has no
+// ocean, so nothing indexes the arrays of the block, and the copies are scalar
+// registers.  Against a copy in LDS, whose every word goes to a vector register (16
+// tanks, us a launch): g2p 185 -> 176, normFaces 17.0 -> 15.0, divergence 19.1 -> 16.2,
+// project 16.5 -> 14.4.  (g2p kept to five waves per SIMD spills: 206.)
+#define BATCH_LOCAL \
+  DParams uP;       \
+  __builtin_memcpy(&uP, (ConstDParams*)T.P, sizeof(DParams)); \
   const DGrid G = T.G
 
 // need[0..ntiles) and binCount[0..ntiles] to zero
@@ -3164,10 +3160,10 @@ __global__ void __launch_bounds__(WG) kb_classify(BATCH_ARGS) {
 }
 __global__ void __launch_bounds__(WG) kb_norm_faces(BATCH_ARGS, const uint32_t* __restrict__ cells) {
   BATCH_TANK;
-  BATCH_STAGED;
-  norm_faces_body<false>(&sP, TC, G, cells[b.t + 1u] - cells[b.t], b.blk, b.nblk);  // a batch has no ocean
+  BATCH_LOCAL;
+  norm_faces_body<false>(&uP, TC, G, cells[b.t + 1u] - cells[b.t], b.blk, b.nblk);  // a batch has no ocean
 }
-__global__ void __launch_bounds__(WG) kb_divergence(BATCH_ARGS) { BATCH_TANK; BATCH_STAGED; divergence_body(&sP, G, b.blk, b.nblk); }
+__global__ void __launch_bounds__(WG) kb_divergence(BATCH_ARGS) { BATCH_TANK; BATCH_LOCAL; divergence_body(&uP, G, b.blk, b.nblk); }
 // one SOR iteration, pres -> pres2 (odd = 0) or back, or pass `pass` of the few-tile
 // form; every tank's range is a multiple of 8 workgroups starting at a multiple of
 // 8, so a workgroup's place within its tank keeps the XCD it runs on
@@ -3305,13 +3301,11 @@ __global__ void __launch_bounds__(COOP_WG) kb_sor_resident(const BTank* __restri
   }
 }
 
-__global__ void __launch_bounds__(WG) kb_project(BATCH_ARGS) { BATCH_TANK; BATCH_STAGED; project_body(&sP, G, b.blk, b.nblk); }
-__global__ void __launch_bounds__(WG, 4) kb_g2p_tile(BATCH_ARGS) {
+__global__ void __launch_bounds__(WG) kb_project(BATCH_ARGS) { BATCH_TANK; BATCH_LOCAL; project_body(&uP, G, b.blk, b.nblk); }
+__global__ void __launch_bounds__(WG) kb_g2p_tile(BATCH_ARGS) {
   BATCH_TANK;
-  __shared__ DParams sP;
-  batch_stage_params(sP, TP);
-  const DGrid G = T.G;  // local: the body's stores cannot touch it
-  g2p_tile_body(&sP, TC, G, 1u, T.split, b.blk, b.nblk);
+  BATCH_LOCAL;
+  g2p_tile_body<false>(&uP, TC, G, 1u, T.split, b.blk, b.nblk);
 }
 
 // ---------------------------------------------------------------------------
@@ -3513,8 +3507,10 @@ void launch_g2p(hipStream_t st, const LaunchCtx& L) {
   if (!L.n) return;
   if (L.binNext) launch_marks_clear(st, L);  // the next substep's tile marks and bin counts start here
   const uint32_t split = g2p_split(L.fullTiles);
-  uint32_t g = std::min<uint32_t>(L.ntiles * split, 8192u);
-  hipLaunchKernelGGL(k_g2p_tile, dim3(g), dim3(WG), 0, st, L.P, L.C, L.G, L.binNext ? 1u : 0u, split);
+  const uint32_t g = std::min<uint32_t>(L.ntiles * split, 8192u);
+  const uint32_t keys = L.binNext ? 1u : 0u;
+  if (L.ocean) hipLaunchKernelGGL(k_g2p_tile<true>, dim3(g), dim3(WG), 0, st, L.P, L.C, L.G, keys, split);
+  else hipLaunchKernelGGL(k_g2p_tile<false>, dim3(g), dim3(WG), 0, st, L.P, L.C, L.G, keys, split);
 }
 
 // the same with every id checked against n: *bad is set for one out of range
