@@ -257,20 +257,20 @@ int zeroSlots(Sim* s, uint32_t from, uint32_t to) {
 }
 
 void freeNb(NbScratch& S) {
-  dfree(S.deadFlag); dfree(S.deadStart); dfree(S.deadList); dfree(S.need); dfree(S.needStart); dfree(S.ent); dfree(S.entIdx);
+  dfree(S.dead); dfree(S.deadList); dfree(S.deadCount); dfree(S.need); dfree(S.needStart); dfree(S.entIdx); dfree(S.entCount);
   dfree(S.sums);
   S.ncap = S.nmax = 0;
 }
 // reseed scratch sized for the pool and the particle capacity
 int ensureNb(Sim* s) {
   uint32_t ncap = s->scap * 512u;
-  if (s->nb.deadFlag && s->nb.ncap == ncap && s->nb.nmax == s->maxn) return ST_OK;
+  if (s->nb.dead && s->nb.ncap == ncap && s->nb.nmax == s->maxn) return ST_OK;
   freeNb(s->nb);
-  size_t M = s->maxn, big = std::max<size_t>(M, ncap);
+  const size_t M = s->maxn;
   int rc;
-  if ((rc = dalloc(&s->nb.deadFlag, M)) || (rc = dalloc(&s->nb.deadStart, M + 1)) || (rc = dalloc(&s->nb.deadList, M)) ||
-      (rc = dalloc(&s->nb.need, ncap)) || (rc = dalloc(&s->nb.needStart, size_t(ncap) + 1)) || (rc = dalloc(&s->nb.ent, ncap)) ||
-      (rc = dalloc(&s->nb.entIdx, size_t(ncap) + 1)) || (rc = dalloc(&s->nb.sums, big / 1024 + 2))) {
+  if ((rc = dalloc(&s->nb.dead, M)) || (rc = dalloc(&s->nb.deadList, M)) || (rc = dalloc(&s->nb.deadCount, 1)) ||
+      (rc = dalloc(&s->nb.need, ncap)) || (rc = dalloc(&s->nb.needStart, size_t(ncap) + 1)) || (rc = dalloc(&s->nb.entIdx, ncap)) ||
+      (rc = dalloc(&s->nb.entCount, 1)) || (rc = dalloc(&s->nb.sums, nb_sum_count()))) {
     freeNb(s->nb);
     return rc;
   }

@@ -51,19 +51,20 @@ struct LaunchCtx {
   uint8_t* exMask;    // its face masks, two per pool cell (ping-pong)
 };
 
-// scratch of the narrow-band reseed: dead-slot compaction over particles and the
+// scratch of the narrow-band reseed: the dead slots' list over particles and the
 // deficit scan over active cells (ncap = pool cells)
 struct NbScratch {
-  uint32_t* deadFlag;   // N
-  uint32_t* deadStart;  // N + 1
+  uint32_t* dead;       // N: by particle id, where the particle is stored if it is dead, else ST_NONE
   uint32_t* deadList;   // N
+  uint32_t* deadCount;
   uint32_t* need;       // ncap
   uint32_t* needStart;  // ncap + 1
-  uint32_t* ent;        // ncap
-  uint32_t* entIdx;     // ncap + 1
-  uint32_t* sums;       // per-1024 block sums of the scans
+  uint32_t* entIdx;     // ncap
+  uint32_t* entCount;
+  uint64_t* sums;       // nb_sum_count() block totals of the two scans
   uint32_t ncap, nmax;
 };
+size_t nb_sum_count();
 
 // Batched tanks.  Per tank: the device copies of the step's parameter block and
 // collider records, and the tank's device pointers.

@@ -2987,74 +2987,132 @@ __device__ __forceinline__ void save_vel_body(const DGrid& G, uint32_t bid, uint
 __global__ void k_save_vel(DGrid G) {
   save_vel_body(G, blockIdx.x, gridDim.x);
 }
-// nbKill (wgsl-narrowband.js:94-102): calm particles below the band are removed
-__global__ void k_nb_kill(const DParams* __restrict__ PP, DGrid G) {
+// The reseed (wgsl-narrowband.js:94-149) in four launches, where flags, lists and
+// three scans of three launches each took fourteen of about 4.7 us: 57 -> 27 us at
+// 350 thousand particles.
+// nbKill (wgsl-narrowband.js:94-102): calm particles below the band are removed.
+// Then nbDead (wgsl-narrowband.js:107-110) as a word per particle id, where the dead
+// particle is stored: the reference's particle index is its id (its arrays are never
+// reordered by default), and the particle arrays here are in bin order, so the dead
+// slots are listed in id order.
+__global__ void k_nb_kill(const DParams* __restrict__ PP, DGrid G, uint32_t* __restrict__ dead) {
   const DParams& P = *PP;
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= P.n) return;
   float4 q = G.pos[i];
-  if (q.y < ST_DEADY) return;
-  // inside the ocean's boundary, or above the ocean surface in its inner half
-  const float lw = d_layerW(P, make_float3(q.x, q.y, q.z));
-  bool kill = lw >= 0.5f || (lw > 0.25f && q.y > d_oceanEta(P, q.x, q.z) + 0.5f * P.h);
-  float4 v = G.vel[i];
-  if (!kill && P.nb != 0u && d_calmV(P, make_float3(v.x, v.y, v.z))) {
-    int3 cc = d_particleCell(P, make_float3(q.x, q.y, q.z));
-    uint32_t sl = G.tmap[d_tileOf(P, cc.x, cc.y, cc.z)];
-    if (sl != ST_NONE && d_phiOfBits(G.ctype[d_cellIdx(P, G.tmap, cc.x, cc.y, cc.z)]) < -P.band) kill = true;
-  }
-  if (kill) {
-    G.pos[i] = make_float4(0.0f, -1.0e6f, 0.0f, 0.0f);
-    G.vel[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  }
-}
-// nbDead (wgsl-narrowband.js:107-110) as a flag per particle id, compacted in id
-// order: the reference's particle index is its id (its arrays are never
-// reordered by default), and the particle arrays here are in bin order, so the
-// k-th dead slot listed is the storage of the k-th dead id
-__global__ void k_nb_dead_flags(const DParams* __restrict__ PP, DGrid G, uint32_t* __restrict__ flag) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= PP->n) return;
-  flag[G.pid[i]] = G.pos[i].y < ST_DEADY ? 1u : 0u;
-}
-__global__ void k_nb_dead_list(const DParams* __restrict__ PP, DGrid G, const uint32_t* __restrict__ flag,
-                               const uint32_t* __restrict__ start, uint32_t* __restrict__ list) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= PP->n) return;
-  const uint32_t id = G.pid[i];
-  if (flag[id]) list[start[id]] = i;
-}
-// nbDeficit (wgsl-narrowband.js:113-130): per active cell (slotList order) how
-// many particles it is short; a scan of these gives each cell's entry number and
-// the first dead slot it fills, the order the reference's atomics would give
-// when its threads run in cell order
-__global__ void k_nb_deficit(const DParams* __restrict__ PP, DGrid G, uint32_t* __restrict__ needA, uint32_t* __restrict__ entA,
-                             uint32_t ncap) {
-  const DParams& P = *PP;
-  uint32_t tot = G.ctl[4] * 512u;
-  for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < ncap; t += gridDim.x * blockDim.x) {
-    uint32_t need = 0u;
-    if (t < tot) {
-      uint32_t s = G.slotList[t >> 9], local = t & 511u, c = s * 512u + local;
-      int3 p = d_slotCoord(P, G.slotTile, s, local);
-      uint32_t ct = G.ctype[c];
-      float ph = d_phiOfBits(ct);
-      bool ok = d_inDom(P, p) && ((ct >> 8) & 0xffu) == 0u;
-      if (ok) {
-        const float3 cx = d_cellCenter(P, p.x, p.y, p.z);
-        const float lw = d_layerW(P, cx);
-        if (lw > 0.25f && lw < 0.5f)  // the inner half of the ocean's boundary is always full below the surface
-          ok = !(cx.y > d_oceanEta(P, cx.x, cx.z) - 0.25f * P.h || ph < -P.band);
-        else
-          ok = (ct & 0xffu) == 1u && !(ph > -1.0f) && !(ph < -P.band) && d_calmV(P, d_velGVec(P, G, cx));
-      }
-      if (ok) {
-        uint32_t n = uint32_t(max(G.cnt[c], 0));
-        if (!(float(n) >= 0.55f * P.rest)) need = min(st_f2u_sat(rintf(0.85f * P.rest)) - n, 64u);
-      }
+  bool kill = q.y < ST_DEADY;
+  if (!kill) {
+    // inside the ocean's boundary, or above the ocean surface in its inner half
+    const float lw = d_layerW(P, make_float3(q.x, q.y, q.z));
+    kill = lw >= 0.5f || (lw > 0.25f && q.y > d_oceanEta(P, q.x, q.z) + 0.5f * P.h);
+    float4 v = G.vel[i];
+    if (!kill && P.nb != 0u && d_calmV(P, make_float3(v.x, v.y, v.z))) {
+      int3 cc = d_particleCell(P, make_float3(q.x, q.y, q.z));
+      uint32_t sl = G.tmap[d_tileOf(P, cc.x, cc.y, cc.z)];
+      if (sl != ST_NONE && d_phiOfBits(G.ctype[d_cellIdx(P, G.tmap, cc.x, cc.y, cc.z)]) < -P.band) kill = true;
     }
-    needA[t] = need;
-    entA[t] = need ? 1u : 0u;
+    if (kill) {
+      G.pos[i] = make_float4(0.0f, -1.0e6f, 0.0f, 0.0f);
+      G.vel[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+  }
+  dead[G.pid[i]] = kill ? i : ST_NONE;
+}
+// nbDeficit (wgsl-narrowband.js:113-130): how many particles cell c is short
+__device__ __forceinline__ uint32_t nb_deficit(const DParams& P, const DGrid& G, uint32_t s, uint32_t local) {
+  const uint32_t c = s * 512u + local, ct = G.ctype[c];
+  const int3 p = d_slotCoord(P, G.slotTile, s, local);
+  const float ph = d_phiOfBits(ct);
+  bool ok = d_inDom(P, p) && ((ct >> 8) & 0xffu) == 0u;
+  if (ok) {
+    const float3 cx = d_cellCenter(P, p.x, p.y, p.z);
+    const float lw = d_layerW(P, cx);
+    if (lw > 0.25f && lw < 0.5f)  // the inner half of the ocean's boundary is always full below the surface
+      ok = !(cx.y > d_oceanEta(P, cx.x, cx.z) - 0.25f * P.h || ph < -P.band);
+    else
+      ok = (ct & 0xffu) == 1u && !(ph > -1.0f) && !(ph < -P.band) && d_calmV(P, d_velGVec(P, G, cx));
+  }
+  if (!ok) return 0u;
+  const uint32_t n = uint32_t(max(G.cnt[c], 0));
+  return float(n) >= 0.55f * P.rest ? 0u : min(st_f2u_sat(rintf(0.85f * P.rest)) - n, 64u);
+}
+// Two scans, in two launches: nb_count leaves each block's total (and the cells'
+// deficits), nb_place adds up the totals before its block and numbers its items.  The
+// first `nd` workgroups take the dead slots, listed in id order; the others the cells
+// in use (slotList order): each cell's deficit, its entry number and the first dead
+// slot it fills, the order the reference's atomics would give when its threads run
+// in cell order.  At most NB_BLOCKS blocks of each, so that the totals stay few.  (One
+// launch, with totals published as in tiles_scan, took 41 us or more: its blocks
+// queue at the ticket or, when few, walk too many items one after another.)
+#define NB_BLOCKS 2048u
+__device__ __forceinline__ uint32_t nb_block(uint32_t items, uint32_t nb, uint32_t unit) { return ((items + nb * unit - 1u) / (nb * unit)) * unit; }
+// the sum of sums[0..b) (every thread)
+__device__ __forceinline__ uint64_t nb_before(const uint64_t* __restrict__ sums, uint32_t b) {
+  uint64_t v = 0, tot;
+  for (uint32_t q = threadIdx.x; q < b; q += WG) v += sums[q];
+  (void)wg_scan_u64(v, &tot);
+  return tot;
+}
+__global__ void __launch_bounds__(WG) k_nb_count(const DParams* __restrict__ PP, DGrid G, NbScratch S, uint32_t nd) {
+  const DParams& P = *PP;
+  uint64_t mine = 0, tot;
+  if (blockIdx.x < nd) {
+    const uint32_t per = nb_block(P.n, nd, TB), beg = blockIdx.x * per, end = min(P.n, beg + per);
+    for (uint32_t i = beg + threadIdx.x; i < end; i += WG) mine += S.dead[i] != ST_NONE ? 1u : 0u;
+    (void)wg_scan_u64(mine, &tot);
+    if (threadIdx.x == 0u) S.sums[blockIdx.x] = tot;
+    return;
+  }
+  const uint32_t b = blockIdx.x - nd, cells = G.ctl[4] * 512u, per = nb_block(cells, gridDim.x - nd, WG), beg = b * per;
+  if (beg >= cells) return;
+  const uint32_t end = min(cells, beg + per);
+  for (uint32_t t = beg + threadIdx.x; t < end; t += WG) {
+    const uint32_t need = nb_deficit(P, G, G.slotList[t >> 9], t & 511u);
+    S.need[t] = need;
+    mine += uint64_t(need) << 32 | (need ? 1u : 0u);
+  }
+  (void)wg_scan_u64(mine, &tot);
+  if (threadIdx.x == 0u) S.sums[NB_BLOCKS + b] = tot;  // needs << 32 | entries
+}
+__global__ void __launch_bounds__(WG) k_nb_place(const DParams* __restrict__ PP, DGrid G, NbScratch S, uint32_t nd) {
+  const uint32_t n = PP->n;
+  uint64_t tot;
+  if (blockIdx.x < nd) {
+    const uint32_t per = nb_block(n, nd, TB), beg = blockIdx.x * per, end = min(n, beg + per);
+    if (beg >= end) return;
+    uint32_t at = uint32_t(nb_before(S.sums, blockIdx.x));
+    for (uint32_t i0 = beg; i0 < end; i0 += TB) {
+      const uint32_t i = i0 + threadIdx.x * 4u;
+      uint32_t slot[4], cnt = 0;
+      for (uint32_t q = 0; q < 4u; q++) {
+        slot[q] = i + q < end ? S.dead[i + q] : ST_NONE;
+        cnt += slot[q] != ST_NONE ? 1u : 0u;
+      }
+      uint32_t k = at + uint32_t(wg_scan_u64(cnt, &tot));
+      for (uint32_t q = 0; q < 4u; q++)
+        if (slot[q] != ST_NONE) S.deadList[k++] = slot[q];
+      at += uint32_t(tot);
+    }
+    if (end == n && threadIdx.x == 0u) *S.deadCount = at;
+    return;
+  }
+  const uint32_t b = blockIdx.x - nd, cells = G.ctl[4] * 512u, per = nb_block(cells, gridDim.x - nd, WG), beg = b * per;
+  if (b == 0u && cells == 0u && threadIdx.x == 0u) *S.entCount = 0u;
+  if (beg >= cells) return;
+  const uint32_t end = min(cells, beg + per);
+  const uint64_t before = nb_before(S.sums + NB_BLOCKS, b);
+  uint32_t need = uint32_t(before >> 32), ent = uint32_t(before);
+  for (uint32_t t = beg + threadIdx.x; t < end; t += WG) {  // blocks and cells are whole workgroups
+    const uint32_t mine = S.need[t];
+    const uint64_t at = wg_scan_u64(uint64_t(mine) << 32 | (mine ? 1u : 0u), &tot);
+    S.needStart[t] = need + uint32_t(at >> 32);
+    S.entIdx[t] = ent + uint32_t(at);
+    need += uint32_t(tot >> 32);
+    ent += uint32_t(tot);
+  }
+  if (end == cells && threadIdx.x == 0u) {
+    S.needStart[cells] = need;
+    *S.entCount = ent;
   }
 }
 __device__ __forceinline__ float d_hash1(uint32_t n0) {
@@ -3067,12 +3125,14 @@ __device__ __forceinline__ float d_hash1(uint32_t n0) {
 // one (each finds its cell by a search in the cells' starts): a short cell wants up
 // to 64, and one thread after another making a cell's left the others idle (217 ->
 // 27 us in the ocean, whose boundary cells are refilled each substep).
-__global__ void __launch_bounds__(WG) k_nb_spawn(const DParams* __restrict__ PP, DGrid G, const uint32_t* __restrict__ needA,
-                           const uint32_t* __restrict__ needStart, const uint32_t* __restrict__ entIdx,
-                           const uint32_t* __restrict__ deadList, const uint32_t* __restrict__ deadCount, uint32_t ncap) {
+__global__ void __launch_bounds__(WG) k_nb_spawn(const DParams* __restrict__ PP, DGrid G, NbScratch S) {
   const DParams& P = *PP;
   __shared__ uint32_t sStart[WG];
-  const uint32_t tot = G.ctl[4] * 512u, ndead = *deadCount, avail = min(ndead, P.lcap), nent = entIdx[ncap];
+  const uint32_t* __restrict__ needA = S.need;
+  const uint32_t* __restrict__ needStart = S.needStart;
+  const uint32_t* __restrict__ entIdx = S.entIdx;
+  const uint32_t* __restrict__ deadList = S.deadList;
+  const uint32_t tot = G.ctl[4] * 512u, ndead = *S.deadCount, avail = min(ndead, P.lcap), nent = *S.entCount;
   const uint32_t maxe = P.lcap / 2u;
   for (uint32_t t0 = blockIdx.x * WG; t0 < tot; t0 += gridDim.x * WG) {  // tot is whole workgroups
     const uint32_t mine = t0 + threadIdx.x, need0 = needA[mine];
@@ -3466,19 +3526,15 @@ void launch_narrowband(hipStream_t st, const LaunchCtx& L) {
   hipLaunchKernelGGL(k_nb_jac, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G, 1u);
 }
 
+size_t nb_sum_count() { return 2u * NB_BLOCKS; }
+
 void launch_reseed(hipStream_t st, const LaunchCtx& L, const NbScratch& S) {
   if (!L.n) return;
-  uint32_t gp = gridFor(L.n, WG);
-  hipLaunchKernelGGL(k_nb_kill, dim3(gp), dim3(WG), 0, st, L.P, L.G);
-  hipLaunchKernelGGL(k_nb_dead_flags, dim3(gp), dim3(WG), 0, st, L.P, L.G, S.deadFlag);
-  launch_scan(st, S.deadFlag, S.deadStart, L.n, S.sums, nullptr);
-  hipLaunchKernelGGL(k_nb_dead_list, dim3(gp), dim3(WG), 0, st, L.P, L.G, (const uint32_t*)S.deadFlag, (const uint32_t*)S.deadStart,
-                     S.deadList);
-  hipLaunchKernelGGL(k_nb_deficit, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G, S.need, S.ent, S.ncap);
-  launch_scan(st, S.need, S.needStart, S.ncap, S.sums, nullptr);
-  launch_scan(st, S.ent, S.entIdx, S.ncap, S.sums, nullptr);
-  hipLaunchKernelGGL(k_nb_spawn, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G, (const uint32_t*)S.need, (const uint32_t*)S.needStart,
-                     (const uint32_t*)S.entIdx, (const uint32_t*)S.deadList, (const uint32_t*)(S.deadStart + L.n), S.ncap);
+  const uint32_t nd = std::min(gridFor(L.n, TB), NB_BLOCKS), nc = std::min(gridFor(S.ncap, WG), NB_BLOCKS);
+  hipLaunchKernelGGL(k_nb_kill, dim3(gridFor(L.n, WG)), dim3(WG), 0, st, L.P, L.G, S.dead);
+  hipLaunchKernelGGL(k_nb_count, dim3(nd + nc), dim3(WG), 0, st, L.P, L.G, S, nd);
+  hipLaunchKernelGGL(k_nb_place, dim3(nd + nc), dim3(WG), 0, st, L.P, L.G, S, nd);
+  hipLaunchKernelGGL(k_nb_spawn, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G, S);
 }
 
 void launch_norm_faces(hipStream_t st, const LaunchCtx& L) {
