@@ -2912,54 +2912,107 @@ __global__ void __launch_bounds__(WG) k_nb_phi_init(const DParams* __restrict__ 
       for (uint32_t ax = 0; ax < 3; ax++) G.velG[c * 3 + ax] = v[ax];
   }
 }
-// nbPhi (wgsl-narrowband.js:39-49): depth carried by the kept grid velocity
+// nbPhi (wgsl-narrowband.js:39-49): depth carried by the kept grid velocity, into pres2
+// (the pressure solve's scratch) for k_nb_jac, whose tiles read each other's
 __device__ __forceinline__ void nb_phi_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid) {
   const DParams& P = *PP;
   FOR_ACTIVE(G) {
     uint32_t s = G.slotList[t >> 9], local = t & 511u, c = s * 512u + local;
     int3 p = d_slotCoord(P, G.slotTile, s, local);
-    if (!d_inDom(P, p)) { G.rhs[c] = 8.0f; continue; }
-    if (((G.ctype[c] >> 8) & 0xffu) != 0u) { G.rhs[c] = 0.5f; continue; }
+    if (!d_inDom(P, p)) { G.pres2[c] = 8.0f; continue; }
+    if (((G.ctype[c] >> 8) & 0xffu) != 0u) { G.pres2[c] = 0.5f; continue; }
     float3 x = d_cellCenter(P, p.x, p.y, p.z);
     float phA = d_phiSample(P, G, f3sub(x, f3mul(d_velGVec(P, G, x), P.dt)));
     bool inside = G.cnt[c] > 0 || phA < -1.0f;
     if (P.ocean != 0u && d_layerW(P, x) >= 0.5f) inside = x.y < d_oceanEta(P, x.x, x.z);  // the ocean surface decides
-    G.rhs[c] = inside ? st_clampf(phA, -7.9f, -0.5f) : st_clampf(phA, 0.5f, 7.9f);
+    G.pres2[c] = inside ? st_clampf(phA, -7.9f, -0.5f) : st_clampf(phA, 0.5f, 7.9f);
   }
 }
 __global__ void k_nb_phi(const DParams* __restrict__ PP, DGrid G) {
   nb_phi_body(PP, G, blockIdx.x, gridDim.x);
 }
-// jacNb, nbJacA (fromRhs: phi <- from rhs) and nbJacB (rhs <- from phi) (wgsl-narrowband.js:51-68)
-__device__ __forceinline__ void nb_jac_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t fromRhs, uint32_t bid,
-                                            uint32_t nbid) {
-  const DParams& P = *PP;
-  FOR_ACTIVE(G) {
-    uint32_t s = G.slotList[t >> 9], local = t & 511u, c = s * 512u + local;
-    int3 p = d_slotCoord(P, G.slotTile, s, local);
-    float cur = fromRhs ? G.rhs[c] : d_phiOfBits(G.ctype[c]);
-    float out;
-    if (!d_inDom(P, p)) out = 8.0f;
-    else if (cur >= 0.0f) out = cur;
-    else {
-      float m = -8.0f;
-      for (uint32_t q = 0; q < 6; q++) {
-        int3 n = p;
-        if (q == 0) n.x -= 1; else if (q == 1) n.x += 1; else if (q == 2) n.y -= 1; else if (q == 3) n.y += 1; else if (q == 4) n.z -= 1; else n.z += 1;
-        if (!d_inDom(P, n)) continue;
-        uint32_t cq = d_cellIdx(P, G.tmap, n.x, n.y, n.z);
-        uint32_t ct = G.ctype[cq];
-        if (((ct >> 8) & 0xffu) != 0u) continue;
-        m = fmaxf(m, fromRhs ? G.rhs[cq] : d_phiOfBits(ct));
-      }
-      out = st_clampf(m - 1.0f, -7.9f, -0.5f);
-    }
-    if (fromRhs) G.ctype[c] = d_phiPutBits(G.ctype[c], out);
-    else G.rhs[c] = out;
-  }
+// jacNb, nbJacA (phi <- from rhs), nbJacB (rhs <- from phi) and nbJacA again
+// (wgsl-narrowband.js:51-68) in one launch: a workgroup per tile on the tile and three
+// cells around it in LDS, of which each sweep needs one less.  As launches of their
+// own the sweeps read seven cells per cell behind tile map lookups, and wrote them
+// back, each time (three launches 30 -> 19 us at 96^3).  Depths are at least -7.9, so
+// -8 stands for the cells a sweep passes over (outside the box, collider): it is where
+// the maximum starts.  phi has the 16 bits of its place in ctype between sweeps.  Cells
+// of tiles without storage keep the values of slot 0.
+#define JW 14
+#define JW3 (JW * JW * JW)
+#define JB 12
+#define JAC_SKIP (-8.0f)
+__device__ __forceinline__ float jac_new(float cur, const float* w, int sx, int sy, int sz) {
+  if (cur >= 0.0f) return cur;
+  float m = JAC_SKIP;
+  m = fmaxf(m, w[-sx]);
+  m = fmaxf(m, w[sx]);
+  m = fmaxf(m, w[-sy]);
+  m = fmaxf(m, w[sy]);
+  m = fmaxf(m, w[-sz]);
+  m = fmaxf(m, w[sz]);
+  return st_clampf(m - 1.0f, -7.9f, -0.5f);
 }
-__global__ void k_nb_jac(const DParams* __restrict__ PP, DGrid G, uint32_t fromRhs) {
-  nb_jac_body(PP, G, fromRhs, blockIdx.x, gridDim.x);
+__device__ __forceinline__ float jac_phi(float v) { return d_phiOfBits(d_phiPutBits(0u, v)); }
+__global__ void __launch_bounds__(512) k_nb_jac(const DParams* __restrict__ PP, DGrid G) {
+  const DParams& P = *PP;
+  __shared__ float sA[JW3], sB[JB * JB * JB];  // rhs, phi
+  __shared__ uint32_t sSlot[27];
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t b = blockIdx.x, nact = G.ctl[4]; b < nact; b += gridDim.x) {
+    const TileAt T = tile_at(G, b);
+    if (tid < 27u) {
+      const uint32_t ns = G.nbrL[b * 27u + tid];
+      sSlot[tid] = sor_missing(ns) ? 0u : ns;
+    }
+    __syncthreads();
+    auto slotOf = [&](uint32_t x, uint32_t y, uint32_t z) { return sSlot[((x + 5u) >> 3) + 3u * ((y + 5u) >> 3) + 9u * ((z + 5u) >> 3)]; };
+    for (uint32_t q = tid; q < JW3; q += 512u) {
+      const uint32_t x = q % JW, y = (q / JW) % JW, z = q / (JW * JW);
+      float v = JAC_SKIP, ph = JAC_SKIP;
+      if (d_inDom(P, make_int3(T.x - 3 + int32_t(x), T.y - 3 + int32_t(y), T.z - 3 + int32_t(z)))) {
+        const uint32_t s = slotOf(x, y, z), c = s * 512u + ((x + 5u) & 7u) + 8u * ((y + 5u) & 7u) + 64u * ((z + 5u) & 7u);
+        const uint32_t ct = G.ctype[c];
+        if (((ct >> 8) & 0xffu) == 0u) {
+          v = s ? G.pres2[c] : G.rhs[c];
+          ph = d_phiOfBits(ct);
+        }
+        if (s == 0u && x - 1u < JB && y - 1u < JB && z - 1u < JB) sB[(x - 1u) + JB * ((y - 1u) + JB * (z - 1u))] = ph;
+      }
+      sA[q] = v;
+    }
+    const uint32_t lx = tid & 7u, ly = (tid >> 3) & 7u, lz = tid >> 6, c = T.s * 512u + tid, ct = G.ctype[c];
+    const bool in = d_inDom(P, make_int3(T.x + int32_t(lx), T.y + int32_t(ly), T.z + int32_t(lz)));
+    const bool col = ((ct >> 8) & 0xffu) != 0u;
+    const float cur = G.pres2[c];
+    __syncthreads();
+    for (uint32_t q = tid; q < JB * JB * JB; q += 512u) {
+      const uint32_t x = q % JB, y = (q / JB) % JB, z = q / (JB * JB), w = (x + 1u) + JW * ((y + 1u) + JW * (z + 1u));
+      if (sA[w] == JAC_SKIP) sB[q] = JAC_SKIP;
+      else if (slotOf(x + 1u, y + 1u, z + 1u)) sB[q] = jac_phi(jac_new(sA[w], sA + w, 1, JW, JW * JW));
+    }
+    __syncthreads();
+    for (uint32_t q = tid; q < 1000u; q += 512u) {
+      const uint32_t x = q % 10u, y = (q / 10u) % 10u, z = q / 100u, w = (x + 1u) + JB * ((y + 1u) + JB * (z + 1u));
+      if (sB[w] != JAC_SKIP && slotOf(x + 2u, y + 2u, z + 2u)) sA[(x + 2u) + JW * ((y + 2u) + JW * (z + 2u))] = jac_new(sB[w], sB + w, 1, JB, JB * JB);
+    }
+    __syncthreads();
+    const uint32_t w = (lx + 3u) + JW * ((ly + 3u) + JW * (lz + 3u));
+    float rhs, phi;
+    if (!in) {
+      rhs = phi = 8.0f;
+    } else if (col) {  // a collider cell's own depth is positive: the sweeps keep it
+      rhs = jac_phi(cur);
+      phi = rhs;
+    } else {
+      rhs = sA[w];
+      phi = jac_new(rhs, sA + w, 1, JW, JW * JW);
+    }
+    G.rhs[c] = rhs;
+    G.ctype[c] = d_phiPutBits(ct, phi);
+    __syncthreads();
+  }
 }
 // nbVel (wgsl-narrowband.js:71-85): water faces no particle reached take the kept
 // grid velocity, carried along.  A workgroup takes a tile, a cell a thread, and where
@@ -3559,9 +3612,7 @@ void launch_classify(hipStream_t st, const LaunchCtx& L, bool solid, bool counts
 
 void launch_narrowband(hipStream_t st, const LaunchCtx& L) {
   hipLaunchKernelGGL(k_nb_phi, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G);
-  hipLaunchKernelGGL(k_nb_jac, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G, 1u);
-  hipLaunchKernelGGL(k_nb_jac, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G, 0u);
-  hipLaunchKernelGGL(k_nb_jac, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G, 1u);
+  hipLaunchKernelGGL(k_nb_jac, dim3(L.tileGrid), dim3(512), 0, st, L.P, L.G);
 }
 
 size_t nb_sum_count() { return 2u * NB_BLOCKS; }
