@@ -687,7 +687,7 @@ class AdjointC:
 
     def set_sor_path(self, one_launch):
         """True: the transposed solve in one cooperative launch where the
-        device allows it; False (the default): one launch per sweep."""
+        device allows it; False (the default): one launch per iteration."""
         self._call("set_sor_path", 1 if one_launch else 0)
 
     def sor_path(self):

@@ -73,6 +73,6 @@ uint32_t adj_sor_coop_grid(uint32_t cus);
 // state after it), writes G.gPos2/gVel2 (gradient of the state before it) and the
 // pressure carry for the substep before.  With coopGrid > 0 the transposed
 // solve runs as one cooperative launch of that many workgroups (the same
-// arithmetic as one launch per sweep, which runs when coopGrid is 0 or the
+// arithmetic as one launch per iteration, which runs when coopGrid is 0 or the
 // cooperative launch is refused); returns whether the one launch ran.
 bool launch_adjoint_step(hipStream_t st, const AdjTape& T, const AdjGrad& G, uint32_t scap, uint32_t ntiles, uint32_t coopGrid);

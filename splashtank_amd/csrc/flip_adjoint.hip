@@ -434,16 +434,112 @@ __device__ __forceinline__ void adj_sor_body(const AdjTape& T, const AdjGrad& G,
     }
   }
 }
-__global__ void __launch_bounds__(AWG) k_adj_sor(AdjTape T, AdjGrad G, const float* __restrict__ gin, float* __restrict__ gout,
-                                                 uint32_t colour) {
-  adj_sor_body(T, G, gin, gout, colour, T.P->omega);
+
+// Both colours of one iteration in one launch: a workgroup takes a tile and two cells
+// around it in LDS, where the red cells up to one cell around are swept too (a black
+// cell gathers from them), so that no tile waits for another's.  Bound by the launch
+// and the window's loads, which 512 threads keep in flight together.  An iteration of
+// two launches, its gathers through sorNb, 9.7 us at 64^3 (123 full tiles), one for
+// both 5.1 (256 threads: 6.8); a reversed substep of 40 iterations 670 -> 515 us at
+// 32^3, 769 -> 594 at 64^3, 3572 -> 2822 at 128^3.
+// The same values in the same order as two adj_sor_body: a cell's part in its
+// neighbours' sums is one product, rounded once, and -0 (which changes no sum) where
+// it has none.
+#define ASW 12
+#define ASW3 (ASW * ASW * ASW)
+#define ASW_WG 512
+// the slots of the 27 tiles around each tile in use, in sorNb
+__global__ void __launch_bounds__(AWG) k_adj_sor_tiles(AdjTape T, AdjGrad G) {
+  const DParams& P = *T.P;
+  const uint32_t tot = T.ctl[4] * 27u;
+  for (uint32_t t = blockIdx.x * AWG + threadIdx.x; t < tot; t += gridDim.x * AWG) {
+    const uint32_t tile = T.slotTile[T.slotList[t / 27u]], q = t % 27u;
+    const int32_t i = int32_t(tile % P.tx) + int32_t(q % 3u) - 1, j = int32_t((tile / P.tx) % P.ty) + int32_t((q / 3u) % 3u) - 1,
+                  k = int32_t(tile / (P.tx * P.ty)) + int32_t(q / 9u) - 1;
+    const bool in = i >= 0 && j >= 0 && k >= 0 && i < int32_t(P.tx) && j < int32_t(P.ty) && k < int32_t(P.tz);
+    G.sorNb[t] = in ? T.tmap[uint32_t(i) + P.tx * (uint32_t(j) + P.ty * uint32_t(k))] : ST_NONE;
+  }
+}
+__global__ void __launch_bounds__(ASW_WG) k_adj_sor_pass(AdjTape T, AdjGrad G, const float* __restrict__ gin, float* __restrict__ gout) {
+  __shared__ float sV[ASW3], sW[8];  // red: gradient, then part; black: part
+  __shared__ uint8_t sSten[ASW3];
+  __shared__ uint32_t sSlot[27];
+  const uint32_t tid = threadIdx.x;
+  const float w = T.P->omega;
+  if (tid < 8u) sW[tid] = w / float(tid);
+  auto around = [&](uint32_t at, float g) {
+    g += sV[at - 1u];
+    g += sV[at + 1u];
+    g += sV[at - ASW];
+    g += sV[at + ASW];
+    g += sV[at - ASW * ASW];
+    g += sV[at + ASW * ASW];
+    return g;
+  };
+  for (uint32_t b = blockIdx.x, nact = T.ctl[4]; b < nact; b += gridDim.x) {
+    if (tid < 27u) sSlot[tid] = G.sorNb[b * 27u + tid];
+    __syncthreads();
+    const uint32_t s = sSlot[13];
+    for (uint32_t q = tid; q < ASW3; q += ASW_WG) {
+      const uint32_t x = q % ASW + 6u, y = (q / ASW) % ASW + 6u, z = q / (ASW * ASW) + 6u;
+      const uint32_t ns = sSlot[(x >> 3) + 3u * (y >> 3) + 9u * (z >> 3)];
+      float v = -0.0f;
+      uint32_t st = 0u;
+      if (ns != ST_NONE) {
+        const uint32_t c = ns * 512u + (x & 7u) + 8u * (y & 7u) + 64u * (z & 7u);
+        st = T.sten[c];
+        const float g = gin[c];
+        if (((x + y + z) & 1u) == 0u) v = g;
+        else if ((st & 0x80u) && (st & 7u)) v = sW[st & 7u] * g;
+      }
+      sV[q] = v;
+      sSten[q] = uint8_t(st);
+    }
+    __syncthreads();
+    // the red cells of the tile and across its faces: gathered, then swept
+    for (uint32_t q = tid; q < 500u; q += ASW_WG) {
+      const uint32_t y = (q / 5u) % 10u + 1u, z = q / 50u + 1u, x = 1u + 2u * (q % 5u) + ((1u + y + z) & 1u);
+      const uint32_t out = uint32_t(x - 2u >= 8u) + uint32_t(y - 2u >= 8u) + uint32_t(z - 2u >= 8u);
+      if (out > 1u) continue;
+      const uint32_t at = x + ASW * (y + ASW * z), st = sSten[at], n = st & 7u, c = s * 512u + (x - 2u) + 8u * (y - 2u) + 64u * (z - 2u);
+      float part = -0.0f, next = 0.0f;
+      if (st & 0x80u) {
+        const float g = around(at, sV[at]);
+        if (n) {
+          part = sW[n] * g;
+          next = (1.f - w) * g;
+        }
+      }
+      sV[at] = part;
+      if (out == 0u) {
+        if ((st & 0x80u) && n) G.gRhs[c] += part;
+        gout[c] = next;
+      }
+    }
+    __syncthreads();
+    // the tile's black cells: swept, then gathered
+    if (tid < 256u) {
+      const uint32_t y = ((tid >> 2) & 7u) + 2u, z = (tid >> 5) + 2u, x = 2u + 2u * (tid & 3u) + ((1u + y + z) & 1u);
+      const uint32_t at = x + ASW * (y + ASW * z), st = sSten[at], c = s * 512u + (x - 2u) + 8u * (y - 2u) + 64u * (z - 2u);
+      float g = 0.0f;
+      if (st & 0x80u) {
+        if (st & 7u) {
+          G.gRhs[c] += sV[at];
+          g = (1.f - w) * gin[c];
+        }
+        g = around(at, g);
+      }
+      gout[c] = g;
+    }
+    __syncthreads();
+  }
 }
 
 // The whole transposed solve in one cooperative launch: the sweeps of
-// k_adj_sor in the same order (per iteration black then red, ping-pong from
+// k_adj_sor_pass in the same order (per iteration black then red, ping-pong from
 // gPres), a grid barrier between consecutive sweeps (the gathers of one read
 // what the last wrote in other workgroups).  2 iters sweeps leave the result in
-// gPres, as the launches per sweep do.  A barrier time-out (counted in
+// gPres.  A barrier time-out (counted in
 // bar[ADJ_BAR_FAILS]) ends the solve early; the host reports it.
 __global__ void __launch_bounds__(AWG) k_adj_sor_all(AdjTape T, AdjGrad G) {
   __shared__ uint32_t sFail;
@@ -598,21 +694,24 @@ bool launch_adjoint_step(hipStream_t st, const AdjTape& T, const AdjGrad& G, uin
   // the solve reversed: per iteration, black then red, ping-pong gPres <-> gPres2
   float* a = G.gPres;
   float* b = G.gPres2;
-  hipLaunchKernelGGL(k_adj_sor_prep, dim3(cg), dim3(AWG), 0, st, T, G);
   bool one = false;
   if (coopGrid && T.iters) {
+    hipLaunchKernelGGL(k_adj_sor_prep, dim3(cg), dim3(AWG), 0, st, T, G);
     hipLaunchKernelGGL(k_adj_clear_bar, dim3(1), dim3(AWG), 0, st, G.bar);
     AdjTape t = T;
     AdjGrad g = G;
     void* args[] = {(void*)&t, (void*)&g};
     one = hipLaunchCooperativeKernel((const void*)k_adj_sor_all, dim3(std::min(coopGrid, ADJ_SOR_MAX_WG)), dim3(AWG), args, 0, st) == hipSuccess;
-    if (!one) (void)hipGetLastError();  // the launches per sweep below do the solve
+    if (!one) (void)hipGetLastError();  // the launches per iteration below do the solve
   }
-  for (uint32_t it = 0; !one && it < T.iters; it++)
-    for (int colour = 1; colour >= 0; colour--) {
-      hipLaunchKernelGGL(k_adj_sor, dim3(cg), dim3(AWG), 0, st, T, G, (const float*)a, b, uint32_t(colour));
+  if (!one) {
+    const uint32_t tg = std::max<uint32_t>(1u, std::min<uint32_t>(scap, 8192u));
+    hipLaunchKernelGGL(k_adj_sor_tiles, dim3(std::min(grid_for(size_t(scap) * 27u), 1024u)), dim3(AWG), 0, st, T, G);
+    for (uint32_t it = 0; it < T.iters; it++) {
+      hipLaunchKernelGGL(k_adj_sor_pass, dim3(tg), dim3(ASW_WG), 0, st, T, G, (const float*)a, b);
       std::swap(a, b);
     }
+  }
   // a holds the gradient of the warm start: the carry for the substep before
   hipLaunchKernelGGL(k_adj_zero, dim3(grid_for(size_t(ntiles) * 512u)), dim3(AWG), 0, st, G.carry, size_t(ntiles) * 512u);
   hipLaunchKernelGGL(k_adj_carry, dim3(cg), dim3(AWG), 0, st, T, G, (const float*)a);

@@ -842,7 +842,7 @@ struct Adj {
   std::vector<const float*> sdfAt;
   std::vector<uint32_t> ncols;    // per tape: colliders of its substep
   uint32_t lastCols = 0;          // colliders of the substep reversed last
-  uint32_t coopGrid = 0;          // workgroups of the one-launch transposed solve (0: one launch per sweep)
+  uint32_t coopGrid = 0;          // workgroups of the one-launch transposed solve (0: one launch per iteration)
   bool oneLaunch = false;         // st_adj_set_sor_path: use the one launch when coopGrid > 0
   bool lastOne = false;           // the last reversed substep's solve ran as one launch
   AdjGrad G{};
@@ -2170,7 +2170,7 @@ int st_adj_create(void* p, uint32_t max_steps, void** out) {
 
 // After a synchronisation: a time-out of the one-launch solve's grid barrier
 // (a workgroup that never arrived) left gradients that are not valid.  It is
-// reported once, and the context falls back to one launch per sweep.
+// reported once, and the context falls back to one launch per iteration.
 static int adjBarrierCheck(Adj* a, const char* who) {
   uint32_t fails = 0;
   HIPCHK(hipMemcpy(&fails, a->G.bar + ADJ_BAR_FAILS, sizeof(uint32_t), hipMemcpyDeviceToHost));
@@ -2178,7 +2178,7 @@ static int adjBarrierCheck(Adj* a, const char* who) {
   HIPCHK(hipMemset(a->G.bar + ADJ_BAR_FAILS, 0, sizeof(uint32_t)));
   a->coopGrid = 0;
   return fail(ST_ERR_HIP, std::string(who) + ": a grid barrier of the one-launch adjoint solve timed out " + std::to_string(fails) +
-                              " times; the gradients are not valid (later solves use one launch per sweep)");
+                              " times; the gradients are not valid (later solves use one launch per iteration)");
 }
 
 int st_adj_destroy(void* adj) {
