@@ -320,7 +320,7 @@ def summarize_counters(src: str, workload: str, command: str, calib_mb: int):
         # ones are the parameter uploads)
         cg = max([int(r["Grid_Size"]) for r in rows if "copyBuffer" in r["Kernel_Name"]] or [0])
         for r in rows:
-            k = r["Kernel_Name"].split("(")[0]
+            k = r["Kernel_Name"].split("(")[0].removeprefix("void ").split("<")[0]  # without template arguments
             if "copyBuffer" in k:
                 if int(r["Grid_Size"]) == cg:
                     calib_rows.setdefault(r["Counter_Name"], []).append(float(r["Counter_Value"]))
@@ -516,8 +516,7 @@ def main():
         # its time per launch (HIP events around its stage on the sim's stream):
         #  - pressure: 16 B per fluid cell per red-black iteration (rhs, type,
         #    pressure read and write); the cooperative solve runs all iterations
-        #    in one launch (k_sor_resident; the stage also holds three small list
-        #    kernels of a few us), the per-iteration path one per iteration;
+        #    in one launch (k_sor_resident), the per-iteration path one per iteration;
         #  - g2p: 64 B per particle (state read and written) and 28 B per active
         #    cell (new and old face velocities, count);
         #  - p2g: 32 B per particle (state read) and 56 B per active cell (three

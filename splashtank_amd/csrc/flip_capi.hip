@@ -122,6 +122,7 @@ struct Sim {
   uint32_t sorResident = 2048;  // SOR workgroups resident at once on this device
   uint32_t coopGrid = 0;        // resident-SOR workgroups (0: not available)
   uint32_t sorTiles = 0;        // resident workgroups of the one-per-tile solve (0: not available)
+  uint32_t sorSafe = 0;         // as many fit whatever other streams run
   uint32_t sorSeq = 0;          // pressure solves so far
   uint32_t sorTag = 1;          // tag of the next substep's first halo exchange (0 is never used)
   uint32_t sorMode = 0;         // this step's pressure path (st_params.sor_mode, a tuned choice for 3)
@@ -183,6 +184,7 @@ struct Sim {
     L.coopGrid = sorMode == 1u ? 0u : coopGrid;
     L.sorStream = sorMode == 2u;
     L.sorTiles = sorTiles;
+    L.sorSafe = sorSafe;
     L.sorTag = 0u;
     L.sorSeq = sorSeq;
     L.full = !onlyTiles;
@@ -914,6 +916,7 @@ int st_create(const st_opts* o, void** out) {
     s->sorResident = sor_resident_grid(uint32_t(cus));
     s->coopGrid = sor_coop_grid(uint32_t(cus));
     s->sorTiles = s->coopGrid ? sor_tiles_grid(uint32_t(cus)) : 0u;
+    s->sorSafe = sor_tiles_safe(uint32_t(cus));
   }
   double rt = o->ratio > 0 ? o->ratio : 2.0;
   rt = std::max(1.4, std::min(4.0, rt));
@@ -953,7 +956,7 @@ int st_create(const st_opts* o, void** out) {
       (rc = dalloc(&s->G.tmap, s->ntiles)) || (rc = dalloc(&s->G.need, s->ntiles)) || (rc = dalloc(&s->G.newList, size_t(s->ntiles) * 2)) ||
       (rc = dalloc(&s->G.wg, scan_word_count(s->ntiles))) || (rc = dalloc(&s->G.ctl, 16)) || (rc = allocSlots(s, s->scap)) ||
       (rc = dalloc(&s->G.part, 2 * 8192 + 64)) || (rc = dalloc(&s->G.foamTab, FOAM_TAB)) ||
-      (rc = dalloc(&s->G.mortonTiles, s->ntiles)) || (rc = dalloc(&s->G.sorBar, COOP_MAX_WG + 5)) ||
+      (rc = dalloc(&s->G.mortonTiles, s->ntiles)) || (rc = dalloc(&s->G.sorBar, SOR_BAR_WORDS)) ||
       (rc = dalloc(&s->dSlots, RING))) {
     destroySim(s);
     return rc;
@@ -980,7 +983,7 @@ int st_create(const st_opts* o, void** out) {
   if (hipMemcpy(s->G.fstack, st.data(), size_t(s->scap) * 4, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(s->G.tmap, tm.data(), size_t(s->ntiles) * 4, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(s->G.mortonTiles, mort.data(), size_t(s->ntiles) * 4, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemsetAsync(s->G.sorBar, 0, (COOP_MAX_WG + 5) * 4, s->st) != hipSuccess ||
+      hipMemsetAsync(s->G.sorBar, 0, SOR_BAR_WORDS * 4, s->st) != hipSuccess ||
       hipMemsetAsync(s->G.scanW, 0, scan_word_count(s->ntiles) * 8, s->st) != hipSuccess ||
       hipMemcpy(s->G.ctl, ctl, 64, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(s->G.pos, 0, M * 16) != hipSuccess || hipMemset(s->G.vel, 0, M * 16) != hipSuccess ||
@@ -1750,6 +1753,7 @@ int st_batch_create(void* const* sims, uint32_t n, void** out) {
     (void)hipGetLastError();
     b->coopGrid = 0;  // launches per iteration
   }
+  if (b->dPlan) launch_fill_u32(b->st, b->dPlan, batch_plan_words(n), 0u);
   *out = b;
   return ST_OK;
 }
@@ -1831,7 +1835,7 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
     // a cap on the one-launch solve (st_batch_sor_grid) caps the one-per-tile form too
     const Sim* s0 = b->tanks[0];
     const uint32_t tiles = b->coopGrid < s0->coopGrid ? std::min(b->coopGrid, s0->sorTiles) : s0->sorTiles;
-    b->lastResident = launch_batch_step(b->st, (const BTank*)d, (const uint32_t*)(d + b->offTab), hTab, nt, itersMax, b->coopGrid, tiles,
+    b->lastResident = launch_batch_step(b->st, (const BTank*)d, (const uint32_t*)(d + b->offTab), hTab, nt, itersMax, b->coopGrid, tiles, s0->sorSafe,
                                         most, full, passes, b->dPlan) ? 1u : 0u;
   } else {
     // the block tables fix every launch's grid and kernel choice; the tank
@@ -1847,7 +1851,7 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
       HIPCHK(hipGraphLaunch(hit->exec, b->st));
     } else {
       HIPCHK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
-      launch_batch_step(b->st, (const BTank*)d, (const uint32_t*)(d + b->offTab), hTab, nt, itersMax, 0u, 0u, 0u, 0u, passes, nullptr);
+      launch_batch_step(b->st, (const BTank*)d, (const uint32_t*)(d + b->offTab), hTab, nt, itersMax, 0u, 0u, 0u, 0u, 0u, passes, nullptr);
       hipError_t le = hipGetLastError();
       hipGraph_t g = nullptr;
       hipError_t ce = hipStreamEndCapture(b->st, &g);
@@ -1923,6 +1927,7 @@ int st_batch_sor_grid(void* p, uint32_t workgroups) {
     HIPCHK(hipSetDevice(b->dev));
     int rc = dalloc(&b->dPlan, batch_plan_words(uint32_t(b->tanks.size())));
     if (rc) return rc;
+    launch_fill_u32(b->st, b->dPlan, batch_plan_words(uint32_t(b->tanks.size())), 0u);
   }
   // a tank that streams tile windows runs four pipelines per workgroup over
   // eight XCD groups, which needs at least two workgroups

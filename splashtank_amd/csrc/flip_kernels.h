@@ -20,6 +20,13 @@
 #define COOP_MAX_WG 1024
 // most tiles in use of the one-per-tile solve: its exchange words are numbered in 20 bits
 #define SOR_TILES_MAX 2048u
+// its arrival words: one and TS_SUBS counters, a line of TS_LINE words each, in sorBar
+// from SOR_HERE on (a batch: after its plan)
+#define TS_SUBS 32u
+#define TS_LINE 32u
+#define SOR_HERE_WORDS (TS_LINE * (1u + TS_SUBS))
+#define SOR_HERE (COOP_MAX_WG + 32u)
+#define SOR_BAR_WORDS (SOR_HERE + SOR_HERE_WORDS)
 
 struct LaunchCtx {
   const DParams* P;
@@ -34,6 +41,7 @@ struct LaunchCtx {
   uint32_t pipeGrid;  // persistent SOR workgroups (about eight per CU)
   uint32_t coopGrid;  // resident-SOR workgroups (one per CU), 0 when cooperative launches are unavailable
   uint32_t sorTiles;  // workgroups of the one-per-tile solve resident at once (0: not available)
+  uint32_t sorSafe;   // as many are resident at once whatever other streams run
   uint32_t sorTag;    // tag of this solve's first exchange
   uint32_t sorSeq;    // sequence number of this pressure solve
   bool sorStream;     // the cooperative solve streams tile windows even when the tiles fit in LDS
@@ -106,9 +114,10 @@ bool batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t full, uint32_t it
 // resident workgroups, else (or when the launch is refused) one launch per
 // iteration, or per two where `passes` (batch_tables); returns whether it ran
 // resident
-inline size_t batch_plan_words(uint32_t nt) { return size_t(nt) * 4u + 2u; }
+inline __host__ __device__ uint32_t batch_here(uint32_t nt) { return (nt * 4u + 2u + TS_LINE - 1u) / TS_LINE * TS_LINE; }
+inline size_t batch_plan_words(uint32_t nt) { return size_t(batch_here(nt)) + SOR_HERE_WORDS; }
 bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, const uint32_t* htab, uint32_t nt, uint32_t itersMax,
-                       uint32_t coopGrid, uint32_t sorTiles, uint32_t most, uint32_t full, bool passes, uint32_t* dPlan);
+                       uint32_t coopGrid, uint32_t sorTiles, uint32_t sorSafe, uint32_t most, uint32_t full, bool passes, uint32_t* dPlan);
 
 // device-to-device copies made by one launch: whole words, starts aligned to 16
 // bytes (allocations are), at most COPY_LIST_MAX
@@ -143,6 +152,8 @@ uint32_t sor_resident_grid(uint32_t cus);
 uint32_t sor_coop_grid(uint32_t cus);
 // workgroups of the one-per-tile SOR resident at once (at most SOR_TILES_MAX), 0 if none fits
 uint32_t sor_tiles_grid(uint32_t cus);
+// as many of them as are resident at once whatever other streams run
+uint32_t sor_tiles_safe(uint32_t cus);
 // tile indices in Morton order of their (ti, tj, tk) coordinates
 void morton_tiles(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t* out);
 void launch_project(hipStream_t st, const LaunchCtx& L);

@@ -1869,6 +1869,8 @@ __device__ __forceinline__ void sor_resident_body(const DParams* __restrict__ PP
 }
 __global__ void __launch_bounds__(COOP_WG) k_sor_resident(const DParams* __restrict__ PP, DGrid G, uint32_t iters,
                                                           uint32_t seq, uint32_t tag0, uint32_t stream) {
+  if (blockIdx.x == 0u)  // k_sor_tiles' arrivals
+    for (uint32_t q = threadIdx.x; q < SOR_HERE_WORDS; q += COOP_WG) G.sorBar[SOR_HERE + q] = 0u;
   if (G.sorBar[COOP_MAX_WG + 4] == seq) return;  // k_sor_tiles did this solve
   sor_resident_body(PP, G, iters, seq, tag0, stream, blockIdx.x, gridDim.x);
 }
@@ -2190,14 +2192,48 @@ __device__ __forceinline__ void sor_tile_body(const DParams* __restrict__ PP, co
   pres[tid] = sp[own];
   pres[tid + 256u] = sp[own + half];
 }
+// Whether all `total` workgroups with a tile are resident; else none solves.  The
+// launch alone does not see to that: kernels of other streams share the CUs, and a
+// workgroup placed beside one of their waves can leave, once that wave has gone, holes
+// in the register file or the LDS too small for the seventh workgroup, which would
+// then never start while the others wait for it.  Up to sor_tiles_safe workgroups
+// always fit, whatever the holes: at four per CU or fewer, 72 registers a wave and 21
+// KB, the free part of some CU is more than the holes between them can hide.  Above,
+// the workgroups arrive here first; one that has waited about 0.2 ms ends the launch
+// for all, unless the last has just arrived (both change the one word).  here: that
+// word, then 32 counters, a line each; zero before, cleared by the launch after.
+#define TS_LATE 0x80000000u
+#define TS_HERE_SPINS 256u
+__device__ __forceinline__ bool ts_all_here(uint32_t* here, uint32_t w, uint32_t total) {
+  __shared__ uint32_t sOk;
+  if (threadIdx.x == 0u) {
+    const uint32_t sub = w % TS_SUBS, members = (total - sub + TS_SUBS - 1u) / TS_SUBS;
+    if (atomicAdd(&here[TS_LINE * (1u + sub)], 1u) + 1u == members) atomicAdd(here, 1u);
+    uint32_t v = __hip_atomic_load(here, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (uint32_t spins = 0; !(v & TS_LATE) && v != TS_SUBS; spins++) {
+      if (spins >= TS_HERE_SPINS) {
+        const uint32_t was = atomicCAS(here, v, v | TS_LATE);
+        v = was == v ? v | TS_LATE : was;
+        continue;
+      }
+      __builtin_amdgcn_s_sleep(4);
+      v = __hip_atomic_load(here, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    sOk = v == TS_SUBS ? 1u : 0u;
+  }
+  __syncthreads();
+  return sOk != 0u;
+}
 // seq: marks the solve as done (the resident launch that follows where the tiles in
-// use may exceed the workgroups then has nothing to do)
-__global__ void __launch_bounds__(WG, TS_WAVES) k_sor_tiles(const DParams* __restrict__ PP, DGrid G, uint32_t iters, uint32_t tag0, uint32_t seq) {
+// use may exceed `safe` then has nothing to do)
+__global__ void __launch_bounds__(WG, TS_WAVES) k_sor_tiles(const DParams* __restrict__ PP, DGrid G, uint32_t iters, uint32_t tag0, uint32_t seq,
+                                                            uint32_t safe) {
   const uint32_t nact = G.ctl[4], w = blockIdx.x;
   if (nact > G.tileCap) return;
   uint32_t total;
   const uint32_t b = ts_find(G, nact, w, &total);
   if (total > gridDim.x) return;
+  if (b != ST_NONE && total > safe && !ts_all_here(G.sorBar + SOR_HERE, w, total)) return;
   if (w == 0u && threadIdx.x == 0u) {
     G.sorBar[COOP_MAX_WG + 4] = seq;
     G.sorBar[COOP_MAX_WG + 3] = 1u;
@@ -3441,7 +3477,7 @@ __global__ void __launch_bounds__(WG) kb_sor_counts(const BTank* __restrict__ TT
 }
 // every tank's solve with a workgroup per fluid tile, where they all fit at once
 __global__ void __launch_bounds__(WG, TS_WAVES) kb_sor_tiles(const BTank* __restrict__ TT, const uint32_t* __restrict__ act, uint32_t nt,
-                                                             uint32_t* __restrict__ plan) {
+                                                             uint32_t* __restrict__ plan, uint32_t safe) {
   static_assert(ST_BATCH_MAX <= WG, "a thread per tank");
   __shared__ uint32_t sT, sW;
   const uint32_t tid = threadIdx.x, w = blockIdx.x;
@@ -3450,6 +3486,7 @@ __global__ void __launch_bounds__(WG, TS_WAVES) kb_sor_tiles(const BTank* __rest
   uint64_t tot;
   const uint64_t before = wg_scan_u64(cnt, &tot);
   if (tot > gridDim.x) return;
+  if (w < uint32_t(tot) && tot > safe && !ts_all_here(plan + batch_here(nt), w, uint32_t(tot))) return;
   if (w == 0u) {
     if (tid == 0u) plan[3u * nt + 1u] = 1u;
     if (tid < nt && act[tid + 1u] != act[tid]) TT[tid].G.sorBar[COOP_MAX_WG + 3] = 1u;
@@ -3478,6 +3515,7 @@ __global__ void __launch_bounds__(WG) kb_sor_plan(const BTank* __restrict__ TT, 
                                                   uint32_t tiled, uint32_t* __restrict__ plan) {
   // the tanks' tile counts, loaded side by side (one thread after the other took 17 us for 16 tanks)
   __shared__ uint32_t sAct[WG];
+  for (uint32_t q = threadIdx.x; q < SOR_HERE_WORDS; q += WG) plan[batch_here(nt) + q] = 0u;  // kb_sor_tiles' arrivals
   if (threadIdx.x < nt) sAct[threadIdx.x] = act[threadIdx.x + 1u] != act[threadIdx.x] ? TT[threadIdx.x].G.ctl[4] : 0u;
   __syncthreads();
   if (threadIdx.x != 0u || blockIdx.x != 0u) return;
@@ -3650,6 +3688,7 @@ uint32_t sor_coop_grid(uint32_t cus) {
   return std::min<uint32_t>(cus, COOP_MAX_WG);
 }
 
+uint32_t sor_tiles_safe(uint32_t cus) { return cus * 4u; }
 uint32_t sor_tiles_grid(uint32_t cus) {
   int nb = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sor_tiles, WG, 0) != hipSuccess || nb < 1) return 0u;
@@ -3692,15 +3731,17 @@ hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters) {
     // in use, and about as many as the particles would fill, and their neighbours
     const uint32_t most = std::min<uint32_t>(L.ntiles, L.scap - 1u);
     if (!stream && L.sorTiles && (most <= L.sorTiles || sor_tiles_likely(L.fullTiles, L.sorTiles))) {
-      void* args[] = {(void*)&P, (void*)&G, (void*)&it, (void*)&tag, (void*)&seq};
+      uint32_t safe = L.sorSafe;
+      void* args[] = {(void*)&P, (void*)&G, (void*)&it, (void*)&tag, (void*)&seq, (void*)&safe};
       coopErr = hipLaunchCooperativeKernel((const void*)k_sor_tiles, dim3(std::min(most, L.sorTiles)), dim3(WG), args, 0, st);
-      if (coopErr == hipSuccess && most <= L.sorTiles) return hipSuccess;
+      if (coopErr == hipSuccess && most <= L.sorSafe) return hipSuccess;
       if (coopErr != hipSuccess) (void)hipGetLastError();  // the launch below does the solve
     }
     void* args[] = {(void*)&P, (void*)&G, (void*)&it, (void*)&seq, (void*)&tag, (void*)&stream};
     coopErr = hipLaunchCooperativeKernel((const void*)k_sor_resident, dim3(L.coopGrid), dim3(COOP_WG), args, 0, st);
     if (coopErr == hipSuccess) return hipSuccess;
     (void)hipGetLastError();  // the per-iteration launches below do the solve
+    launch_fill_u32(st, L.G.sorBar + SOR_HERE, SOR_HERE_WORDS, 0u);
   }
   // one or two iterations a launch, ping-pong between the two pressure buffers; an
   // odd count of single ones leaves the result in pres2 and it is copied back
@@ -3850,7 +3891,7 @@ bool batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t full, uint32_t it
 }
 
 bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, const uint32_t* htab, uint32_t nt, uint32_t itersMax,
-                       uint32_t coopGrid, uint32_t sorTiles, uint32_t most, uint32_t full, bool passes, uint32_t* dPlan) {
+                       uint32_t coopGrid, uint32_t sorTiles, uint32_t sorSafe, uint32_t most, uint32_t full, bool passes, uint32_t* dPlan) {
   const size_t w = size_t(nt) + 1u;
   auto tab = [&](uint32_t k) { return dtab + k * w; };
   auto tot = [&](uint32_t k) { return htab[k * w + nt]; };
@@ -3882,10 +3923,11 @@ bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, co
     if (tiles) {
       hipLaunchKernelGGL(kb_sor_counts, dim3(nt), dim3(WG), 0, st, dT, actTab, nt, dPlan);
       uint32_t* plan = dPlan;
-      void* args[] = {(void*)&a0, (void*)&actTab, (void*)&nt, (void*)&plan};
+      uint32_t safe = sorSafe;
+      void* args[] = {(void*)&a0, (void*)&actTab, (void*)&nt, (void*)&plan, (void*)&safe};
       done = hipLaunchCooperativeKernel((const void*)kb_sor_tiles, dim3(std::max(1u, std::min(most, sorTiles))), dim3(WG), args, 0, st) == hipSuccess;
       if (!done) (void)hipGetLastError();
-      done = done && most <= sorTiles;  // else the launches below do the solve where it did not fit
+      done = done && most <= sorSafe;  // else the launches below do the solve where it did not fit
     }
     if (!done) hipLaunchKernelGGL(kb_sor_plan, dim3(1), dim3(WG), 0, st, dT, actTab, nt, coopGrid, tiles ? 1u : 0u, dPlan);
     const uint32_t* a1 = dPlan;
