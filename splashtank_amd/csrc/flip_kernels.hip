@@ -9,12 +9,14 @@
 //    round) with LDS integer atomics and adds the window to HBM once; the sums
 //    are fixed point, so the order the atomics land in does not matter;
 //  * g2p stages the same window of face velocities and counts in LDS;
-//  * cell kernels are grid-stride loops over the device-side count of tiles in
-//    use (ctl[4]), so no launch needs a host readback and all can live in a graph;
-//  * the red-black SOR runs every iteration of a solve in one cooperative
-//    launch, each CU keeping the pressure of a Morton-ordered range of tiles in
-//    LDS and exchanging face halos with the others through a grid barrier; a
-//    per-iteration tile-window kernel is the other path.
+//  * cell kernels walk the tiles in use, by half tile or cell by cell; their count
+//    (ctl[4]) is on the device, so no launch needs a host readback and all can live
+//    in a graph;
+//  * the red-black SOR runs every iteration of a solve in one cooperative launch:
+//    with a workgroup per fluid tile that exchanges once per two iterations where
+//    the tiles are few, else each CU keeping the pressure of a Morton-ordered range
+//    of tiles in LDS; tagged words carry the values between workgroups.  Launches of
+//    one or two iterations on tile windows are the other path.
 // The reference's kernels each of these replaces are cited at the kernel.
 #include "flip_device.h"
 #include "flip_kernels.h"
@@ -2574,7 +2576,7 @@ __device__ __forceinline__ void d_sampleBoth(const DParams& P, const GridT& g, f
 // The part of g2p that depends only on the density sum csum (the count of the
 // 8 cells around the particle, or 8 x its own cell's count): air, shield, the
 // foam decay exp(-dt / tau) and the drag factor 1 - exp(-kd dt)
-// (wgsl-solver.js:221-245).  Per step, k_foam_table evaluates it for every
+// (wgsl-solver.js:221-245).  Per step, tiles_finish evaluates it for every
 // integer csum below FOAM_TAB; g2p reads the table, which gives the same bits
 // as evaluating it in place.
 __device__ __forceinline__ float4 d_foamRow(const DParams& P, float csum) {
