@@ -2330,13 +2330,19 @@ __global__ void k_copy_tiles(DGrid G, const float* __restrict__ src, float* __re
 }
 
 // projBody / project (wgsl-solver.js:165-180)
+// SAVE: the narrow band's saveVel (wgsl-narrowband.js:88-91) too, the faces being at hand
+// (a launch of its own took 5 us)
+template <bool SAVE>
 __device__ __forceinline__ void project_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid) {
   const DParams& P = *PP;
   FOR_TILES(G, T, l) {
     const uint32_t c = T.s * 512u + l;
     const int3 at = make_int3(T.x + int32_t(l & 7u), T.y + int32_t((l >> 3) & 7u), T.z + int32_t(l >> 6));
     const uint32_t th = type_at(P, G, at.x, at.y, at.z, c);
-    if (th == 2u) continue;
+    if (th == 2u) {
+      if constexpr (SAVE) face3_put(reinterpret_cast<int32_t*>(G.velG), c, face3(G.accV, c));
+      continue;
+    }
     const uint32_t cl[3] = {nb_down(T.s, T.xm, l, 0u), nb_down(T.s, T.ym, l, 3u), nb_down(T.s, T.zm, l, 6u)};
     const float ph = th == 1u ? G.pres[c] : 0.0f;
     Face3 fv = face3(G.accV, c);
@@ -2351,10 +2357,12 @@ __device__ __forceinline__ void project_body(const DParams* __restrict__ PP, con
       set = true;
     }
     if (set) face3_put(G.accV, c, fv);
+    if constexpr (SAVE) face3_put(reinterpret_cast<int32_t*>(G.velG), c, fv);
   }
 }
+template <bool SAVE>
 __global__ void __launch_bounds__(WG) k_project(const DParams* __restrict__ PP, DGrid G) {
-  project_body(PP, G, blockIdx.x, gridDim.x);
+  project_body<SAVE>(PP, G, blockIdx.x, gridDim.x);
 }
 
 // Opt-in velocity extrapolation after the projection (no counterpart in the
@@ -3578,7 +3586,7 @@ __global__ void __launch_bounds__(COOP_WG) kb_sor_resident(const BTank* __restri
   }
 }
 
-__global__ void __launch_bounds__(WG) kb_project(BATCH_ARGS) { BATCH_TANK; BATCH_LOCAL; project_body(&uP, G, b.blk, b.nblk); }
+__global__ void __launch_bounds__(WG) kb_project(BATCH_ARGS) { BATCH_TANK; BATCH_LOCAL; project_body<false>(&uP, G, b.blk, b.nblk); }
 __global__ void __launch_bounds__(WG) kb_g2p_tile(BATCH_ARGS) {
   BATCH_TANK;
   BATCH_LOCAL;
@@ -3762,15 +3770,18 @@ hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters) {
 }
 
 void launch_project(hipStream_t st, const LaunchCtx& L) {
-  hipLaunchKernelGGL(k_project, dim3(L.faceGrid), dim3(WG), 0, st, L.P, L.G);
-  if (L.extrap && L.exMask) {
+  const bool extrap = L.extrap && L.exMask;
+  // the kept velocity is the extrapolated one where there is that
+  if (L.nbOn && !extrap) hipLaunchKernelGGL(k_project<true>, dim3(L.faceGrid), dim3(WG), 0, st, L.P, L.G);
+  else hipLaunchKernelGGL(k_project<false>, dim3(L.faceGrid), dim3(WG), 0, st, L.P, L.G);
+  if (extrap) {
     const size_t C = size_t(L.scap) * 512u;
     hipLaunchKernelGGL(k_extrap_init, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G, L.exMask);
     for (uint32_t l = 0; l < L.extrap; l++)
       hipLaunchKernelGGL(k_extrap_layer, dim3(L.cellGrid), dim3(WG), 0, st, L.P, L.G, (const uint8_t*)(L.exMask + (l & 1u) * C),
                          L.exMask + ((l + 1u) & 1u) * C);
   }
-  if (L.nbOn) hipLaunchKernelGGL(k_save_vel, dim3(L.cellGrid), dim3(WG), 0, st, L.G);
+  if (L.nbOn && extrap) hipLaunchKernelGGL(k_save_vel, dim3(L.cellGrid), dim3(WG), 0, st, L.G);
 }
 
 // Workgroups that share one tile's particles in g2p.  A full tile is 16 rounds of
