@@ -73,14 +73,18 @@ def build_napi() -> str | None:
     return ADDON
 
 
-def build_checks() -> str:
-    """Device self-checks the GPU tests run (tests/c/*.hip), as a library beside them."""
-    src = os.path.join(ROOT, "tests", "c", "convert_check.hip")
-    out = os.path.join(ROOT, "tests", "c", "libconvert_check.so")
-    tmp = out + ".tmp"
-    _run([HIPCC, *HIP_FLAGS, "-shared", src, "-o", tmp])
-    os.replace(tmp, out)
-    return out
+def build_checks() -> list:
+    """What the tests load beside the library (tests/c/*.hip): a device self-check and
+    a HIP runtime of host memory, which must not bind the real one."""
+    outs = []
+    for name, extra in (("convert_check", []), ("host_hip", ["-no-hip-rt"])):
+        src = os.path.join(ROOT, "tests", "c", name + ".hip")
+        out = os.path.join(ROOT, "tests", "c", f"lib{name}.so")
+        tmp = out + ".tmp"
+        _run([HIPCC, *HIP_FLAGS, "-shared", *extra, src, "-o", tmp])
+        os.replace(tmp, out)
+        outs.append(out)
+    return outs
 
 
 def build_oracle() -> str:

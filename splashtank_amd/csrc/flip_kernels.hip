@@ -3744,7 +3744,8 @@ hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters) {
       uint32_t safe = L.sorSafe;
       void* args[] = {(void*)&P, (void*)&G, (void*)&it, (void*)&tag, (void*)&seq, (void*)&safe};
       coopErr = hipLaunchCooperativeKernel((const void*)k_sor_tiles, dim3(std::min(most, L.sorTiles)), dim3(WG), args, 0, st);
-      if (coopErr == hipSuccess && most <= L.sorSafe) return hipSuccess;
+      // it is all there is to do only where every tile that can be in use has a workgroup
+      if (coopErr == hipSuccess && most <= std::min(L.sorSafe, L.sorTiles)) return hipSuccess;
       if (coopErr != hipSuccess) (void)hipGetLastError();  // the launch below does the solve
     }
     void* args[] = {(void*)&P, (void*)&G, (void*)&it, (void*)&seq, (void*)&tag, (void*)&stream};
@@ -3940,7 +3941,9 @@ bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, co
       void* args[] = {(void*)&a0, (void*)&actTab, (void*)&nt, (void*)&plan, (void*)&safe};
       done = hipLaunchCooperativeKernel((const void*)kb_sor_tiles, dim3(std::max(1u, std::min(most, sorTiles))), dim3(WG), args, 0, st) == hipSuccess;
       if (!done) (void)hipGetLastError();
-      done = done && most <= sorSafe;  // else the launches below do the solve where it did not fit
+      // every tile that can be in use has a workgroup (a cap may leave fewer, whatever
+      // `full` says); else the launches below do the solve where it did not fit
+      done = done && most <= std::min(sorSafe, sorTiles);
     }
     if (!done) hipLaunchKernelGGL(kb_sor_plan, dim3(1), dim3(WG), 0, st, dT, actTab, nt, coopGrid, tiles ? 1u : 0u, dPlan);
     const uint32_t* a1 = dPlan;
