@@ -3724,6 +3724,13 @@ void morton_tiles(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t* out) {
   for (size_t m = 0; m < key.size(); m++) out[m] = key[m].second;
 }
 
+// whether a device word holds v once the stream's work is done (only where a
+// cooperative launch has been refused)
+static bool word_is(hipStream_t st, const uint32_t* p, uint32_t v) {
+  uint32_t w = ~v;
+  return hipMemcpyAsync(&w, p, 4, hipMemcpyDeviceToHost, st) == hipSuccess && hipStreamSynchronize(st) == hipSuccess && w == v;
+}
+
 hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters) {
   hipError_t coopErr = hipSuccess;
   if (L.coopGrid && iters > 0) {
@@ -3737,6 +3744,7 @@ hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters) {
     const DParams* P = L.P;
     DGrid G = L.G;
     uint32_t it = uint32_t(iters), seq = L.sorSeq, tag = L.sorTag, stream = L.sorStream ? 1u : 0u;
+    bool tiled = false;
     // a workgroup per tile where every tile in use has one: at most `most` tiles are
     // in use, and about as many as the particles would fill, and their neighbours
     const uint32_t most = std::min<uint32_t>(L.ntiles, L.scap - 1u);
@@ -3746,13 +3754,15 @@ hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters) {
       coopErr = hipLaunchCooperativeKernel((const void*)k_sor_tiles, dim3(std::min(most, L.sorTiles)), dim3(WG), args, 0, st);
       // it is all there is to do only where every tile that can be in use has a workgroup
       if (coopErr == hipSuccess && most <= std::min(L.sorSafe, L.sorTiles)) return hipSuccess;
-      if (coopErr != hipSuccess) (void)hipGetLastError();  // the launch below does the solve
+      tiled = coopErr == hipSuccess;
+      if (!tiled) (void)hipGetLastError();  // the launch below does the solve
     }
     void* args[] = {(void*)&P, (void*)&G, (void*)&it, (void*)&seq, (void*)&tag, (void*)&stream};
     coopErr = hipLaunchCooperativeKernel((const void*)k_sor_resident, dim3(L.coopGrid), dim3(COOP_WG), args, 0, st);
     if (coopErr == hipSuccess) return hipSuccess;
     (void)hipGetLastError();  // the per-iteration launches below do the solve
     launch_fill_u32(st, L.G.sorBar + SOR_HERE, SOR_HERE_WORDS, 0u);
+    if (tiled && word_is(st, L.G.sorBar + COOP_MAX_WG + 4, seq)) return coopErr;  // unless k_sor_tiles did
   }
   // one or two iterations a launch, ping-pong between the two pressure buffers; an
   // odd count of single ones leaves the result in pres2 and it is copied back
@@ -3933,24 +3943,27 @@ bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, co
     const BTank* a0 = dT;
     const uint32_t* actTab = tab(BT_PIPE0);
     const bool tiles = sorTiles && (most <= sorTiles || sor_tiles_likely(full, sorTiles));
-    bool done = false;
+    bool done = false, tiled = false;
     if (tiles) {
       hipLaunchKernelGGL(kb_sor_counts, dim3(nt), dim3(WG), 0, st, dT, actTab, nt, dPlan);
       uint32_t* plan = dPlan;
       uint32_t safe = sorSafe;
       void* args[] = {(void*)&a0, (void*)&actTab, (void*)&nt, (void*)&plan, (void*)&safe};
-      done = hipLaunchCooperativeKernel((const void*)kb_sor_tiles, dim3(std::max(1u, std::min(most, sorTiles))), dim3(WG), args, 0, st) == hipSuccess;
-      if (!done) (void)hipGetLastError();
+      tiled = hipLaunchCooperativeKernel((const void*)kb_sor_tiles, dim3(std::max(1u, std::min(most, sorTiles))), dim3(WG), args, 0, st) == hipSuccess;
+      if (!tiled) (void)hipGetLastError();
       // every tile that can be in use has a workgroup (a cap may leave fewer, whatever
       // `full` says); else the launches below do the solve where it did not fit
-      done = done && most <= std::min(sorSafe, sorTiles);
+      done = tiled && most <= std::min(sorSafe, sorTiles);
     }
     if (!done) hipLaunchKernelGGL(kb_sor_plan, dim3(1), dim3(WG), 0, st, dT, actTab, nt, coopGrid, tiles ? 1u : 0u, dPlan);
     const uint32_t* a1 = dPlan;
     uint32_t a2 = nt;
     void* args[] = {(void*)&a0, (void*)&a1, (void*)&a2};
     resident = done || hipLaunchCooperativeKernel((const void*)kb_sor_resident, dim3(coopGrid), dim3(COOP_WG), args, 0, st) == hipSuccess;
-    if (!resident) (void)hipGetLastError();  // the launches per iteration below do the solve
+    if (!resident) {  // refused: the launches per iteration below do the solve, unless kb_sor_tiles did
+      (void)hipGetLastError();
+      resident = tiled && word_is(st, dPlan + 3u * nt + 1u, 1u);
+    }
   }
   if (!resident) {
     if (passes) {
