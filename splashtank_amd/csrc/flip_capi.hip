@@ -638,7 +638,10 @@ int runStage(Sim* s, int stage, bool alone = false) {
     default: return fail(ST_ERR_ARG, "st_stage: unknown stage");
   }
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(ST_ERR_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
+  if (e != hipSuccess) {  // what the stage's launches should have left may not be there
+    s->binned = s->marksClean = s->barClean = false;
+    return fail(ST_ERR_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
+  }
   return ST_OK;
 }
 
@@ -723,17 +726,38 @@ int graphStep(Sim* s, const st_params* o) {
   e.extrap = s->extrapOnStep;
   e.exec = nullptr;
   HIPCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
+  // the stages change the tank's host state as they are captured; where the graph
+  // does not run, none of that has happened
+  const bool barClean = s->barClean;
+  const uint32_t sorSeq = s->sorSeq;
+  auto undo = [&] {
+    s->G = e.G;
+    s->binned = e.binned;
+    s->marksClean = e.marksClean;
+    s->barClean = barClean;
+    s->solidDirty = e.solid;
+    s->sorSeq = sorSeq;
+  };
   for (int st = 0; st < ST_STAGE_COUNT && !rc; st++) rc = runStage(s, st);
   hipGraph_t g = nullptr;
   hipError_t ce = hipStreamEndCapture(s->st, &g);
   if (rc || ce != hipSuccess) {
     if (g) (void)hipGraphDestroy(g);
+    undo();
     return rc ? rc : fail(ST_ERR_HIP, std::string("st_step_n: stream capture: ") + hipGetErrorString(ce));
   }
   hipError_t ie = hipGraphInstantiate(&e.exec, g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
-  if (ie != hipSuccess) return fail(ST_ERR_HIP, std::string("st_step_n: hipGraphInstantiate: ") + hipGetErrorString(ie));
-  HIPCHK(hipGraphLaunch(e.exec, s->st));
+  if (ie != hipSuccess) {
+    undo();
+    return fail(ST_ERR_HIP, std::string("st_step_n: hipGraphInstantiate: ") + hipGetErrorString(ie));
+  }
+  ie = hipGraphLaunch(e.exec, s->st);
+  if (ie != hipSuccess) {
+    (void)hipGraphExecDestroy(e.exec);
+    undo();
+    return fail(ST_ERR_HIP, std::string("st_step_n: hipGraphLaunch: ") + hipGetErrorString(ie));
+  }
   if (s->graphs.size() >= GRAPH_CACHE) {
     HIPCHK(hipStreamSynchronize(s->st));
     (void)hipGraphExecDestroy(s->graphs.front().exec);
@@ -1875,7 +1899,10 @@ static int batchStep(Batch* b, const st_params* prm, uint32_t nprm, bool graph) 
     }
   }
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(ST_ERR_HIP, std::string("batched launch: ") + hipGetErrorString(e));
+  if (e != hipSuccess) {
+    for (Sim* s : b->tanks) s->binned = s->marksClean = s->barClean = false;
+    return fail(ST_ERR_HIP, std::string("batched launch: ") + hipGetErrorString(e));
+  }
   // what the single-tank stages leave behind: g2p wrote the new state into the
   // other buffers and binned it for the next substep
   for (uint32_t t = 0; t < nt; t++) {

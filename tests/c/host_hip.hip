@@ -1,6 +1,7 @@
 // A HIP runtime of host memory, for CPU tests of the library's host code: device
 // memory is the heap, copies are memcpy, and a launch only writes a line to a log
-// (kernel name, workgroups, threads, cooperative or not).  Loaded with global
+// (kernel name, workgroups, threads, cooperative or not; the id-order readback also
+// does its work).  Loaded with global
 // symbols before libsplashtank_hip.so, whose HIP calls then come here.  Built by the
 // package build into tests/c/libhost_hip.so and used through tests/host_hip.py.
 // host_hip_set makes calls fail, and lets the one-per-tile solves mark their work
@@ -27,6 +28,7 @@ static int64_t g_live = 0;
 static int g_refuse = 0;      // cooperative launches of this many threads are refused
 static int g_solves = 0;      // the one-per-tile solves do their work
 static int g_failCapture = 0; // the next capture ends with an error
+static int g_failLaunch = 0;  // the next look for a launch's error finds one
 static char g_any[64];        // what handles point at
 
 static hipError_t logf(const char* what, const void* f, dim3 g, dim3 b, hipStream_t st) {
@@ -43,6 +45,7 @@ void host_hip_set(const char* what, int v) {
   if (!strcmp(what, "refuse")) g_refuse = v;
   if (!strcmp(what, "solves")) g_solves = v;
   if (!strcmp(what, "failCapture")) g_failCapture = v;
+  if (!strcmp(what, "failLaunch")) g_failLaunch = v;
 }
 
 void** __hipRegisterFatBinary(const void*) { return (void**)g_any; }
@@ -69,7 +72,11 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int
   *n = threads >= 1024 ? 1 : 7;
   return hipSuccess;
 }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = g_failLaunch ? hipErrorLaunchFailure : hipSuccess;
+  g_failLaunch = 0;
+  return e;
+}
 const char* hipGetErrorString(hipError_t) { return "host"; }
 hipError_t hipGetSymbolAddress(void** p, const void*) { *p = g_any; return hipSuccess; }
 
@@ -120,7 +127,14 @@ hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float* t, hipEvent_t, hipEvent_t) { *t = 1.0f; return hipSuccess; }
 
-hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void**, size_t, hipStream_t st) { return logf("launch", f, g, b, st); }
+hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t, hipStream_t st) {
+  if (kernels()[f].find("8k_unsortP") != std::string::npos) {  // the id-order readback: (src, ids, out, n)
+    const float4* src = *(const float4**)args[0];
+    const uint32_t* id = *(const uint32_t**)args[1];
+    for (uint32_t i = 0; i < *(uint32_t*)args[3]; i++) (*(float4**)args[2])[id[i]] = src[i];
+  }
+  return logf("launch", f, g, b, st);
+}
 hipError_t hipLaunchCooperativeKernel(const void* f, dim3 g, dim3 b, void** args, unsigned int, hipStream_t st) {
   if (g_refuse && b.x == unsigned(g_refuse)) {
     logf("refused", f, g, b, st);

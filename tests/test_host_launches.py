@@ -60,3 +60,85 @@ def test_refused_second_launch_does_not_repeat_a_solve(batch, solved):
     assert [w for w, n in names if n.endswith("sor_tiles")] == ["coop"]
     assert [w for w, n in names if n.endswith("resident")] == ["refused"]
     assert bool(per_iteration) == (not solved), names
+
+
+@pytest.mark.parametrize("steps", [0, 1, 2])
+def test_failed_capture_leaves_the_tank_as_it_was(steps):
+    """A substep whose capture fails has run no kernel: the particles are those
+    before it, and the next substep marks and bins what a tank without it would."""
+    out = json.loads(run(f"""
+        import json
+        sc = scenes.sparse_splash(d=1.0 / 64, iters=6)
+        cf, sdf, sig = sc.collider_state(0.0, sc.params["dt"])
+        prm = capi.make_params(**sc.params)
+        out = []
+        for fails in (0, 1):
+            g = capi.FlipSimC(opts_for(sc))
+            g.upload(sc.pos, sc.vel)
+            for _ in range({steps}):
+                g.step(prm)
+            before = g.read_particles()
+            g.set_colliders(cf, sdf, sig)
+            if fails:
+                hip.host_hip_set(b"failCapture", 1)
+                try:
+                    g.step_n(prm, 1, graph=True)
+                    raise SystemExit("the capture did not fail")
+                except capi.StError:
+                    pass
+                assert np.array_equal(g.read_particles(), before)
+            log()
+            g.step(prm)
+            out.append(launches())
+            g.step_n(prm, 2, graph=True)
+            out.append(log())
+        print(json.dumps(out))
+        """))
+    assert out[:2] == out[2:]
+
+
+def test_failed_launch_clears_the_marks_again():
+    """A blocks stage that failed may not have cleared the tile marks and bin counts:
+    the next substep does before it marks."""
+    out = json.loads(run("""
+        import json
+        sc = scenes.dam_break(d=1.0 / 32, iters=6)
+        prm = capi.make_params(**sc.params)
+        g = capi.FlipSimC(opts_for(sc))
+        g.upload(sc.pos, sc.vel)
+        g.begin_step(prm)
+        g.stage(capi.ST_STAGE_SORT)
+        log()
+        hip.host_hip_set(b"failLaunch", 1)
+        try:
+            g.stage(capi.ST_STAGE_BLOCKS)
+            raise SystemExit("the stage did not fail")
+        except capi.StError:
+            out = [[n for _, n, _, _ in launches()][:4]]
+        g.step(prm)
+        out.append([n for _, n, _, _ in launches()][:4])
+        print(json.dumps(out))
+        """))
+    assert out[0] == out[1] == ["k_fill_u32", "k_fill_u32", "k_mark_bin", "k_tiles_scan"]
+
+
+def test_failed_batch_launch_clears_the_marks_again():
+    out = json.loads(run("""
+        import json
+        sc = scenes.dam_break(d=1.0 / 32, iters=6)
+        prm = capi.make_params(**sc.params)
+        g = capi.FlipSimC(opts_for(sc))
+        g.upload(sc.pos, sc.vel)
+        g.begin_step(prm)
+        g.stages(capi.ST_STAGE_BLOCKS)  # leaves the marks and counts cleared
+        b = capi.FlipBatchC([g])
+        hip.host_hip_set(b"failLaunch", 1)
+        try:
+            b.step(prm)
+            raise SystemExit("the step did not fail")
+        except capi.StError:
+            log()
+        b.step(prm)
+        print(json.dumps([n for _, n, _, _ in launches()][:3]))
+        """))
+    assert out == ["kb_fill_bins", "kb_mark_bin", "kb_tiles_scan"]
