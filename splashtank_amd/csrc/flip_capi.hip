@@ -1223,8 +1223,18 @@ int st_grow(void* p, uint32_t n) {
   s->G.slotList = nullptr; s->G.nbr = nullptr; s->G.nbrL = nullptr; s->G.tileRec = nullptr; s->G.slotPos = nullptr; s->G.posFluid = nullptr;
   s->G.sorTileW = nullptr; s->G.coopList = nullptr; s->G.sorHalo = nullptr;
   int rc = allocSlots(s, n);
+  uint8_t* mask = nullptr;  // two per pool cell, made anew each time it is used
+  if (!rc && s->exMask) rc = dalloc(&mask, size_t(n) * 512u * 2u);
   if (rc) { freeSlots(s); s->G = keep; return rc; }
-  // the wg scratch and grid sizes follow the pool
+  if (mask) {
+    dfree(s->exMask);
+    s->exMask = mask;
+    s->exCells = n * 512u;
+  }
+  // the clears above run on the tank's stream, the copies below do not
+  HIPCHK(hipStreamSynchronize(s->st));
+  // everything a later stage reads, as the pool may grow between two stages of a
+  // substep; the wg scratch and grid sizes follow the pool
   size_t C = size_t(old) * 512;
   HIPCHK(hipMemcpy(s->G.cnt, keep.cnt, C * 4, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.ctype, keep.ctype, C * 4, hipMemcpyDeviceToDevice));
@@ -1238,6 +1248,8 @@ int st_grow(void* p, uint32_t n) {
   HIPCHK(hipMemcpy(s->G.slotTile, keep.slotTile, size_t(old) * 4, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.fstack, keep.fstack, size_t(old) * 4, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.slotList, keep.slotList, size_t(old) * 4, hipMemcpyDeviceToDevice));
+  HIPCHK(hipMemcpy(s->G.nbr, keep.nbr, size_t(old) * 27 * 4, hipMemcpyDeviceToDevice));
+  HIPCHK(hipMemcpy(s->G.nbrL, keep.nbrL, size_t(old) * 27 * 4, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.slotPos, keep.slotPos, size_t(old) * 4, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.posFluid, keep.posFluid, size_t(old) * 2, hipMemcpyDeviceToDevice));
   HIPCHK(hipMemcpy(s->G.tileRec, keep.tileRec, size_t(old) * 48, hipMemcpyDeviceToDevice));

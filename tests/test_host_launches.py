@@ -142,3 +142,27 @@ def test_failed_batch_launch_clears_the_marks_again():
         print(json.dumps([n for _, n, _, _ in launches()][:3]))
         """))
     assert out == ["kb_fill_bins", "kb_mark_bin", "kb_tiles_scan"]
+
+
+def test_grown_pool_is_cleared_before_it_is_filled():
+    """st_grow clears new arrays on the tank's stream and copies the old ones in
+    without a stream: a wait lies between."""
+    out = json.loads(run("""
+        import json
+        sc = scenes.dam_break(d=1.0 / 32, iters=6)
+        g = capi.FlipSimC(opts_for(sc, slots=20))
+        g.upload(sc.pos, sc.vel)
+        log()
+        g.grow(25)
+        print(json.dumps(log()))
+        """))
+    assert out.index("memset stream") < out.index("copy null")
+    pending = False
+    for line in out[:len(out) - out[::-1].index("copy null")]:
+        if line == "memset stream":
+            pending = True
+        if line == "sync":
+            pending = False
+        if line == "copy null":
+            assert not pending
+            break
