@@ -217,6 +217,8 @@ class Rollout:
     def backward_raw(self, snaps, g_pos: np.ndarray, g_vel: np.ndarray):
         """Gradient of the initial (pos, vel), and of the key positions of each
         keyed collider, from that of the final state."""
+        if snaps:
+            snaps[-1].restore()  # this pass's particle count, whatever ran since
         n = self.sim.count()
         gp, gv = (q.numpy() for q in self._host_rows(n))
         for dst, src in ((gp, g_pos), (gv, g_vel)):
