@@ -118,10 +118,8 @@ class Rollout:
         self.t0 = float(t0)
         self.keys = [None] * len(self.cols)
         # kept for the rollout's life: two (n, 4) pinned host buffers that states and
-        # gradients cross through, and the adjoint context with its tapes
+        # gradients cross through
         self._rows = None
-        self._adj = None
-        self._adj_slots = 0
         self._sdf = np.concatenate([c.data for c in self.cols]) if self.cols else np.zeros(0, np.float32)
 
     def __call__(self, pos0: torch.Tensor, vel0: torch.Tensor, *keys: torch.Tensor):
@@ -184,11 +182,7 @@ class Rollout:
         """Reverse the recorded segments from the final state's gradient in the host
         rows, which then hold the initial state's; returns the key gradients."""
         gp, gv = self._host_rows(n)
-        if self._adj is None or self._adj_slots != self.sim.dims.scap:
-            self._drop_adjoint()
-            self._adj = capi.AdjointC(self.sim, self.every)
-            self._adj_slots = self.sim.dims.scap
-        adj = self._adj
+        adj = capi.AdjointC(self.sim, max(1, min(self.every, self.nsteps)))
         gkeys = [np.zeros((len(c.times), 3)) for c in self.cols]
         try:
             for k in reversed(range(len(snaps))):
@@ -209,9 +203,8 @@ class Rollout:
                             gkeys[q] += np.outer(wc, g[q, 0:3]) + np.outer(wv, g[q, 3:6])
             if snaps:
                 adj._call("grad", gp.data_ptr(), gv.data_ptr())
-        except Exception:
-            self._drop_adjoint()  # it may hold tapes of substeps that were not reversed
-            raise
+        finally:
+            adj.close()  # its tapes are most of the memory of a pass, and none of it is needed between passes
         return gkeys
 
     def backward_raw(self, snaps, g_pos: np.ndarray, g_vel: np.ndarray):
@@ -227,13 +220,8 @@ class Rollout:
         gkeys = self._reverse(n, snaps)
         return gp[:, :3].copy(), gv[:, :3].copy(), gkeys
 
-    def _drop_adjoint(self):
-        if self._adj is not None:
-            self._adj.close()
-            self._adj = None
-
     def close(self):
-        self._drop_adjoint()
+        self._rows = None
         self.base.close()
         self.sim.close()
 

@@ -44,10 +44,47 @@ struct StepSlot {
 };
 const int RING = 64;
 
+// The largest block of device memory that an adjoint context freed lately, of
+// SPARE_MAX bytes at most, kept for the next context of about its size: freeing device
+// memory costs 0.25 to 0.6 ms an allocation beyond the 64 MB that the runtime keeps,
+// and a program that reverses passes makes and frees a context each time (adjoint of a
+// 64^3 tank, four substeps: 7.75 ms a pass without it, 7.4 with it).  Given back when
+// an allocation fails and when the last tank goes.  A context's stream has been waited
+// for before its blocks come here, so any stream and thread may have them next.
+const size_t SPARE_MAX = size_t(256) << 20;
+struct Block {
+  uint8_t* p = nullptr;
+  size_t bytes = 0;
+  int dev = 0;
+};
+std::mutex g_spareLock;
+Block g_spare;
+uint32_t g_sims = 0;
+bool dropSpare() {
+  std::lock_guard<std::mutex> l(g_spareLock);
+  const bool had = g_spare.p != nullptr;
+  if (had) (void)hipFree(g_spare.p);
+  g_spare = Block{};
+  return had;
+}
+void countSims(int d) {
+  bool last;
+  {
+    std::lock_guard<std::mutex> l(g_spareLock);
+    g_sims += uint32_t(d);
+    last = g_sims == 0;
+  }
+  if (last) (void)dropSpare();
+}
+
 template <class T> int dalloc(T** p, size_t n) {
   *p = nullptr;
   if (n == 0) n = 1;
   hipError_t e = hipMalloc((void**)p, n * sizeof(T));
+  if (e != hipSuccess && dropSpare()) {
+    (void)hipGetLastError();
+    e = hipMalloc((void**)p, n * sizeof(T));
+  }
   if (e != hipSuccess) return fail(ST_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
   return ST_OK;
 }
@@ -55,6 +92,40 @@ template <class T> void dfree(T*& p) {
   if (p) (void)hipFree((void*)p);
   p = nullptr;
 }
+int takeBlock(Block& b, size_t bytes, int dev) {
+  {
+    std::lock_guard<std::mutex> l(g_spareLock);
+    if (g_spare.p && g_spare.dev == dev && g_spare.bytes >= bytes && g_spare.bytes / 2u <= bytes) {
+      b = g_spare;
+      g_spare = Block{};
+      return ST_OK;
+    }
+  }
+  b.bytes = bytes;
+  b.dev = dev;
+  return dalloc(&b.p, bytes);
+}
+void giveBlock(Block b) {
+  {
+    std::lock_guard<std::mutex> l(g_spareLock);
+    if (g_sims && b.bytes <= SPARE_MAX && b.bytes >= g_spare.bytes) std::swap(b, g_spare);
+  }
+  dfree(b.p);
+}
+
+// Several arrays in one allocation, each at a multiple of 256 bytes
+struct Slab {
+  std::vector<std::pair<void**, size_t>> parts;
+  size_t bytes = 0;
+  template <class T> Slab& add(T*& p, size_t n) {
+    parts.emplace_back((void**)&p, bytes);
+    bytes += (std::max<size_t>(n, 1) * sizeof(T) + 255u) & ~size_t(255u);
+    return *this;
+  }
+  void place(uint8_t* base) const {
+    for (auto& q : parts) *q.first = base + q.second;
+  }
+};
 
 // A captured plain substep and what it was captured for: the device pointers
 // (by value in every kernel's arguments), the host flags that select kernels,
@@ -87,6 +158,8 @@ struct PinCache {
 };
 
 struct Sim {
+  Sim() { countSims(1); }
+  ~Sim() { countSims(-1); }
   int dev = 0;
   hipStream_t st = nullptr;
   // sizes (sim.js:47-65)
@@ -845,6 +918,7 @@ int ensureRing(Batch* b, uint32_t iters) {
 // A copy of the state a substep starts from (particles, tile tables, pool
 // pressure and cell types, host scalars), to re-run substeps from it.
 struct Snap {
+  uint8_t* base = nullptr;  // the allocation of all the arrays
   float4* pos = nullptr;
   float4* vel = nullptr;
   uint32_t* pid = nullptr;
@@ -854,8 +928,7 @@ struct Snap {
   double tm = 0;
 };
 void freeSnap(Snap* q) {
-  dfree(q->pos); dfree(q->vel); dfree(q->pid); dfree(q->tmap); dfree(q->slotTile); dfree(q->fstack); dfree(q->slotList);
-  dfree(q->ctl); dfree(q->ctype); dfree(q->pres);
+  dfree(q->base);
   delete q;
 }
 
@@ -863,6 +936,7 @@ void freeSnap(Snap* q) {
 struct Adj {
   Sim* s = nullptr;
   uint32_t maxSteps = 0, depth = 0, scap = 0;
+  std::vector<Block> blocks;      // the gradients and first tapes, then more tapes as they are needed
   std::vector<AdjTape> tapes;
   std::vector<uint64_t> sdfSig;   // per tape: the collider grids it was recorded with
   std::vector<const float*> sdfAt;
@@ -873,26 +947,34 @@ struct Adj {
   bool lastOne = false;           // the last reversed substep's solve ran as one launch
   AdjGrad G{};
 };
-void freeTape(AdjTape& T) {
-  dfree(T.pos); dfree(T.vel); dfree(T.pid); dfree(T.binStart); dfree(T.binIdx); dfree(T.tmap0); dfree(T.tmap); dfree(T.slotTile); dfree(T.slotList); dfree(T.ctl);
-  dfree(T.ctype); dfree(T.sten); dfree(T.accWraw); dfree(T.accVfin); dfree(T.accWfin); dfree(T.P); dfree(T.C);
-}
 void freeAdj(Adj* a) {
-  for (AdjTape& T : a->tapes) freeTape(T);
-  AdjGrad& G = a->G;
-  dfree(G.gPos); dfree(G.gVel); dfree(G.gPos2); dfree(G.gVel2); dfree(G.gFN); dfree(G.gFO); dfree(G.gPres); dfree(G.gPres2);
-  dfree(G.gRhs); dfree(G.carry); dfree(G.sorNb); dfree(G.sorCoef); dfree(G.gCol); dfree(G.bar);
+  for (const Block& b : a->blocks) giveBlock(b);
   delete a;
 }
-int allocTape(Sim* s, AdjTape& T) {
+void addTape(Sim* s, Slab& S, AdjTape& T) {
   size_t M = s->maxn, C = size_t(s->scap) * 512u;
-  int rc;
-  if ((rc = dalloc(&T.pos, M)) || (rc = dalloc(&T.vel, M)) || (rc = dalloc(&T.pid, M)) || (rc = dalloc(&T.tmap0, s->ntiles)) ||
-      (rc = dalloc(&T.binStart, size_t(s->ntiles) + 2)) || (rc = dalloc(&T.binIdx, M)) ||
-      (rc = dalloc(&T.tmap, s->ntiles)) || (rc = dalloc(&T.slotTile, s->scap)) || (rc = dalloc(&T.slotList, s->scap)) ||
-      (rc = dalloc(&T.ctl, 16)) || (rc = dalloc(&T.ctype, C)) || (rc = dalloc(&T.sten, C)) || (rc = dalloc(&T.accWraw, C * 3)) ||
-      (rc = dalloc(&T.accVfin, C * 3)) || (rc = dalloc(&T.accWfin, C * 3)) || (rc = dalloc(&T.P, 1)) || (rc = dalloc(&T.C, 1)))
-    return rc;
+  S.add(T.pos, M).add(T.vel, M).add(T.pid, M).add(T.tmap0, s->ntiles).add(T.binStart, size_t(s->ntiles) + 2).add(T.binIdx, M);
+  S.add(T.tmap, s->ntiles).add(T.slotTile, s->scap).add(T.slotList, s->scap).add(T.ctl, 16).add(T.ctype, C).add(T.sten, C);
+  S.add(T.accWraw, C * 3).add(T.accVfin, C * 3).add(T.accWfin, C * 3).add(T.P, 1).add(T.C, 1);
+}
+// Adds tapes, and what S holds already, in one allocation: as many tapes as the
+// context may still need, of SPARE_MAX bytes in all (but one tape at least).
+int growTapes(Adj* a, Slab& S) {
+  AdjTape T{};
+  Slab one;
+  addTape(a->s, one, T);
+  const size_t have = a->tapes.size(), most = S.bytes < SPARE_MAX ? std::max<size_t>(1, (SPARE_MAX - S.bytes) / one.bytes) : 1;
+  std::vector<AdjTape> add(std::min<size_t>(a->maxSteps - have, most), T);
+  for (AdjTape& t : add) addTape(a->s, S, t);
+  Block b;
+  int rc = takeBlock(b, S.bytes, a->s->dev);
+  if (rc) return rc;
+  a->blocks.push_back(b);
+  S.place(b.p);
+  a->tapes.insert(a->tapes.end(), add.begin(), add.end());
+  a->sdfSig.resize(a->tapes.size(), 0);
+  a->sdfAt.resize(a->tapes.size(), nullptr);
+  a->ncols.resize(a->tapes.size(), 0);
   return ST_OK;
 }
 
@@ -1996,12 +2078,14 @@ int st_snapshot_create(void* p, void** out) {
   Snap* q = new Snap();
   size_t M = s->maxn, C = size_t(s->scap) * 512u;
   int rc;
-  if ((rc = dalloc(&q->pos, M)) || (rc = dalloc(&q->vel, M)) || (rc = dalloc(&q->pid, M)) || (rc = dalloc(&q->tmap, s->ntiles)) ||
-      (rc = dalloc(&q->slotTile, s->scap)) || (rc = dalloc(&q->fstack, s->scap)) || (rc = dalloc(&q->slotList, s->scap)) ||
-      (rc = dalloc(&q->ctl, 16)) || (rc = dalloc(&q->ctype, C)) || (rc = dalloc(&q->pres, C))) {
+  Slab S;
+  S.add(q->pos, M).add(q->vel, M).add(q->pid, M).add(q->tmap, s->ntiles).add(q->slotTile, s->scap).add(q->fstack, s->scap);
+  S.add(q->slotList, s->scap).add(q->ctl, 16).add(q->ctype, C).add(q->pres, C);
+  if ((rc = dalloc(&q->base, S.bytes))) {
     freeSnap(q);
     return rc;
   }
+  S.place(q->base);
   CopyList L;
   D2D(L, q->pos, s->G.pos, M); D2D(L, q->vel, s->G.vel, M); D2D(L, q->pid, s->G.pid, M); D2D(L, q->tmap, s->G.tmap, s->ntiles);
   D2D(L, q->slotTile, s->G.slotTile, s->scap); D2D(L, q->fstack, s->G.fstack, s->scap); D2D(L, q->slotList, s->G.slotList, s->scap);
@@ -2188,11 +2272,12 @@ int st_adj_create(void* p, uint32_t max_steps, void** out) {
   a->scap = s->scap;
   size_t M = s->maxn, C = size_t(s->scap) * 512u;
   AdjGrad& G = a->G;
-  int rc;
-  if ((rc = dalloc(&G.gPos, M)) || (rc = dalloc(&G.gVel, M)) || (rc = dalloc(&G.gPos2, M)) || (rc = dalloc(&G.gVel2, M)) ||
-      (rc = dalloc(&G.gFN, C * 3)) || (rc = dalloc(&G.gFO, C * 3)) || (rc = dalloc(&G.gPres, C)) || (rc = dalloc(&G.gPres2, C)) ||
-      (rc = dalloc(&G.gRhs, C)) || (rc = dalloc(&G.carry, size_t(s->ntiles) * 512u)) || (rc = dalloc(&G.sorNb, C * 6)) ||
-      (rc = dalloc(&G.sorCoef, C * 6)) || (rc = dalloc(&G.gCol, size_t(ADJ_MAX_COLS) * 9)) || (rc = dalloc(&G.bar, ADJ_BAR_WORDS))) {
+  Slab S;
+  S.add(G.gPos, M).add(G.gVel, M).add(G.gPos2, M).add(G.gVel2, M).add(G.gFN, C * 3).add(G.gFO, C * 3).add(G.gPres, C).add(G.gPres2, C);
+  S.add(G.gRhs, C).add(G.carry, size_t(s->ntiles) * 512u).add(G.sorNb, C * 6).add(G.sorCoef, C * 6);
+  S.add(G.gCol, size_t(ADJ_MAX_COLS) * 9).add(G.bar, ADJ_BAR_WORDS);
+  int rc = growTapes(a, S);
+  if (rc) {
     freeAdj(a);
     return rc;
   }
@@ -2248,12 +2333,8 @@ int st_adj_record(void* adj, const st_params* prm) {
     return fail(ST_ERR_ARG, "st_adj_record: the adjoint follows at most " + std::to_string(ADJ_MAX_COLS) + " colliders");
   HIPCHK(hipSetDevice(s->dev));
   if (a->tapes.size() <= a->depth) {
-    a->tapes.emplace_back();
-    std::memset(&a->tapes.back(), 0, sizeof(AdjTape));
-    a->sdfSig.push_back(0);
-    a->sdfAt.push_back(nullptr);
-    a->ncols.push_back(0);
-    int rc = allocTape(s, a->tapes.back());
+    Slab S;
+    int rc = growTapes(a, S);
     if (rc) return rc;
   }
   AdjTape& T = a->tapes[a->depth];

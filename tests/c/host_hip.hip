@@ -29,6 +29,7 @@ static int g_refuse = 0;      // cooperative launches of this many threads are r
 static int g_solves = 0;      // the one-per-tile solves do their work
 static int g_failCapture = 0; // the next capture ends with an error
 static int g_failLaunch = 0;  // the next look for a launch's error finds one
+static int g_failMalloc = 0;  // the next allocation fails
 static char g_any[64];        // what handles point at
 
 static hipError_t logf(const char* what, const void* f, dim3 g, dim3 b, hipStream_t st) {
@@ -46,6 +47,7 @@ void host_hip_set(const char* what, int v) {
   if (!strcmp(what, "solves")) g_solves = v;
   if (!strcmp(what, "failCapture")) g_failCapture = v;
   if (!strcmp(what, "failLaunch")) g_failLaunch = v;
+  if (!strcmp(what, "failMalloc")) g_failMalloc = v;
 }
 
 void** __hipRegisterFatBinary(const void*) { return (void**)g_any; }
@@ -81,6 +83,10 @@ const char* hipGetErrorString(hipError_t) { return "host"; }
 hipError_t hipGetSymbolAddress(void** p, const void*) { *p = g_any; return hipSuccess; }
 
 hipError_t hipMalloc(void** p, size_t n) {
+  if (g_failMalloc) {
+    g_failMalloc = 0;
+    return hipErrorOutOfMemory;
+  }
   *p = calloc(1, n ? n : 1);
   if (!*p) return hipErrorOutOfMemory;
   g_live += int64_t(malloc_usable_size(*p));

@@ -166,3 +166,50 @@ def test_grown_pool_is_cleared_before_it_is_filled():
         if line == "copy null":
             assert not pending
             break
+
+
+def test_adjoint_context_gives_its_memory_back():
+    """A context's memory is free again after it but for one block, which the next
+    context takes, and which goes with the last tank or when memory runs out. A tape
+    that could not be allocated is allocated again by the next record."""
+    out = json.loads(run("""
+        import json
+        sc = scenes.dam_break(d=1.0 / 32, iters=6)
+        prm = capi.make_params(**sc.params)
+        g = capi.FlipSimC(opts_for(sc))
+        g.upload(sc.pos, sc.vel)
+        g.step(prm)
+        live = dict(before=hip.host_hip_live())
+        a = capi.AdjointC(g, 2000)
+        for k in ("failed", "again"):
+            hip.host_hip_set(b"failMalloc", 1)
+            try:  # until the tapes of one allocation are used up
+                for _ in range(2000):
+                    a.record(prm)
+                raise SystemExit("no record failed")
+            except capi.StError:
+                live[k] = hip.host_hip_live()
+        a.record(prm)
+        live["more"] = hip.host_hip_live()
+        a.close()
+        live["closed"] = hip.host_hip_live()
+        for k in ("second", "third"):
+            a = capi.AdjointC(g, 2000)
+            a.record(prm)
+            live[k] = hip.host_hip_live()
+            a.close()
+        hip.host_hip_set(b"failMalloc", 1)
+        q = capi.SnapshotC(g)
+        q.close()
+        live["dropped"] = hip.host_hip_live()
+        capi.AdjointC(g, 1).close()
+        live["kept"] = hip.host_hip_live()
+        g.close()
+        live["end"] = hip.host_hip_live()
+        print(json.dumps(live))
+        """))
+    assert out["failed"] == out["again"] < out["more"]
+    assert out["before"] < out["closed"] <= out["before"] + 2**28 + 4096
+    assert out["second"] == out["third"] == out["closed"]
+    assert out["dropped"] == out["before"] < out["kept"]
+    assert out["end"] == 0
