@@ -270,6 +270,7 @@ struct Sim {
     L.initStep = initStep;
     L.smax = sprayCap;
     L.fullTiles = fullTiles();
+    L.wetTiles = nbOn ? std::min(ntiles, scap - 1u) : L.fullTiles;
     L.extrap = extrapOnStep;
     L.exMask = exMask;
     return L;

@@ -55,6 +55,7 @@ struct LaunchCtx {
   uint32_t initStep;  // narrow-band start: 1 restart, 2 water added, 0 none
   uint32_t smax;      // whitewater slots (host copy of P->smax)
   uint32_t fullTiles; // tiles the particles would fill (n / particles of a full tile), for launch shapes
+  uint32_t wetTiles;  // tiles that may hold water: fullTiles, or with a narrow band (water without particles) the pool's
   uint32_t extrap;    // opt-in face velocity extrapolation: layers (host copy of P->extrap)
   uint8_t* exMask;    // its face masks, two per pool cell (ping-pong)
 };

@@ -2251,13 +2251,14 @@ __global__ void __launch_bounds__(WG, TS_WAVES) k_sor_tiles(const DParams* __res
 // iteration, one launch each before: 16^3 tank 4.65 -> 3.93 us, 64^3 4.88 -> 4.01,
 // 96^3 (particles of 415 full tiles) 5.84 -> 5.24; at 128^3 (1050) the windows'
 // extra cells cost more than the launches they save, 7.4 -> 7.8, and at 256^3
-// 27 -> 32: there k_sor_pipe.
+// 27 -> 32: there k_sor_pipe.  A narrow band is taken to fill its pool: half a 192^3
+// box (7757 tiles) 33 us an iteration, 23 with k_sor_pipe; at 96^3 (1245) 6.7 and 6.6.
 // The launches of a solve are even in number, so that the result ends in pres: two
 // iterations each, and one each in the last two or three where the count asks for
 // it.  A solve of one iteration takes k_sor_pipe.
 __host__ __device__ __forceinline__ uint32_t sor_pass_doubles(uint32_t iters) { return (iters >> 1) - (((iters + (iters & 1u)) >> 1) & 1u); }
 __host__ __device__ __forceinline__ uint32_t sor_passes(uint32_t iters) { return iters - sor_pass_doubles(iters); }
-static bool sor_passes_few(uint32_t fullTiles, uint32_t iters) { return iters >= 2u && fullTiles < 700u; }
+static bool sor_passes_few(uint32_t wetTiles, uint32_t iters) { return iters >= 2u && wetTiles < 700u; }
 __device__ __forceinline__ void sor_pass_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t iters, uint32_t pass, uint32_t bid,
                                               uint32_t nbid) {
   __shared__ float sp[TS_W3];
@@ -3705,8 +3706,13 @@ uint32_t sor_tiles_grid(uint32_t cus) {
   return std::min<uint32_t>(cus * uint32_t(nb), SOR_TILES_MAX);
 }
 // Whether the fluid tiles probably fit: about a fifth more than the particles would
-// fill (1223 for 1050 at the 128^3 splash).  A miss costs an idle launch (5 us).
+// fill (1223 for 1050 at the 128^3 splash).  A narrow band's water has no particles:
+// it may fit where the pool is at most three times the grid (a box of a third that
+// depth), and is not tried beyond.  A miss costs an idle launch (a half-full 192^3
+// band, solve 423 us without it, 442 with), a hit saves a quarter of the solve (457 ->
+// 338 us at 1223 fluid tiles).
 static bool sor_tiles_likely(uint32_t fullTiles, uint32_t grid) { return fullTiles + fullTiles / 5u <= grid; }
+static bool sor_tiles_likely(const LaunchCtx& L) { return L.nbOn ? L.wetTiles <= 3u * L.sorTiles : sor_tiles_likely(L.fullTiles, L.sorTiles); }
 
 void morton_tiles(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t* out) {
   auto spread = [](uint64_t v) {  // bit i of v to bit 3i
@@ -3748,7 +3754,7 @@ hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters) {
     // a workgroup per tile where every tile in use has one: at most `most` tiles are
     // in use, and about as many as the particles would fill, and their neighbours
     const uint32_t most = std::min<uint32_t>(L.ntiles, L.scap - 1u);
-    if (!stream && L.sorTiles && (most <= L.sorTiles || sor_tiles_likely(L.fullTiles, L.sorTiles))) {
+    if (!stream && L.sorTiles && (most <= L.sorTiles || sor_tiles_likely(L))) {
       uint32_t safe = L.sorSafe;
       void* args[] = {(void*)&P, (void*)&G, (void*)&it, (void*)&tag, (void*)&seq, (void*)&safe};
       coopErr = hipLaunchCooperativeKernel((const void*)k_sor_tiles, dim3(std::min(most, L.sorTiles)), dim3(WG), args, 0, st);
@@ -3766,7 +3772,7 @@ hipError_t launch_pressure(hipStream_t st, const LaunchCtx& L, int iters) {
   }
   // one or two iterations a launch, ping-pong between the two pressure buffers; an
   // odd count of single ones leaves the result in pres2 and it is copied back
-  if (sor_passes_few(L.fullTiles, uint32_t(iters))) {
+  if (sor_passes_few(L.wetTiles, uint32_t(iters))) {
     for (uint32_t k = 0; k < sor_passes(uint32_t(iters)); k++)
       hipLaunchKernelGGL(k_sor_pass, dim3(L.pipeGrid), dim3(WG), 0, st, L.P, L.G, uint32_t(iters), k);
     return coopErr;

@@ -213,3 +213,36 @@ def test_adjoint_context_gives_its_memory_back():
     assert out["second"] == out["third"] == out["closed"]
     assert out["dropped"] == out["before"] < out["kept"]
     assert out["end"] == 0
+
+
+@pytest.mark.parametrize("sor_mode,cells,expect", [(1, 80, "k_sor_pipe"), (1, 64, "k_sor_pipe"), (0, 80, "k_sor_tiles"), (0, 112, "k_sor_tiles"),
+                                                   (0, 150, "k_sor_resident")])
+def test_band_routes_go_by_its_water_not_its_particles(sor_mode, cells, expect):
+    """A narrow band has particles under the surface only: few of them say nothing of
+    how many tiles hold water. Its launches per iteration are those of many tiles
+    unless the pool itself is small, and the one-per-tile solve is tried only where
+    the pool is at most three times what it holds."""
+    names = json.loads(run(f"""
+        import json
+        d = 1.0 / {2 * cells}
+        sc = scenes.dam_break(d=d, frac=(0.2, 0.05, 0.2), iters=6)
+        g = capi.FlipSimC(opts_for(sc))
+        g.upload(sc.pos, sc.vel)
+        log()
+        g.step(capi.make_params(**dict(sc.params, nb_on=1, nb_band=3.0, sor_mode={sor_mode})))
+        print(json.dumps([n for _, n, _, _ in launches() if "sor" in n]))
+        """))
+    assert names[0] == expect, names
+
+
+def test_small_band_takes_two_iterations_a_launch():
+    names = json.loads(run("""
+        import json
+        sc = scenes.dam_break(d=1.0 / 96, frac=(0.2, 0.05, 0.2), iters=6)
+        g = capi.FlipSimC(opts_for(sc))
+        g.upload(sc.pos, sc.vel)
+        log()
+        g.step(capi.make_params(**dict(sc.params, nb_on=1, nb_band=3.0, sor_mode=1)))
+        print(json.dumps([n for _, n, _, _ in launches() if "sor" in n]))
+        """))
+    assert set(names) == {"k_sor_pass"}
