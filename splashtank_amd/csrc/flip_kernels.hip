@@ -144,26 +144,39 @@ __device__ __forceinline__ void mark_around(const DParams& P, const DGrid& G, ui
 // atomic per workgroup: a tile's particles come in a few hundred runs when they are in
 // the order of a fill, and atomics on one word follow each other.  A run that finds no
 // place in the table within MB_PROBE steps counts and marks in memory as bin_mark does.
-// In the order of a fill, 4.3 million particles 174 -> 48 us, 500 thousand 41 -> 15,
-// 33.5 million 434 -> 230 (floor by bytes 160); reseeded bins (350 thousand) 22 -> 10.
+// A workgroup's places in a bin are consecutive, and g2p keeps them so from then on, so
+// its groups of WG particles are MB_STEP groups apart, those between going to its
+// neighbours: eight groups on end are neighbouring rows of a fill, which share cells,
+// and p2g, whose waves take entries near each other in a bin, then waits for its LDS
+// atomics.  p2g stage of 33.5 million particles (a fill on a lattice, substeps 2 to 20):
+// 600 us with groups on end, 520 with 4 apart (2 apart 595, 8 520, 16 535; a count per
+// wave run, in no order, 530); p2g kernel of 4.3 million 90 -> 77, mark_bin 47 -> 58.  Where the tables are not full (under a million particles)
+// p2g takes as long either way, 34 us at 500 thousand, and groups on end share bins.
+// In the order of a fill, against a count per wave run: 33.5 million particles 434 -> 231
+// us (floor by bytes 160), 4.3 million 174 -> 58, 500 thousand 41 -> 15, reseeded bins
+// (350 thousand) 22 -> 10.
 #define MB_K 8u
 #define MB_HASH 512u
 #define MB_PROBE 16u
+#define MB_STEP 4u
 __device__ __forceinline__ void mark_bin_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid) {
   const DParams& P = *PP;
   __shared__ uint32_t hKey[MB_HASH], hCount[MB_HASH], hMark[MB_HASH], sPlace[MB_K * WG];
   const uint32_t tid = threadIdx.x, ln = lane_id();
-  const uint32_t chunk = ((P.n + nbid * WG - 1u) / (nbid * WG)) * WG, end = min(P.n, (bid + 1u) * chunk);
-  for (uint32_t b0 = bid * chunk; b0 < end; b0 += MB_K * WG) {
-    const uint32_t e = min(end, b0 + MB_K * WG);
+  // groups a workgroup takes; `apart` workgroups (the last ones, what is left) share as
+  // many times that in a row
+  const uint32_t groups = (P.n + nbid * WG - 1u) / (nbid * WG), apart = groups < MB_K ? 1u : MB_STEP;
+  const uint32_t w0 = bid / apart * apart, step = min(apart, nbid - w0) * WG;
+  for (uint32_t j0 = 0; j0 < groups; j0 += MB_K) {
+    const uint32_t first = (w0 * groups + bid - w0) * WG + j0 * step + tid, cnt = min(MB_K, groups - j0);
     for (uint32_t h = tid; h < MB_HASH; h += WG) {
       hKey[h] = ST_NONE;
       hCount[h] = hMark[h] = 0u;
     }
     __syncthreads();
-    for (uint32_t i0 = b0; i0 < e; i0 += WG) {
-      const uint32_t i = i0 + tid;
-      const bool valid = i < e;
+    for (uint32_t j = 0; j < cnt; j++) {
+      const uint32_t i = first + j * step;
+      const bool valid = i < P.n;
       const float4 q = valid ? G.pos[i] : make_float4(0.f, -1.0e6f, 0.f, 0.f);
       uint32_t key, rank, count, marks = 0u, base = 0u, h = MB_HASH;
       int32_t off;
@@ -189,7 +202,7 @@ __device__ __forceinline__ void mark_bin_body(const DParams* __restrict__ PP, co
       h = (uint32_t)__shfl((int)h, lead);
       base = (uint32_t)__shfl((int)base, lead);
       if (valid) {
-        sPlace[i - b0] = h == MB_HASH ? ST_NONE : (h << 16) | (base + rank);
+        sPlace[j * WG + tid] = h == MB_HASH ? ST_NONE : (h << 16) | (base + rank);
         if (h == MB_HASH) {
           G.binKey[i] = key;
           G.binRank[i] = base + rank;
@@ -204,9 +217,9 @@ __device__ __forceinline__ void mark_bin_body(const DParams* __restrict__ PP, co
       for (uint32_t marks = hMark[h]; marks; marks &= marks - 1u) mark_around(P, G, key, uint32_t(__ffs(marks) - 1));
     }
     __syncthreads();
-    for (uint32_t i = b0 + tid; i < e; i += WG) {
-      const uint32_t place = sPlace[i - b0];
-      if (place == ST_NONE) continue;
+    for (uint32_t j = 0; j < cnt; j++) {
+      const uint32_t i = first + j * step, place = sPlace[j * WG + tid];
+      if (i >= P.n || place == ST_NONE) continue;
       G.binKey[i] = hKey[place >> 16];
       G.binRank[i] = hCount[place >> 16] + (place & 0xffffu);
     }
