@@ -74,10 +74,11 @@ def build_napi() -> str | None:
 
 
 def build_checks() -> list:
-    """What the tests load beside the library (tests/c/*.hip): a device self-check and
-    a HIP runtime of host memory, which must not bind the real one."""
+    """What the tests load beside the library (tests/c/*.hip): a device self-check, a layer
+    before the cooperative launch, and a HIP runtime of host memory, which must not
+    bind the real one."""
     outs = []
-    for name, extra in (("convert_check", []), ("host_hip", ["-no-hip-rt"])):
+    for name, extra in (("convert_check", []), ("coop_shim", []), ("host_hip", ["-no-hip-rt"])):
         src = os.path.join(ROOT, "tests", "c", name + ".hip")
         out = os.path.join(ROOT, "tests", "c", f"lib{name}.so")
         tmp = out + ".tmp"

@@ -2213,7 +2213,9 @@ __device__ __forceinline__ void sor_tile_body(const DParams* __restrict__ PP, co
 // in the register file or the LDS too small for the seventh workgroup, which would
 // then never start while the others wait for it.  Up to sor_tiles_safe workgroups
 // always fit, whatever the holes: at four per CU or fewer, 72 registers a wave and 21
-// KB, the free part of some CU is more than the holes between them can hide.  Above,
+// KB, the free part of some CU is more than the holes between them can hide (beside
+// kernels that end by themselves: HIP runs one cooperative launch at a time, and two
+// solves of four a CU that wait at once would not fit in its seven).  Above,
 // the workgroups arrive here first; one that has waited about 0.2 ms ends the launch
 // for all, unless the last has just arrived (both change the one word).  here: that
 // word, then 32 counters, a line each; zero before, cleared by the launch after.

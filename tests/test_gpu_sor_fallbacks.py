@@ -1,0 +1,64 @@
+"""What follows a one-per-tile pressure solve that gives up (its workgroups were not
+all resident) or a resident launch that is refused: the tank, and a batch of tanks,
+keep the bits of an undisturbed run. The arrival word is marked late, or the launch
+refused, from the host (tests/c/coop_shim.hip), in a process of its own."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+CODE = """
+import ctypes
+import numpy as np
+shim = ctypes.CDLL("tests/c/libcoop_shim.so", mode=ctypes.RTLD_GLOBAL)
+from splashtank_amd import capi, scenes
+from tests.helpers import opts_for
+
+BATCH = {batch}
+sc = scenes.dam_break(d=1.0 / 176, frac=(0.3, 0.2, 0.6), iters=9)  # 12^3 tiles: more than are sure to fit at once
+prm = capi.make_params(**sc.params)
+shim.coop_shim_batch(int(BATCH))
+
+def run(mode):
+    shim.coop_shim_set(mode)
+    sims = [capi.FlipSimC(opts_for(sc)) for _ in range(2 if BATCH else 1)]
+    for s in sims:
+        s.upload(sc.pos, sc.vel)
+    step = capi.FlipBatchC(sims) if BATCH else sims[0]
+    for _ in range(3):
+        step.step(prm)
+        step.sync()
+    hits = shim.coop_shim_hits()
+    path = step.sor_path()
+    out = [s.dump(f) for s in sims for f in ("pres", "pos", "vel")]
+    if BATCH:
+        step.close()
+    for s in sims:
+        s.sync()  # reports waits that timed out
+        s.close()
+    return out, hits, int(path)
+
+plain, hits, path = run(0)
+assert hits == 0 and path == 1 and np.any(plain[0] != 0)
+for mode in (1, 2):
+    print("[sor fallbacks] batch", BATCH, "mode", mode, flush=True)
+    out, hits, path = run(mode)
+    assert hits == (3 if mode == 1 or BATCH else 1), hits
+    assert path == (1 if mode == 1 or BATCH else 0), path
+    for a, b in zip(out, plain):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), mode
+print("done")
+"""
+
+
+@pytest.mark.parametrize("batch", [False, True])
+def test_fallbacks_keep_the_bits(batch):
+    r = subprocess.run([sys.executable, "-c", textwrap.dedent(CODE.format(batch=batch))], cwd=ROOT, text=True, capture_output=True, timeout=100)
+    print(r.stdout, flush=True)
+    assert r.returncode == 0 and r.stdout.endswith("done\n"), r.stdout + r.stderr
