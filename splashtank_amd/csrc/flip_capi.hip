@@ -668,7 +668,9 @@ int runStage(Sim* s, int stage, bool alone = false) {
       s->binned = false;
       s->marksClean = s->barClean = true;
       break;
-    case ST_STAGE_CLEAR: break;  // part of the blocks stage's last launch
+    case ST_STAGE_CLEAR:  // part of the blocks stage's last launch, but p2g may be run again without that
+      if (full && alone) launch_clear(st, L);
+      break;
     case ST_STAGE_P2G: if (full) launch_p2g(st, L); break;
     case ST_STAGE_NARROWBAND: if (full && s->nbOn) launch_narrowband(st, L); break;
     case ST_STAGE_CLASSIFY:

@@ -134,6 +134,7 @@ struct CopyList {
 void launch_copies(hipStream_t st, const CopyList& L);
 void launch_fill_u32(hipStream_t st, uint32_t* p, size_t n, uint32_t v);
 void launch_blocks(hipStream_t st, const LaunchCtx& L);
+void launch_clear(hipStream_t st, const LaunchCtx& L);
 void launch_p2g(hipStream_t st, const LaunchCtx& L);
 // counts: the fluid counts into ctl[0], ctl[1] now (normFaces does it too)
 void launch_classify(hipStream_t st, const LaunchCtx& L, bool solid, bool counts);

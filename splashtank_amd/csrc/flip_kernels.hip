@@ -581,6 +581,9 @@ __device__ __forceinline__ void clear_body(const DGrid& G, uint32_t bid, uint32_
   }
 }
 
+// on its own, for a caller that takes the stages one by one
+__global__ void __launch_bounds__(WG) k_clear(DGrid G) { clear_body(G, blockIdx.x, gridDim.x); }
+
 __device__ __forceinline__ void foam_table_body(const DParams* __restrict__ PP, const DGrid& G, uint32_t bid, uint32_t nbid);
 
 // The rest of the tile bookkeeping (after tiles_place): the first workgroups list
@@ -3656,6 +3659,8 @@ void launch_blocks(hipStream_t st, const LaunchCtx& L) {
   if (L.initStep && L.ocean) hipLaunchKernelGGL(k_nb_phi_init<true>, dim3(L.faceGrid), dim3(WG), 0, st, L.P, L.C, L.G);
   else if (L.initStep) hipLaunchKernelGGL(k_nb_phi_init<false>, dim3(L.faceGrid), dim3(WG), 0, st, L.P, L.C, L.G);
 }
+
+void launch_clear(hipStream_t st, const LaunchCtx& L) { hipLaunchKernelGGL(k_clear, dim3(512 / WG), dim3(WG), 0, st, L.G); }
 
 void launch_p2g(hipStream_t st, const LaunchCtx& L) {
   if (!L.n) return;

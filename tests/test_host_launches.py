@@ -246,3 +246,25 @@ def test_small_band_takes_two_iterations_a_launch():
         print(json.dumps([n for _, n, _, _ in launches() if "sor" in n]))
         """))
     assert set(names) == {"k_sor_pass"}
+
+
+def test_clear_stage_on_its_own_clears():
+    """A whole step clears the spare slot in the blocks stage; a caller that runs p2g
+    twice with the clear stage between gets it cleared there."""
+    out = json.loads(run("""
+        import json
+        sc = scenes.dam_break(d=1.0 / 32, iters=6)
+        prm = capi.make_params(**sc.params)
+        g = capi.FlipSimC(opts_for(sc))
+        g.upload(sc.pos, sc.vel)
+        log()
+        g.step(prm)
+        out = [[n for _, n, _, _ in launches()]]
+        g.begin_step(prm)
+        g.stages(capi.ST_STAGE_P2G)
+        log()
+        g.stage(capi.ST_STAGE_CLEAR)
+        out.append([n for _, n, _, _ in launches()])
+        print(json.dumps(out))
+        """))
+    assert "k_clear" not in out[0] and out[1] == ["k_clear"]
