@@ -692,7 +692,7 @@ int runStage(Sim* s, int stage, bool alone = false) {
     case ST_STAGE_PROJECT: if (full) launch_project(st, L); break;
     case ST_STAGE_G2P:
       if (full) {
-        launch_g2p(st, L);
+        launch_g2p(st, L, alone);
         s->binned = L.binNext && L.n != 0;
         if (s->binned) s->marksClean = false;
         if (L.n) {  // g2p wrote the new state into the other buffer

@@ -159,7 +159,8 @@ uint32_t sor_tiles_safe(uint32_t cus);
 // tile indices in Morton order of their (ti, tj, tk) coordinates
 void morton_tiles(uint32_t tx, uint32_t ty, uint32_t tz, uint32_t* out);
 void launch_project(hipStream_t st, const LaunchCtx& L);
-void launch_g2p(hipStream_t st, const LaunchCtx& L);
+// table: make the foam table of this step's parameters first (tiles_finish has, of its step's)
+void launch_g2p(hipStream_t st, const LaunchCtx& L, bool table);
 // g2p workgroups per tile for particles that would fill this many tiles
 uint32_t g2p_split(uint32_t fullTiles);
 void launch_unsort(hipStream_t st, const float4* src, const uint32_t* pid, float4* out, uint32_t n);

@@ -2620,6 +2620,8 @@ __device__ __forceinline__ void foam_table_body(const DParams* __restrict__ PP, 
   for (uint32_t t = bid * blockDim.x + threadIdx.x; t < FOAM_TAB; t += nbid * blockDim.x)
     G.foamTab[t] = d_foamRow(*PP, float(t));
 }
+// on its own, for a caller that takes the stages one by one
+__global__ void __launch_bounds__(WG) k_foam_table(const DParams* __restrict__ PP, DGrid G) { foam_table_body(PP, G, blockIdx.x, gridDim.x); }
 
 template <bool OCEAN, class GridT>
 __device__ __forceinline__ void g2p_particle(const DParams& P, const DCols* __restrict__ C, const DGrid& G, const GridT& g,
@@ -3829,8 +3831,9 @@ void launch_project(hipStream_t st, const LaunchCtx& L) {
 // 8430: 1056 / 1061; a narrow band of 84: 37 / 29 / 32 / 40.
 uint32_t g2p_split(uint32_t fullTiles) { return fullTiles < 48u ? 8u : fullTiles < 256u ? 4u : fullTiles < 2048u ? 2u : 1u; }
 
-void launch_g2p(hipStream_t st, const LaunchCtx& L) {
+void launch_g2p(hipStream_t st, const LaunchCtx& L, bool table) {
   if (!L.n) return;
+  if (table) hipLaunchKernelGGL(k_foam_table, dim3(FOAM_TAB / WG), dim3(WG), 0, st, L.P, L.G);
   if (L.binNext) launch_marks_clear(st, L);  // the next substep's tile marks and bin counts start here
   const uint32_t split = g2p_split(L.fullTiles);
   const uint32_t g = std::min<uint32_t>(L.ntiles * split, 8192u);
