@@ -89,9 +89,10 @@ typedef struct st_params {
   uint32_t nfv;
   float fills[64];
   /* pressure solve: 0 (default) runs every iteration of a solve in one
-   * cooperative launch, with the pressure resident in LDS when the tiles in use
-   * fit and streaming tile windows otherwise; 1 one launch per red-black
-   * iteration; 2 the cooperative launch, always streaming; 3 (ST_SOR_TUNED) the
+   * cooperative launch, with a workgroup per fluid tile where they all fit on the
+   * device, else with the pressure resident in LDS when the tiles in use fit and
+   * streaming tile windows otherwise; 1 a launch per red-black iteration, or per
+   * two where the tiles are few; 2 the cooperative launch, always streaming; 3 (ST_SOR_TUNED) the
    * path and launch width st_tune_sor chose for this sim (0 until it ran).  All
    * give the same bits.  No counterpart in the reference (an implementation
    * choice here). */
@@ -238,9 +239,9 @@ int st_step(void* sim, const st_params* p);
  * replay: the first substep of a kind (particle buffer parity, bins made or
  * not, collider lookup rebuilt or not, sizes) is stream-captured and later
  * ones replay it, with the step's parameters copied into the one device slot
- * the graph reads.  Graphed substeps solve with one launch per SOR iteration
- * (the same bits; a captured cooperative launch is not scheduled as one when
- * other streams run at the same time).  Graphs cover plain substeps only
+ * the graph reads.  Graphed substeps solve with a launch per SOR iteration, or
+ * per two where the tiles are few (the same bits; a captured cooperative launch
+ * is not scheduled as one when other streams run at the same time).  Graphs cover plain substeps only
  * (ST_ERR_ARG with the narrow band or a tile-only step).
  * No counterpart in the reference, which records its dispatches into one
  * compute pass per step (src/flip/sim.js:245-310). */
@@ -449,11 +450,13 @@ int st_batch_sync(void* batch);
 /* Number of tanks. */
 int st_batch_size(void* batch, uint32_t* n);
 /* The batched pressure solve.  By default (st_batch_step, no graph) every
- * tank's SOR runs resident in one cooperative launch of the device's resident
- * workgroups (one per CU): each tank gets a range of them, enough that its
+ * tank's SOR runs in one cooperative launch: with a workgroup per fluid tile of
+ * all tanks where they fit on the device, else resident over one workgroup per
+ * CU: each tank gets a range of them, enough that its
  * tiles fit in LDS (a tank too big for all of them streams tile windows), in
  * as few phases as the tiles allow, and the same bits as alone.  Graph replays
- * and st_batch_sor_grid(batch, 0) use one launch per iteration instead;
+ * and st_batch_sor_grid(batch, 0) use a launch per iteration, or per two where
+ * the tiles are few, instead;
  * st_batch_sor_grid(batch, w) caps the cooperative launch at w workgroups (at
  * least 2, at most the resident count; more phases).  st_batch_sor_path reports whether
  * the last batched substep's solve ran in the one launch. */

@@ -576,7 +576,7 @@ class FlipBatchC:
 
     def sor_grid(self, workgroups: int):
         """Cap the one-launch batched SOR at `workgroups` resident workgroups
-        (0: one launch per iteration)."""
+        (0: a launch per iteration, or per two where the tiles are few)."""
         self._call("sor_grid", self.h, int(workgroups))
 
     def sor_path(self) -> bool:

@@ -725,7 +725,7 @@ int runStage(Sim* s, int stage, bool alone = false) {
 // parameter block and collider records go to one fixed device slot, which the
 // captured kernels read; the first substep of a kind is captured (stream
 // capture of every stage) and later ones replay it.  A graphed substep solves
-// with one launch per SOR iteration (the same bits).  A captured cooperative
+// with a launch per SOR iteration, or per two (the same bits).  A captured cooperative
 // launch does replay, alone with the right bits, but with a second sim
 // stepping on its own stream at the same time the replays gave other bits
 // than the eager substeps (direct cooperative launches kept them): a graph

@@ -12,8 +12,8 @@
 // resident SOR: workgroup size, tiles resident per workgroup, and the largest
 // grid its barrier serves (sorBar holds COOP_MAX_WG epochs, then the sequence
 // number of the last solve it finished, a count of barrier time-outs, the
-// barrier's release word, the path of the last solve: 0 one launch per
-// iteration, 1 resident, 2 streaming, and the sequence number of the last solve
+// barrier's release word, the path of the last solve: 0 launches per
+// iteration or two, 1 resident, 2 streaming, and the sequence number of the last solve
 // with a workgroup per tile)
 #define COOP_WG 1024
 #define COOP_TMAX 54
@@ -99,7 +99,7 @@ struct BTankPlan {
 // range per tank (empty where the tank has no work in that launch).  Table
 // BT_PIPE0 + it belongs to SOR iteration (or pass) it.
 enum BatchTable {
-  BT_FILL_MARK, BT_MARK, BT_SCAN, BT_PLACE, BT_FINISH, BT_ONE, BT_CELL,
+  BT_FILL_MARK, BT_MARK, BT_SCAN, BT_PLACE, BT_FINISH, BT_CELL,
   BT_TILE, BT_SOLID, BT_COPY, BT_G2P, BT_PIPE0
 };
 size_t batch_table_words(uint32_t nt, uint32_t itersMax);

@@ -296,20 +296,10 @@ __global__ void __launch_bounds__(1024) k_scan_top(uint32_t* __restrict__ sums, 
                                                    uint32_t n) {
   scan_top_body(sums, nb, out, n, blockIdx.x, gridDim.x);
 }
-__device__ __forceinline__ void scan_add_body(uint32_t* __restrict__ out, uint32_t n, const uint32_t* __restrict__ sums,
-                                              uint32_t* __restrict__ copy, uint32_t bid, uint32_t nbid) {
-  uint32_t base = bid * (WG * 4) + threadIdx.x * 4;
-  uint32_t add = sums[bid];
-  for (int q = 0; q < 4; q++)
-    if (base + q < n) {
-      uint32_t v = out[base + q] + add;
-      out[base + q] = v;
-      if (copy) copy[base + q] = v;
-    }
-}
-__global__ void __launch_bounds__(WG) k_scan_add(uint32_t* __restrict__ out, uint32_t n, const uint32_t* __restrict__ sums,
-                                                 uint32_t* __restrict__ copy) {
-  scan_add_body(out, n, sums, copy, blockIdx.x, gridDim.x);
+__global__ void __launch_bounds__(WG) k_scan_add(uint32_t* __restrict__ out, uint32_t n, const uint32_t* __restrict__ sums) {
+  const uint32_t base = blockIdx.x * (WG * 4) + threadIdx.x * 4, add = sums[blockIdx.x];
+  for (uint32_t q = 0; q < 4u; q++)
+    if (base + q < n) out[base + q] += add;
 }
 
 // ---------------------------------------------------------------------------
@@ -3449,14 +3439,13 @@ __global__ void __launch_bounds__(P2G_MERGE_WG) kb_p2g_merge(BATCH_ARGS) {
   const DGrid G = T.G;  // local: the body's stores cannot touch it
   p2g_merge_body(G, b.blk, b.nblk);
 }
-// reduces the partials of the launch whose block table is `of`
 __global__ void kb_solid_build(BATCH_ARGS) {
   BATCH_TANK;
   const DGrid G = T.G;  // local: the body's stores cannot touch it
   solid_build_body(TP, TC, G, b.blk, b.nblk);
 }
-// classify keeps reading the parameter block from memory: with the LDS copy it
-// took 104 VGPRs and ran slower (77 against 68 us per 64-tank substep)
+// classify reads the parameter block from memory: it stores little between its reads,
+// and a copy of the block in LDS took 104 VGPRs (77 against 68 us per 64-tank substep)
 __global__ void __launch_bounds__(WG) kb_classify(BATCH_ARGS) {
   BATCH_TANK;
   const DGrid G = T.G;  // local: the body's stores cannot touch it
@@ -3634,11 +3623,11 @@ static void launch_marks_clear(hipStream_t st, const LaunchCtx& L) {
 // workgroups of tiles_finish beside the list's: a few hundred words per tile in use at most
 static uint32_t tiles_finish_grid(uint32_t scap) { return std::max<uint32_t>(8u, std::min<uint32_t>(scap, 2048u)); }
 
-static void launch_scan(hipStream_t st, const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* sums, uint32_t* copy) {
+static void launch_scan(hipStream_t st, const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* sums) {
   uint32_t nb = gridFor(n, WG * 4);
   hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(WG), 0, st, in, out, n, sums);
   hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, st, sums, nb, out, n);
-  hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(WG), 0, st, out, n, (const uint32_t*)sums, copy);
+  hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(WG), 0, st, out, n, (const uint32_t*)sums);
 }
 
 // workgroups of mark_bin: full tables of particles where that still gives two workgroups
@@ -3917,7 +3906,6 @@ bool batch_tables(const BTankPlan* plan, uint32_t nt, uint32_t full, uint32_t it
           case BT_SCAN: c = nb; break;
           case BT_PLACE: c = nb + gridFor(p.n, WG * 4u); break;
           case BT_FINISH: c = nb + batch_share(BATCH_CELL_WG, p.scap, scapTot, tiles_finish_grid(p.scap)); break;
-          case BT_ONE: c = 1u; break;
           case BT_CELL: c = cell; break;
           case BT_TILE: c = batch_share(BATCH_TILE_WG, p.scap, scapTot, std::max<uint32_t>(1u, std::min<uint32_t>(p.scap, 8192u))); break;
           case BT_SOLID: c = p.solid ? cell : 0u; break;
@@ -3965,8 +3953,8 @@ bool launch_batch_step(hipStream_t st, const BTank* dT, const uint32_t* dtab, co
   BLAUNCH(kb_classify, BT_CELL, WG);
   BLAUNCH(kb_norm_faces, BT_TILE, WG, tab(BT_CELL));
   BLAUNCH(kb_divergence, BT_TILE, WG);
-  // pressure: the resident solves of all tanks in one cooperative launch, or
-  // one launch per iteration (ping-pong between pres and pres2)
+  // pressure: the solves of all tanks in one cooperative launch, or a launch per
+  // iteration or two (ping-pong between pres and pres2)
   bool resident = false;
   if (coopGrid && dPlan && itersMax) {
     const BTank* a0 = dT;
@@ -4389,14 +4377,14 @@ void launch_spray(hipStream_t st, const LaunchCtx& L, uint32_t airN, bool air, b
   hipLaunchKernelGGL(k_spray_step, dim3(sg), dim3(WG), 0, st, L.P, L.C, L.G);
   if (emit && L.n) {
     hipLaunchKernelGGL(k_spray_count, dim3(pg), dim3(WG), 0, st, L.P, L.G);
-    launch_scan(st, L.G.sprCnt, L.G.sprOff, L.n, L.G.sprSums, nullptr);
+    launch_scan(st, L.G.sprCnt, L.G.sprOff, L.n, L.G.sprSums);
     hipLaunchKernelGGL(k_spray_emit, dim3(pg), dim3(WG), 0, st, L.P, L.G);
     hipLaunchKernelGGL(k_spray_advance, dim3(1), dim3(64), 0, st, L.P, L.G);
   }
   if (ndrip) {
     const uint32_t dg = std::max<uint32_t>(1u, std::min<uint32_t>(gridFor(ndrip, WG), 1024u));
     hipLaunchKernelGGL(k_drip_flags, dim3(dg), dim3(WG), 0, st, L.P, L.C, L.G);
-    launch_scan(st, L.G.dripFlag, L.G.dripOff, ndrip, L.G.dripSums, nullptr);
+    launch_scan(st, L.G.dripFlag, L.G.dripOff, ndrip, L.G.dripSums);
     hipLaunchKernelGGL(k_drip_emit, dim3(dg), dim3(WG), 0, st, L.P, L.C, L.G);
     hipLaunchKernelGGL(k_drip_advance, dim3(1), dim3(64), 0, st, L.P, L.G);
   }
@@ -4564,7 +4552,7 @@ void launch_deep(hipStream_t st, const LaunchCtx& L, uint32_t ncell, uint32_t pr
   launch_fill_u32(st, all, 1, 0u);
   launch_fill_u32(st, flag, ncell, 0u);  // cells past the slots in use stay unflagged
   hipLaunchKernelGGL(k_deep_flags, dim3(g), dim3(WG), 0, st, L.P, L.G, prev, flag, all);
-  launch_scan(st, flag, off, ncell, sums, nullptr);
+  launch_scan(st, flag, off, ncell, sums);
   hipLaunchKernelGGL(k_deep_emit, dim3(g), dim3(WG), 0, st, L.P, L.G, flag, off, out);
 }
 
@@ -4574,7 +4562,7 @@ void launch_pack_view(hipStream_t st, const LaunchCtx& L, const ViewParams& V, u
   if (sdMax) {
     const uint32_t g = std::max<uint32_t>(1u, std::min<uint32_t>(gridFor(sdMax, WG), 4096u));
     hipLaunchKernelGGL(k_view_spray_flags, dim3(g), dim3(WG), 0, st, L.P, L.G, sdMax, flag);
-    launch_scan(st, flag, off, sdMax, sums, nullptr);
+    launch_scan(st, flag, off, sdMax, sums);
     hipLaunchKernelGGL(k_view_spray_put, dim3(g), dim3(WG), 0, st, L.P, L.G, sdMax, flag, off, sdisp, V.foamLife);
   } else {
     launch_fill_u32(st, off, 1, 0u);
