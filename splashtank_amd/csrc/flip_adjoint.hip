@@ -448,7 +448,7 @@ __device__ __forceinline__ void adj_sor_body(const AdjTape& T, const AdjGrad& G,
 #define ASW 12
 #define ASW3 (ASW * ASW * ASW)
 #define ASW_WG 512
-// the slots of the 27 tiles around each tile in use, in sorNb
+// the slots of the 27 tiles around each tile in use
 __global__ void __launch_bounds__(AWG) k_adj_sor_tiles(AdjTape T, AdjGrad G) {
   const DParams& P = *T.P;
   const uint32_t tot = T.ctl[4] * 27u;
@@ -457,7 +457,7 @@ __global__ void __launch_bounds__(AWG) k_adj_sor_tiles(AdjTape T, AdjGrad G) {
     const int32_t i = int32_t(tile % P.tx) + int32_t(q % 3u) - 1, j = int32_t((tile / P.tx) % P.ty) + int32_t((q / 3u) % 3u) - 1,
                   k = int32_t(tile / (P.tx * P.ty)) + int32_t(q / 9u) - 1;
     const bool in = i >= 0 && j >= 0 && k >= 0 && i < int32_t(P.tx) && j < int32_t(P.ty) && k < int32_t(P.tz);
-    G.sorNb[t] = in ? T.tmap[uint32_t(i) + P.tx * (uint32_t(j) + P.ty * uint32_t(k))] : ST_NONE;
+    G.tileNb[t] = in ? T.tmap[uint32_t(i) + P.tx * (uint32_t(j) + P.ty * uint32_t(k))] : ST_NONE;
   }
 }
 __global__ void __launch_bounds__(ASW_WG) k_adj_sor_pass(AdjTape T, AdjGrad G, const float* __restrict__ gin, float* __restrict__ gout) {
@@ -477,7 +477,7 @@ __global__ void __launch_bounds__(ASW_WG) k_adj_sor_pass(AdjTape T, AdjGrad G, c
     return g;
   };
   for (uint32_t b = blockIdx.x, nact = T.ctl[4]; b < nact; b += gridDim.x) {
-    if (tid < 27u) sSlot[tid] = G.sorNb[b * 27u + tid];
+    if (tid < 27u) sSlot[tid] = G.tileNb[b * 27u + tid];
     __syncthreads();
     const uint32_t s = sSlot[13];
     for (uint32_t q = tid; q < ASW3; q += ASW_WG) {

@@ -2277,7 +2277,7 @@ int st_adj_create(void* p, uint32_t max_steps, void** out) {
   AdjGrad& G = a->G;
   Slab S;
   S.add(G.gPos, M).add(G.gVel, M).add(G.gPos2, M).add(G.gVel2, M).add(G.gFN, C * 3).add(G.gFO, C * 3).add(G.gPres, C).add(G.gPres2, C);
-  S.add(G.gRhs, C).add(G.carry, size_t(s->ntiles) * 512u).add(G.sorNb, C * 6).add(G.sorCoef, C * 6);
+  S.add(G.gRhs, C).add(G.carry, size_t(s->ntiles) * 512u).add(G.tileNb, size_t(s->scap) * 27u);
   S.add(G.gCol, size_t(ADJ_MAX_COLS) * 9).add(G.bar, ADJ_BAR_WORDS);
   int rc = growTapes(a, S);
   if (rc) {
@@ -2431,6 +2431,16 @@ int st_adj_grad(void* adj, float* g_pos4, float* g_vel4) {
 int st_adj_set_sor_path(void* adj, uint32_t one_launch) {
   Adj* a = (Adj*)adj;
   if (!a) return fail(ST_ERR_ARG, "st_adj_set_sor_path: null context");
+  if (one_launch && !a->G.sorNb) {  // its tables: 48 bytes per pool cell
+    HIPCHK(hipSetDevice(a->s->dev));
+    Slab S;
+    S.add(a->G.sorNb, size_t(a->scap) * 512u * 6u).add(a->G.sorCoef, size_t(a->scap) * 512u * 6u);
+    Block b;
+    int rc = takeBlock(b, S.bytes, a->s->dev);
+    if (rc) return rc;
+    a->blocks.push_back(b);
+    S.place(b.p);
+  }
   a->oneLaunch = one_launch != 0u;
   return ST_OK;
 }

@@ -268,3 +268,19 @@ def test_clear_stage_on_its_own_clears():
         print(json.dumps(out))
         """))
     assert "k_clear" not in out[0] and out[1] == ["k_clear"]
+
+
+def test_adjoint_context_makes_the_one_launch_tables_when_asked():
+    out = json.loads(run("""
+        import json
+        sc = scenes.dam_break(d=1.0 / 32, iters=6)
+        g = capi.FlipSimC(opts_for(sc))
+        a = capi.AdjointC(g, 1)
+        live = [hip.host_hip_live()]
+        for one in (0, 1, 0, 1):
+            a.set_sor_path(one)
+            live.append(hip.host_hip_live())
+        print(json.dumps([live, g.dims.scap * 512 * 48]))
+        """))
+    live, tables = out
+    assert live[0] == live[1] and live[2] == live[3] == live[4] and live[2] - live[1] >= tables
