@@ -2256,10 +2256,10 @@ __global__ void __launch_bounds__(WG, TS_WAVES) k_sor_tiles(const DParams* __res
 // read from one pressure buffer and the tiles written to the other.  Tiles without
 // fluid are never read (they stand for zeros) nor written.
 // Bounds: the launch (about 3 us) and the window's three dependent loads.  Per
-// iteration, one launch each before: 16^3 tank 4.65 -> 3.93 us, 64^3 4.88 -> 4.01,
-// 96^3 (particles of 415 full tiles) 5.84 -> 5.24; at 128^3 (1050) the windows'
-// extra cells cost more than the launches they save, 7.4 -> 7.8, and at 256^3
-// 27 -> 32: there k_sor_pipe.  A narrow band is taken to fill its pool: half a 192^3
+// iteration, k_sor_pipe's against these: 15 full tiles 4.4 and 3.9 us, 240 5.0 and 4.5,
+// 526 5.5 and 5.2, 659 5.9 and 5.5, 810 6.2 and 6.2; above, the windows' extra cells
+// cost more than the launches they save, 981 6.6 and 7.1, 1920 9.4 and 11, 256^3 (8430)
+// 27 and 32: there k_sor_pipe.  A narrow band is taken to fill its pool: half a 192^3
 // box (7757 tiles) 33 us an iteration, 23 with k_sor_pipe; at 96^3 (1245) 6.7 and 6.6.
 // The launches of a solve are even in number, so that the result ends in pres: two
 // iterations each, and one each in the last two or three where the count asks for
@@ -3655,9 +3655,11 @@ void launch_clear(hipStream_t st, const LaunchCtx& L) { hipLaunchKernelGGL(k_cle
 
 void launch_p2g(hipStream_t st, const LaunchCtx& L) {
   if (!L.n) return;
-  // 512 threads per tile while the tiles leave CUs idle or lightly loaded (stage
-  // 48.6 -> 37.1 us at 123 full tiles, 121 -> 112 at 1050), 256 above, where more
-  // workgroups per CU hide a tile's barriers better (575 against 620 us at 8430)
+  // 512 threads per tile while the tiles leave CUs idle or lightly loaded, 256 above,
+  // where more workgroups per CU hide a tile's barriers better.  Stage, us at 512 / 256:
+  // dam breaks of 51 full tiles 32 / 41, 240 46 / 49, 659 62 / 62, 981 88 / 82, 1398
+  // 120 / 115, 2556 198 / 181; splashes of 705 79 / 80, 1053 94 / 103, 1764 142 / 146,
+  // 2057 170 / 170, 2739 206 / 210, 8430 560 / 525.
   if (L.fullTiles < 2048u) hipLaunchKernelGGL(k_p2g_tile<512>, dim3(L.tileGrid), dim3(512), 0, st, L.P, L.G);
   else hipLaunchKernelGGL(k_p2g_tile<256>, dim3(L.tileGrid), dim3(256), 0, st, L.P, L.G);
   hipLaunchKernelGGL(k_p2g_merge, dim3(L.tileGrid), dim3(P2G_MERGE_WG), 0, st, L.G);
@@ -3815,9 +3817,13 @@ void launch_project(hipStream_t st, const LaunchCtx& L) {
 // Workgroups that share one tile's particles in g2p.  A full tile is 16 rounds of
 // 256 particles, one after another in one workgroup; with few tiles that chain is
 // the kernel's time, so they are split, each part staging the tile's window again.
-// Measured (g2p stage, us at 1 / 2 / 4 / 8 parts): 15 full tiles 55 / 38 / 30 / 24,
-// 123: 80 / 54 / 48 / 47, 415: 101 / 76 / 78 / 98, 1050: 188 / 171 / 212 / 242,
-// 8430: 1056 / 1061; a narrow band of 84: 37 / 29 / 32 / 40.
+// Measured (g2p stage of dam breaks, us at 1 / 2 / 4 / 8 parts): 15 full tiles 56 / 35
+// / 23 / 18, 51: 63 / 38 / 27 / 27, 82: 69 / 53 / 42 / 32, 175: 68 / 50 / 42 / 45, 240:
+// 74 / 59 / 45 / 53, 415: 89 / 64 / 66 / 83, 659: 106 / 101 / 94 / 121; a narrow band of
+// 84: 37 / 29 / 32 / 40.  From 800 to 2800 it depends on how the tiles fill the 1280
+// workgroups that fit at once, and the line is put between (1 / 2 parts: dam breaks of
+// 981 128 / 157, 1398 189 / 180, 1920 222 / 252, 2556 287 / 317; splashes of 1053 180 /
+// 150, 1500 230 / 225, 2057 319 / 301, 2739 415 / 345); 8430: 1056 / 1061.
 uint32_t g2p_split(uint32_t fullTiles) { return fullTiles < 48u ? 8u : fullTiles < 256u ? 4u : fullTiles < 2048u ? 2u : 1u; }
 
 void launch_g2p(hipStream_t st, const LaunchCtx& L, bool table) {
