@@ -1,6 +1,6 @@
 // Stands before the HIP runtime's cooperative launch, for GPU tests of what follows a
 // one-per-tile pressure solve that gives up, or a resident one that is refused.
-// Loaded with global symbols before libsplashtank_hip.so (tests/test_gpu_sor_fallbacks.py).
+// Loaded with global symbols before libsplashtank_hip.so (tests/test_coop_fallbacks.py).
 // Mode 1: the one-per-tile launches find their arrival word marked late, as the first
 // workgroup that waited too long would leave it, and check it however few they are;
 // every workgroup then ends at once.  Mode 2: launches of 1024 threads are refused.

@@ -1,7 +1,9 @@
 """What follows a one-per-tile pressure solve that gives up (its workgroups were not
 all resident) or a resident launch that is refused: the tank, and a batch of tanks,
 keep the bits of an undisturbed run. The arrival word is marked late, or the launch
-refused, from the host (tests/c/coop_shim.hip), in a process of its own."""
+refused, from the host (tests/c/coop_shim.hip), in a process of its own, which
+gets no cooperative launches while another process of the card has them: before the
+files of GPU tests, none has."""
 import os
 import subprocess
 import sys
@@ -45,7 +47,10 @@ def run(mode):
     return out, hits, int(path)
 
 plain, hits, path = run(0)
-assert hits == 0 and path == 1 and np.any(plain[0] != 0)
+assert hits == 0 and np.any(plain[0] != 0)
+if path == 0:
+    raise SystemExit(77)
+assert path == 1
 for mode in (1, 2):
     print("[sor fallbacks] batch", BATCH, "mode", mode, flush=True)
     out, hits, path = run(mode)
@@ -61,4 +66,6 @@ print("done")
 def test_fallbacks_keep_the_bits(batch):
     r = subprocess.run([sys.executable, "-c", textwrap.dedent(CODE.format(batch=batch))], cwd=ROOT, text=True, capture_output=True, timeout=100)
     print(r.stdout, flush=True)
+    if r.returncode == 77:
+        pytest.skip("another process of this card has its cooperative launches")
     assert r.returncode == 0 and r.stdout.endswith("done\n"), r.stdout + r.stderr
